@@ -5,11 +5,15 @@
 //   serial / parallel / blocked variants.  Write-bound: each thread produces 4
 //   consecutive k of one output row (16-byte stores when K % 4 == 0).
 // cp_reconstruct (tenrso-kernels/src/outer.rs:223-274):
-//   out[i_0..i_{N-1}] = sum_r (prod_k F_k[i_k, r]) * w_r, r ascending, product left to right.
-//   Write-bound; each thread owns one output element.
+//   out[i_0..i_{N-1}] = sum_r (prod_k F_k[i_k, r]) * w_r.
+//   An FP32 matrix product of two Khatri-Rao factors formed in LDS.
+#include <type_traits>
+
 #include "kr_reconstruct.hpp"
 
 namespace tenrso {
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 static inline unsigned cdiv(i64 a, i64 b) { return (unsigned)((a + b - 1) / b); }
 
@@ -44,36 +48,142 @@ int khatri_rao_f32(tenrso_ctx* ctx, const float* A, i64 I, const float* B, i64 J
 }
 
 struct ReconArgs {
-  int nd;
-  i64 R;
+  int nd, h;           // modes [0, h) are the rows of the output matrix, [h, nd) its columns
+  i64 R, M, N;         // M = product of the row modes, N of the column modes
   i64 shape[MAXD_RECON];
   const float* F[MAXD_RECON];
   const float* w;
-  i64 total;
+  int vec;              // R % 4 == 0 and every factor 16-byte aligned: 16-byte factor loads
+  unsigned ctiles;
   const float* xsub;    // not null: out = xsub - reconstruction (a residual)
   const float* gscale;  // not null: out *= gscale[0] (a device scalar)
 };
 
+// out (M x N) = KR(F_0..F_{h-1}) diag(w) KR(F_h..F_{nd-1})^T as an FP32 matrix-core
+// product (v_mfma_f32_16x16x4f32).  A workgroup of 4 waves owns a TILE x TILE
+// tile (TILE = 32 T, a wave 16T x 16T of it): it forms the Khatri-Rao rows of its
+// rows and of its columns in LDS, KT ranks at a time (products left to right, one
+// rounding each), and contracts them.  Ranks past R are zero on both sides.  The
+// columns are the M dimension of the instruction, so a lane ends with four
+// consecutive output elements and stores 16 bytes (VS: N % 4 == 0 and aligned).
+// Operands are read from LDS as 4 consecutive ranks (lane group g, step s
+// contracts rank 16u + 4g + s on both sides); the pitch of KT + 4 floats keeps
+// those 16-byte reads free of bank conflicts.
+// Bound: at 256^3 rank 64 the 2.1 GFLOP take 14 us at the matrix cores' FP32
+// peak and the 64 MiB of output 13 us at 5.2 TB/s; the form with one thread per
+// element, each lane reading factor rows at a stride of R floats, took 2580 us; this
+// one takes 28 us (76 TFLOP/s).
+template <int KT, int T, bool VS>
 __global__ __launch_bounds__(256) void reconstruct_kernel(ReconArgs a, float* __restrict__ out) {
-  const i64 x = (i64)blockIdx.x * 256 + threadIdx.x;
-  if (x >= a.total) return;
-  const float* rows[MAXD_RECON];
-  i64 rem = x;
-  for (int k = a.nd - 1; k >= 0; --k) {
-    const i64 ix = rem % a.shape[k];
-    rem /= a.shape[k];
-    rows[k] = a.F[k] + ix * a.R;
+  constexpr int TILE = 32 * T, PITCH = KT + 4;
+  __shared__ __attribute__((aligned(16))) float sk[2 * TILE * PITCH];  // rows, then columns
+  __shared__ i64 sidx[MAXD_RECON][TILE];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int g = lane >> 4, c = lane & 15;
+  const i64 r_base = (i64)(blockIdx.x / a.ctiles) * TILE, c_base = (i64)(blockIdx.x % a.ctiles) * TILE;
+  // factor rows of every tile row (modes < h) and column (modes >= h); those past
+  // the end repeat the last one and are not stored
+  if (tid < 2 * TILE) {
+    const bool col = tid >= TILE;
+    const int e = col ? tid - TILE : tid;
+    i64 rem = col ? (c_base + e < a.N ? c_base + e : a.N - 1) : (r_base + e < a.M ? r_base + e : a.M - 1);
+    for (int k = (col ? a.nd : a.h) - 1; k >= (col ? a.h : 0); --k) {
+      sidx[k][e] = rem % a.shape[k];
+      rem /= a.shape[k];
+    }
   }
-  float acc = 0.0f;
-  for (i64 r = 0; r < a.R; ++r) {
-    float p = 1.0f;
-    for (int k = 0; k < a.nd; ++k) p = p * rows[k][r];
-    if (a.w) p = p * a.w[r];
-    acc = acc + p;
+  floatx4 acc[T][T];  // [column tile][row tile]
+#pragma unroll
+  for (int j = 0; j < T; ++j)
+#pragma unroll
+    for (int i = 0; i < T; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const float* sr = sk + (16 * T * (wave >> 1) + c) * PITCH + 4 * g;
+  const float* sc = sk + (TILE + 16 * T * (wave & 1) + c) * PITCH + 4 * g;
+  for (i64 r0 = 0; r0 < a.R; r0 += KT) {
+    __syncthreads();  // indices written, or the previous chunk read
+    // one side at a time: a thread's units (4 ranks of one row each) load their
+    // rows of one factor together
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      constexpr int UN = TILE * (KT / 4) / 256;
+      const int q4 = 4 * (tid % (KT / 4));
+      const i64 r = r0 + q4;
+      floatx4 v[UN];
+#pragma unroll
+      for (int u = 0; u < UN; ++u) v[u] = floatx4{1.f, 1.f, 1.f, 1.f};
+      const int k0 = side ? a.h : 0, k1 = side ? a.nd : a.h;
+      for (int k = k0; k < k1; ++k) {
+        const float* Fk = a.F[k];
+        if (a.vec) {
+          const i64 rr = r < a.R ? r : 0;  // ranks past R are zeroed below
+#pragma unroll
+          for (int u = 0; u < UN; ++u)
+            v[u] *= *reinterpret_cast<const floatx4*>(Fk + sidx[k][(tid + 256 * u) / (KT / 4)] * a.R + rr);
+        } else {
+#pragma unroll
+          for (int u = 0; u < UN; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              v[u][q] *= Fk[sidx[k][(tid + 256 * u) / (KT / 4)] * a.R + (r + q < a.R ? r + q : 0)];
+        }
+      }
+      float wq[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) wq[q] = (a.w && side == 0 && r + q < a.R) ? a.w[r + q] : 1.f;
+#pragma unroll
+      for (int u = 0; u < UN; ++u) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[u][q] = r + q < a.R ? v[u][q] * wq[q] : 0.f;
+        *reinterpret_cast<floatx4*>(sk + (side * TILE + (tid + 256 * u) / (KT / 4)) * PITCH + q4) = v[u];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < KT / 16; ++u) {
+      floatx4 rv[T], cv[T];
+#pragma unroll
+      for (int i = 0; i < T; ++i) {
+        rv[i] = *reinterpret_cast<const floatx4*>(sr + 16 * i * PITCH + 16 * u);
+        cv[i] = *reinterpret_cast<const floatx4*>(sc + 16 * i * PITCH + 16 * u);
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < T; ++j)
+#pragma unroll
+          for (int i = 0; i < T; ++i)
+            acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(cv[j][s], rv[i][s], acc[j][i], 0, 0, 0);
+    }
   }
-  if (a.xsub) acc = a.xsub[x] - acc;
-  if (a.gscale) acc = acc * a.gscale[0];
-  out[x] = acc;
+  const float gs = a.gscale ? a.gscale[0] : 1.0f;
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    const i64 row = r_base + 16 * T * (wave >> 1) + 16 * i + c;
+    if (row >= a.M) continue;
+#pragma unroll
+    for (int j = 0; j < T; ++j) {
+      const i64 col = c_base + 16 * T * (wave & 1) + 16 * j + 4 * g;
+      const i64 o = row * a.N + col;
+      floatx4 v = acc[j][i];
+      if constexpr (VS) {
+        if (col < a.N) {
+          if (a.xsub) v = *reinterpret_cast<const floatx4*>(a.xsub + o) - v;
+          if (a.gscale) v *= gs;
+          *reinterpret_cast<floatx4*>(out + o) = v;
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (col + q < a.N) {
+            float x = v[q];
+            if (a.xsub) x = a.xsub[o + q] - x;
+            if (a.gscale) x *= gs;
+            out[o + q] = x;
+          }
+        }
+      }
+    }
+  }
 }
 
 int cp_reconstruct_f32(tenrso_ctx* ctx, int nd, const i64* shape, const float* const* F, i64 R, const float* w,
@@ -88,15 +198,59 @@ int cp_residual_f32(tenrso_ctx* ctx, int nd, const i64* shape, const float* cons
   a.gscale = gscale;
   a.nd = nd;
   a.R = R;
-  a.total = 1;
+  a.w = w;
+  a.vec = R % 4 == 0;
+  i64 total = 1;
   for (int k = 0; k < nd; ++k) {
     a.shape[k] = shape[k];
     a.F[k] = F[k];
-    a.total *= shape[k];
+    a.vec = a.vec && (uintptr_t)F[k] % 16 == 0;
+    total *= shape[k];
   }
-  a.w = w;
-  if (a.total == 0) return TENRSO_OK;
-  hipLaunchKernelGGL(reconstruct_kernel, dim3(cdiv(a.total, 256)), dim3(256), 0, ctx->stream, a, out);
+  if (total == 0) return TENRSO_OK;
+  // The split of the modes into rows and columns of the output matrix that needs
+  // the fewest tiles (the later of equal ones: more factor rows shared by a
+  // workgroup's columns), for 128 x 128 tiles, or 64 x 64 ones where those are
+  // fewer than the CUs (64^3 rank 8: 32 tiles of 128 against 64 of 64).
+  i64 best = 0;
+  int tile = 128;
+  for (int pass = 0; pass < 2; ++pass) {
+    best = 0;
+    i64 M = 1;
+    for (int h = 0; h <= nd; ++h) {
+      const i64 N = total / M, tiles = ((M + tile - 1) / tile) * ((N + tile - 1) / tile);
+      if (best == 0 || tiles <= best) {
+        best = tiles;
+        a.h = h;
+        a.M = M;
+        a.N = N;
+      }
+      if (h < nd) M *= shape[h];
+    }
+    if (pass == 1 || best >= ctx->num_cus) break;
+    tile = 64;
+  }
+  if (best > (i64)INT32_MAX) {
+    set_error("reconstruction of %lld elements exceeds the launch bound", (long long)total);
+    return TENRSO_ERR_UNSUPPORTED;
+  }
+  a.ctiles = cdiv(a.N, tile);
+  const bool vs = a.N % 4 == 0 && (uintptr_t)out % 16 == 0 && (!X || (uintptr_t)X % 16 == 0);
+  auto launch = [&](auto kt, auto t) {
+    if (vs)
+      hipLaunchKernelGGL((reconstruct_kernel<decltype(kt)::value, decltype(t)::value, true>), dim3((unsigned)best),
+                         dim3(256), 0, ctx->stream, a, out);
+    else
+      hipLaunchKernelGGL((reconstruct_kernel<decltype(kt)::value, decltype(t)::value, false>), dim3((unsigned)best),
+                         dim3(256), 0, ctx->stream, a, out);
+  };
+  auto by_rank = [&](auto t) {
+    if (R <= 16) launch(std::integral_constant<int, 16>{}, t);
+    else if (R <= 32) launch(std::integral_constant<int, 32>{}, t);
+    else launch(std::integral_constant<int, 64>{}, t);
+  };
+  if (tile == 128) by_rank(std::integral_constant<int, 4>{});
+  else by_rank(std::integral_constant<int, 2>{});
   TENRSO_HIP_TRY(hipGetLastError());
   return TENRSO_OK;
 }
