@@ -66,8 +66,8 @@ struct tenrso_ctx {
   void* pinned = nullptr;            // small pinned (coherent) host buffer for scalar readback
   double* pinned_dev = nullptr;      // the same buffer as a device pointer (kernels write the fit there)
   // workgroups per CU of each MTTKRP kernel instance (occupancy query cache)
-  const void* occ_kern[32] = {};
-  int occ_val[32] = {};
+  const void* occ_kern[64] = {};
+  int occ_val[64] = {};
   int occ_n = 0;
   void* blas = nullptr;              // rocBLAS handle of the n-mode products, made on first use
   // side stream of the wide-rank ALS job (made on first use): the job overlaps the

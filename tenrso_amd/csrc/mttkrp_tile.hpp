@@ -1,0 +1,312 @@
+// mttkrp_tile.hpp -- what the MFMA MTTKRP kernels share: their arguments, the LDS
+// window of the fastest mode, the block schedule of a wave and the fixed-order
+// reduction of a workgroup.
+#pragma once
+#include <type_traits>
+
+#include "als_job.hpp"
+#include "mttkrp.hpp"
+
+namespace tenrso {
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+
+struct KernArgs {
+  i64 I, Q;           // X viewed as [P, I, Q]
+  i64 R;              // factor row stride (rank)
+  i64 fast_size;      // size of the fastest other mode
+  i64 fast_stride;    // its extent in memory: fast_size, or more in a copy whose last
+                      // mode is padded (Q is then the padded extent too)
+  i64 qs;             // Q / fast_stride: slow indices per p (case A)
+  const float* pre;   // PRE (rows = J / fast_size, stride R) or null (= 1)
+  const float* fast;  // FAST factor (fast_size x R)
+  int kw;             // window of the fastest mode held in LDS (multiple of KB, divides fast_size)
+  int nwin;           // fast_size / kw
+  i64 n_slow;         // J / fast_size
+  i64 total;          // elements of X in memory
+  int slow_splits;    // splits of the slow range; grid.y = nwin * slow_splits
+  i64 slow_q, slow_rem;  // n_slow = slow_q * slow_splits + slow_rem
+  int r0;             // first rank column of this launch
+  int rcount;         // rank columns handled by the launch (<= 16*NT)
+  int rtiles;         // row tiles; workgroup tile -> (tile % rtiles, split = tile / rtiles)
+  int win_vec;        // FAST 16-byte aligned and R % 4 == 0: 16-byte window loads
+};
+
+__device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
+  uint32_t u = __float_as_uint(f);
+  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);  // quiet NaN
+  u += 0x7fffu + ((u >> 16) & 1u);
+  return (uint16_t)(u >> 16);
+}
+
+// Stage FAST[w*kw .. w*kw+kw) (columns r0 .. r0+RT) into LDS transposed: s[r][kk].
+// Work unit u of the workgroup covers ranks r4 .. r4+3 (r4 = 4*(u % (RT/4))) of
+// window rows kk = 2*(u / (RT/4)) and kk + 1, so it leaves LDS as one 8-byte
+// (fp32) or two 4-byte (bf16 hi, lo) pairs per rank.  With a 16-byte aligned
+// FAST and R % 4 == 0 (win_vec) a unit is two 16-byte loads, else eight 4-byte
+// loads (one kernel instance per case, so that every instance has a single
+// load sequence and the waits stay exact).  Ranks past rcount and rows past kw load column r0 of window row 0
+// instead (always inside FAST): those rank columns are never stored and those
+// rows never read, so no value select is needed and no load waits early.
+// Split in two so the window loads are issued before the first X blocks: the
+// LDS writes then wait for the window only (vector loads retire in issue order).
+template <int RT, int NTH, int KWMAX>
+struct FastWindow {
+  static constexpr int UNITS = RT / 4 * (KWMAX / 2);
+  static constexpr int PERU = (UNITS + NTH - 1) / NTH;
+  // every unit index below PERU*NTH maps in bounds: u >= UNITS gives kk >= KWMAX
+  static __device__ __forceinline__ bool live(int u) { return UNITS % NTH == 0 || u < UNITS; }
+  floatx4 v[PERU][2];
+};
+
+// kv: rows of the window that exist (kw, or fewer in the last window of a
+// fastest mode that kw does not divide); a row past kv is read as row 0 (always
+// inside FAST) and stored as zero by stage_window_store*.
+template <bool WV, int RT, int NTH, int KWMAX>
+__device__ __forceinline__ void stage_window_load(FastWindow<RT, NTH, KWMAX>& fw, const KernArgs& a, int w, int kv) {
+  const float* base = a.fast + (i64)w * a.kw * a.R + a.r0;
+  if constexpr (WV) {
+#pragma unroll
+    for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e) {
+      const int u = threadIdx.x + e * NTH;
+      const int r4 = 4 * (u % (RT / 4)), kk = 2 * (u / (RT / 4));
+      const bool ok = kk < kv && r4 < a.rcount;
+      const bool ok1 = ok && kk + 1 < kv;
+      const float* p = base + (ok ? kk * a.R + r4 : 0);
+      fw.v[e][0] = *reinterpret_cast<const floatx4*>(p);
+      fw.v[e][1] = *reinterpret_cast<const floatx4*>(p + (ok1 ? a.R : 0));
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e) {
+      const int u = threadIdx.x + e * NTH;
+      const int r4 = 4 * (u % (RT / 4)), kk = 2 * (u / (RT / 4));
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const bool ok = kk < kv && r4 + q < a.rcount;
+        const bool ok1 = ok && kk + 1 < kv;
+        const float* p = base + (ok ? kk * a.R + r4 + q : 0);
+        fw.v[e][0][q] = p[0];
+        fw.v[e][1][q] = p[ok1 ? a.R : 0];
+      }
+    }
+  }
+}
+
+// rows kk >= kv of a staged pair are zero (they meet masked, zero X elements)
+template <int RT, int NTH, int KWMAX>
+__device__ __forceinline__ void window_zero_tail(FastWindow<RT, NTH, KWMAX>& fw, int kv) {
+#pragma unroll
+  for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e) {
+    const int u = threadIdx.x + e * NTH;
+    const int kk = 2 * (u / (RT / 4));
+    if (kk >= kv) fw.v[e][0] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (kk + 1 >= kv) fw.v[e][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+}
+
+template <int RT, int PITCH, int NTH, int KWMAX>
+__device__ __forceinline__ void stage_window_store(float* __restrict__ s, const FastWindow<RT, NTH, KWMAX>& fw) {
+  static_assert(PITCH % 2 == 0, "pairs of window rows are stored as 8-byte words");
+#pragma unroll
+  for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e) {
+    const int u = threadIdx.x + e * NTH;
+    const int r4 = 4 * (u % (RT / 4)), kk = 2 * (u / (RT / 4));
+    if (!FastWindow<RT, NTH, KWMAX>::live(u)) continue;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<float2*>(&s[(r4 + q) * PITCH + kk]) = float2{fw.v[e][0][q], fw.v[e][1][q]};
+  }
+}
+
+// Same window as an exact bf16 pair: FAST = hi + lo with hi = bf16(FAST) and
+// lo = bf16(FAST - hi), so hi + lo carries 16 significant bits.
+template <int RT, int PITCH, int NTH, int KWMAX>
+__device__ __forceinline__ void stage_window_store_bf16x2(uint16_t* __restrict__ shi, uint16_t* __restrict__ slo,
+                                                          const FastWindow<RT, NTH, KWMAX>& fw) {
+  static_assert(PITCH % 2 == 0, "pairs of window rows are stored as 4-byte words");
+#pragma unroll
+  for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e) {
+    const int u = threadIdx.x + e * NTH;
+    const int r4 = 4 * (u % (RT / 4)), kk = 2 * (u / (RT / 4));
+    if (!FastWindow<RT, NTH, KWMAX>::live(u)) continue;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      // v_cvt_pk_bf16_f32 rounds to nearest even, as f32_to_bf16_rne does for
+      // every non-NaN value; element 0 (row kk) is the low half
+      const floatx2 f = {fw.v[e][0][q], fw.v[e][1][q]};
+      const uint32_t hw = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+      const floatx2 r = {f[0] - __uint_as_float(hw << 16), f[1] - __uint_as_float(hw & 0xffff0000u)};
+      const uint32_t lw = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+      const int o = (r4 + q) * PITCH + kk;
+      *reinterpret_cast<uint32_t*>(&shi[o]) = hw;
+      *reinterpret_cast<uint32_t*>(&slo[o]) = lw;
+    }
+  }
+}
+
+// Same window as an exact bf16 triple: FAST = hi + lo + lo2 (hi = bf16(FAST),
+// lo = bf16(FAST - hi), lo2 = bf16(FAST - hi - lo)); each residual is exact in
+// fp32 and the last one has at most 8 significant bits, so for every normal
+// fp32 value hi + lo + lo2 equals FAST exactly.
+template <int RT, int PITCH, int NTH, int KWMAX>
+__device__ __forceinline__ void stage_window_store_bf16x3(uint16_t* __restrict__ shi, uint16_t* __restrict__ slo,
+                                                          uint16_t* __restrict__ slo2,
+                                                          const FastWindow<RT, NTH, KWMAX>& fw) {
+  static_assert(PITCH % 2 == 0, "pairs of window rows are stored as 4-byte words");
+#pragma unroll
+  for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e) {
+    const int u = threadIdx.x + e * NTH;
+    const int r4 = 4 * (u % (RT / 4)), kk = 2 * (u / (RT / 4));
+    if (!FastWindow<RT, NTH, KWMAX>::live(u)) continue;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const floatx2 f = {fw.v[e][0][q], fw.v[e][1][q]};
+      const uint32_t hw = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+      const floatx2 r = {f[0] - __uint_as_float(hw << 16), f[1] - __uint_as_float(hw & 0xffff0000u)};
+      const uint32_t lw = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+      const floatx2 r2 = {r[0] - __uint_as_float(lw << 16), r[1] - __uint_as_float(lw & 0xffff0000u)};
+      const uint32_t l2w = __builtin_bit_cast(uint32_t, __builtin_convertvector(r2, bf16x2));
+      const int o = (r4 + q) * PITCH + kk;
+      *reinterpret_cast<uint32_t*>(&shi[o]) = hw;
+      *reinterpret_cast<uint32_t*>(&slo[o]) = lw;
+      *reinterpret_cast<uint32_t*>(&slo2[o]) = l2w;
+    }
+  }
+}
+
+// Exact three-way bf16 split of 8 fp32 values (see stage_window_store_bf16x3).
+__device__ __forceinline__ void split_bf16x3(const floatx8& x, bf16x8& h, bf16x8& l, bf16x8& l2) {
+  h = __builtin_convertvector(x, bf16x8);
+  const floatx8 r = x - __builtin_convertvector(h, floatx8);
+  l = __builtin_convertvector(r, bf16x8);
+  const floatx8 r2 = r - __builtin_convertvector(l, floatx8);
+  l2 = __builtin_convertvector(r2, bf16x8);
+}
+
+// A value the compiler cannot prove uniform but that is: move it to scalar registers.
+__device__ __forceinline__ i64 uniform_i64(i64 v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)(uint64_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)v >> 32));
+  return (i64)(((uint64_t)hi << 32) | lo);
+}
+
+// PRE row used when the MTTKRP has no PRE factor (a matrix): KR = FAST.
+#define TENRSO_ONES8 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f
+static __device__ float kPreOnes[64] = {TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8,
+                                       TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8};
+#undef TENRSO_ONES8
+
+// Block schedule of one wave.  Block t of the wave is block kb = t % nkb of the
+// slow index s_lo + wave + WAVES*(t / nkb).  Loads run in t order, so the cursor
+// only steps forward, and it stops on the wave's last block (loads past the end
+// are redirected by the kernels to one cache line).  Every X and PRE load is thus unconditional
+// and the wait before a block's MFMAs counts exactly the loads issued after it,
+// which keeps the prefetch in flight.  A wave with no block reads the block of
+// slow index min(s_lo + wave, n_slow - 1), always inside X, and computes nothing.
+// Case A (X as [P, I, Q], slow = p*qs + sq): the block starts at element
+// p*I*Q + sq*fast_size + w*kw + kb*KB.  Case B: the block covers j = slow*fast_size
+// + w*kw + kb*KB onwards, one row of I elements per j.  All fields are uniform.
+template <int STRIDE, int KB, bool CASE_B>
+struct BlockCursor {
+  int kb, nkb;
+  i64 slow, sq, base, wrap;
+
+  // starts at block kb0 of slow index slow0; each slow index has nkb blocks, and
+  // after its last one the cursor moves STRIDE slow indices on
+  __device__ __forceinline__ BlockCursor(const KernArgs& a, i64 slow0, int w, int nkb_, int kb0) {
+    kb = kb0;
+    nkb = nkb_;
+    slow = slow0 < a.n_slow ? slow0 : a.n_slow - 1;
+    if constexpr (!CASE_B) {
+      // 32-bit division whenever the slow range fits (it nearly always does)
+      const i64 p = (a.n_slow >> 32) ? slow / a.qs : (i64)((uint32_t)slow / (uint32_t)a.qs);
+      sq = slow - p * a.qs;
+      base = p * a.I * a.Q + sq * a.fast_stride + (i64)w * a.kw;
+      wrap = a.I * a.Q - a.qs * a.fast_stride;  // from (p, qs) to (p + 1, 0)
+    } else {
+      sq = 0;
+      wrap = 0;
+      base = slow * a.fast_size + (i64)w * a.kw;
+    }
+  }
+  // element offset in X of the block's first element (lane offsets are added on top)
+  __device__ __forceinline__ i64 offset(const KernArgs& a) const {
+    if constexpr (!CASE_B) return base + (i64)kb * KB;
+    else return (base + (i64)kb * KB) * a.I;
+  }
+  __device__ __forceinline__ void step(const KernArgs& a) {
+    if (++kb == nkb) {
+      kb = 0;
+      slow += STRIDE;
+      base += (i64)STRIDE * a.fast_stride;
+      if constexpr (!CASE_B) {
+        sq += STRIDE;
+        while (sq >= a.qs) {
+          sq -= a.qs;
+          base += wrap;
+        }
+      }
+    }
+  }
+};
+
+// Fixed-order reduction of the WAVES per-wave accumulators of a workgroup, spread
+// over the waves: tile q = mt*NT + nt belongs to wave q % WAVES, which adds the
+// WAVES copies of it in wave order 0, 1, .. (one LDS round trip, 16 bytes per
+// lane and tile) and stores it; every wave stores its own tiles, so the partial
+// leaves the workgroup from all waves at once.  LDS use: MT*NT*WAVES*64 floatx4.
+// SYNC: waits first (the LDS window may still be read by other waves).
+template <int MT, int NT, int WAVES, bool SYNC = true>
+__device__ __forceinline__ void wg_reduce_store(floatx4 (&acc)[MT][NT], float* __restrict__ red, int wave, int lane,
+                                                float* __restrict__ out, i64 rows, i64 R, int r0, int rcount,
+                                                i64 row_base, bool case_b) {
+  floatx4* r4 = reinterpret_cast<floatx4*>(red);
+  const int g = lane >> 4, c = lane & 15;
+  if constexpr (SYNC) __syncthreads();  // LDS window no longer read
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const int q = mt * NT + nt;
+      if (q % WAVES != wave) r4[(q * WAVES + wave) * 64 + lane] = acc[mt][nt];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const int q = mt * NT + nt;
+      if (q % WAVES != wave) continue;
+      floatx4 sum = wave == 0 ? acc[mt][nt] : r4[(q * WAVES + 0) * 64 + lane];
+#pragma unroll
+      for (int wv = 1; wv < WAVES; ++wv) sum += wv == wave ? acc[mt][nt] : r4[(q * WAVES + wv) * 64 + lane];
+      if (16 * nt + c >= rcount) continue;
+      const int col = r0 + 16 * nt + c;
+      // D layout (16x16): lane (g, c), register v -> tile row 4g + v, column c
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const i64 row = case_b ? row_base + MT * (4 * g + v) + mt : row_base + 16 * mt + 4 * g + v;
+        if (row < rows) out[row * R + col] = sum[v];
+      }
+    }
+}
+
+// Fold the per-slow accumulator T into acc with the PRE row of that slow index:
+// acc[:, r] += PRE[slow, r] * T[:, r]  (lane (g, c) holds column 16nt + c).
+template <int MT, int NT>
+__device__ __forceinline__ void fold_slow(floatx4 (&acc)[MT][NT], floatx4 (&T)[MT][NT], const float (&pre)[NT]) {
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      acc[mt][nt] += T[mt][nt] * pre[nt];
+      T[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+}
+
+}  // namespace tenrso

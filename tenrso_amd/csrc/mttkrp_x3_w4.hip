@@ -1,0 +1,13 @@
+// mttkrp_x3_w4.hip -- the 4-wave instances of the fp32 MTTKRP.
+#include "mttkrp_x3.hpp"
+#include "mttkrp_x3_kernel.hpp"
+
+namespace tenrso {
+
+const void* mttkrp_x3_kernel_w4(int nt, bool case_b, bool wv, int xl) {
+  if (nt == 1) return x3_pick<1, 4, false>(case_b, wv, xl);
+  if (nt == 2) return x3_pick<2, 4, false>(case_b, wv, xl);
+  return x3_pick<4, 4, false>(case_b, wv, xl);
+}
+
+}  // namespace tenrso
