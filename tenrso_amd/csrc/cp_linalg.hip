@@ -11,6 +11,7 @@
 #include <cfloat>
 
 #include "als_job.hpp"
+#include "als_job_wide.hpp"
 #include "cp_linalg.hpp"
 #include "mttkrp.hpp"
 
@@ -303,227 +304,9 @@ __global__ __launch_bounds__(JOB_THREADS) void als_job_kernel(AlsJob job) {
 }
 
 // ---------------------------------------------------------------- wide-rank job
-// Ranks SOLVE_RMAX + 1 .. WIDE_NE: the steps of the job (the fit, Gamma_n plus
-// regularisation, its inverse with the ridge retry of cp/helpers.rs:477-490) as a
-// kernel of 1024 threads.  Thread t holds, in registers, column t % 128 of rows
-// t / 128 + 8 m (m = 0..15) of the 128 x 128 matrix, the identity outside R x R.
-// The inverse is Gauss-Jordan with scalar pivots in diagonal order: step k
-// publishes row k and column k (double-buffered in LDS, one barrier a step) and
-// every thread updates its entries from them.  For a symmetric matrix those
-// pivots are the ratios of consecutive leading principal minors, so all of them
-// are positive exactly when the matrix is positive definite: a pivot that is not
-// positive (or not finite) fails the attempt, as a pivot block that is not
-// positive definite fails it in the job of rank <= 64.
-constexpr int WIDE_THREADS = 1024;
-constexpr int WIDE_RPT = WIDE_NE * WIDE_NE / WIDE_THREADS;  // entries per thread
-
-__device__ __forceinline__ double wide_block_sum(double v, double* red) {
-  v = wave_sum(v);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  double s = 0.0;
-#pragma unroll
-  for (int w = 0; w < WIDE_THREADS / 64; ++w) s += red[w];
-  return s;
-}
-
-// 4 x 4 inverse by scalar Gauss-Jordan in registers (every index fixed at compile
-// time); false if a pivot is not positive and finite.
-constexpr int WB = 4;  // pivots per elimination step of the wide-rank inverse
-__device__ __forceinline__ bool wide_inv4(double (&P)[WB][WB]) {
-  bool ok = true;
-#pragma unroll
-  for (int k = 0; k < WB; ++k) {
-    const double p = P[k][k];
-    ok = ok && p > 0.0 && p <= DBL_MAX;
-    const double piv = job_recip(p);
-    double rj[WB], cc[WB];
-#pragma unroll
-    for (int q = 0; q < WB; ++q) {
-      rj[q] = q == k ? 0.0 : P[k][q] * piv;
-      cc[q] = P[q][k];
-    }
-#pragma unroll
-    for (int r = 0; r < WB; ++r)
-#pragma unroll
-      for (int q = 0; q < WB; ++q) P[r][q] = fma(-cc[r], rj[q], P[r][q]);
-#pragma unroll
-    for (int q = 0; q < WB; ++q) {
-      if (q != k) {
-        P[k][q] = rj[q];
-        P[q][k] = -cc[q] * piv;
-      }
-    }
-    P[k][k] = piv;
-  }
-  return ok;
-}
-
-// In-place inverse of the matrix held as described above; false if a pivot
-// block is not positive definite.  Every thread returns at the same step.  Block
-// Gauss-Jordan with 4 x 4 pivot blocks J = {k0..k0+3} (the order padded to a
-// multiple of 4 with the identity), one barrier a step.  With P^-1 = A[J][J]^-1
-// and W = P^-1 A[J][:] (taken as 0 on the columns J):
-//   A[i][j] -= sum_q A[i][J_q] W[q][j]    every entry (columns J stay as they were),
-//   A[J][j]  = W[:, j]                    rows J (the four waves' rows holding them),
-//   A[i][J]  = -A[i][J] P^-1, A[J][J] = P^-1   columns J (four threads per row group).
-// Every thread inverts P itself from the published rows.  The pivot blocks are
-// positive definite exactly when the matrix is (their leading minors are ratios
-// of the matrix's), so the scalar pivots inside them decide the ridge retry.
-// Rows J are published as rk[r][j]; columns J as ck[((i % 8) * 16 + i / 8) * 4 + q],
-// each thread's 64 values contiguous.
-__device__ bool wide_gauss_jordan(double (&a)[WIDE_RPT], int R, double* rowb, double* colb) {
-  const int j = threadIdx.x & (WIDE_NE - 1), i0 = threadIdx.x >> 7;
-  const int Rp = (R + WB - 1) / WB * WB;
-  for (int k0 = 0; k0 < Rp; k0 += WB) {
-    double* rk = rowb + ((k0 / WB) & 1) * WB * WIDE_NE;
-    double* ck = colb + ((k0 / WB) & 1) * WB * WIDE_NE;
-    const int mk = k0 >> 3;          // rows k0..k0+3 are entry mk of their threads
-    const int r_own = i0 - (k0 & 7);
-    const bool row_owner = r_own >= 0 && r_own < WB;  // uniform per wave
-    const int q_own = j - k0;
-    const bool col_owner = q_own >= 0 && q_own < WB;
-    if (row_owner) {
-      // row k0 + r_own, selected without a run-time register index
-      double v = 0.0;
-#pragma unroll
-      for (int m = 0; m < WIDE_RPT; ++m) v = m == mk ? a[m] : v;
-      rk[r_own * WIDE_NE + j] = v;
-    }
-    if (col_owner) {
-#pragma unroll
-      for (int m = 0; m < WIDE_RPT; ++m) ck[(i0 * WIDE_RPT + m) * WB + q_own] = a[m];
-    }
-    __syncthreads();
-    double P[WB][WB], rr[WB];
-#pragma unroll
-    for (int r = 0; r < WB; ++r) {
-#pragma unroll
-      for (int q = 0; q < WB; ++q) P[r][q] = rk[r * WIDE_NE + k0 + q];
-      rr[r] = rk[r * WIDE_NE + j];
-    }
-    if (!wide_inv4(P)) {
-      __syncthreads();  // every thread has read the buffers before they are reused
-      return false;
-    }
-    // one pass of four FMAs per entry: columns J start from 0 and take column
-    // q_own of P^-1 (A[i][J] -> -A[i][J] P^-1), the others start from A[i][j] and
-    // take W[:, j] = P^-1 A[J][j]
-    double X[WB];
-#pragma unroll
-    for (int q = 0; q < WB; ++q) {
-      double w = 0.0;
-#pragma unroll
-      for (int r = 0; r < WB; ++r) w = fma(P[q][r], rr[r], w);
-      const double pq = q_own == 0 ? P[q][0] : (q_own == 1 ? P[q][1] : (q_own == 2 ? P[q][2] : P[q][3]));
-      X[q] = col_owner ? pq : w;
-    }
-    const double* cl = ck + i0 * WIDE_RPT * WB;
-#pragma unroll
-    for (int m = 0; m < WIDE_RPT; ++m) {
-      double v = col_owner ? 0.0 : a[m];
-#pragma unroll
-      for (int q = 0; q < WB; ++q) v = fma(-cl[m * WB + q], X[q], v);
-      a[m] = v;
-    }
-    if (row_owner) {
-      // rows J: W[r_own][j], or P^-1[r_own][q_own] on the columns J
-      const double xo = r_own == 0 ? X[0] : (r_own == 1 ? X[1] : (r_own == 2 ? X[2] : X[3]));
-#pragma unroll
-      for (int m = 0; m < WIDE_RPT; ++m) a[m] = m == mk ? xo : a[m];
-    }
-  }
-  return true;
-}
-
-__global__ __launch_bounds__(WIDE_THREADS) void als_job_wide_kernel(AlsJob a) {
-  __shared__ double rowb[2 * WB * WIDE_NE], colb[2 * WB * WIDE_NE];
-  __shared__ double red0[WIDE_THREADS / 64], red1[WIDE_THREADS / 64];
-  const int R = a.R;
-  const int j = threadIdx.x & (WIDE_NE - 1), i0 = threadIdx.x >> 7;
-  double ipv = 0.0;
-  if (a.do_fit)
-    for (int b = threadIdx.x; b < a.nblk; b += WIDE_THREADS) ipv += a.ip_part[b];
-  // two passes over the Grams, each with one accumulator per entry in registers:
-  // the fit's hadamard of all k, then Gamma's hadamard of k != skip
-  auto hadamard = [&](double (&h)[WIDE_RPT], int skip) {
-#pragma unroll
-    for (int m = 0; m < WIDE_RPT; ++m) h[m] = 1.0;
-    for (int k = 0; k < a.nd; ++k) {
-      if (k == skip) continue;
-      const double* Gk = a.G + (i64)k * R * R + j;
-#pragma unroll
-      for (int m = 0; m < WIDE_RPT; ++m) {
-        const int i = i0 + 8 * m;
-        h[m] *= (i < R && j < R) ? Gk[i * R] : 0.0;
-      }
-    }
-  };
-  if (a.do_fit) {
-    // ||Xhat||^2 = sum_{r,s} prod_k G_k[r,s] (entries outside R x R are 0)
-    double cross[WIDE_RPT];
-    hadamard(cross, -1);
-    double rec = 0.0;
-#pragma unroll
-    for (int m = 0; m < WIDE_RPT; ++m) rec += cross[m];
-    const double recon = wide_block_sum(rec, red0);
-    const double ip = wide_block_sum(ipv, red1);
-    if (threadIdx.x == 0) {
-      double blk[JOB_SC_STAMP];
-#pragma unroll
-      for (int i = 0; i < JOB_SC_STAMP; ++i) blk[i] = a.scal[i];
-      const double nx = blk[JOB_SC_NORM_X];
-      const double err_sq = nx + recon - 2.0 * ip;
-      const double err = sqrt(err_sq > 0.0 ? err_sq : 0.0);
-      double fit = 1.0 - err / sqrt(nx);
-      fit = fit < 0.0 ? 0.0 : (fit > 1.0 ? 1.0 : fit);
-      blk[JOB_SC_FIT] = fit;
-      blk[JOB_SC_IP] = ip;
-      blk[JOB_SC_RECON] = recon;
-      a.scal[JOB_SC_FIT] = fit;
-      a.scal[JOB_SC_IP] = ip;
-      a.scal[JOB_SC_RECON] = recon;
-      if (a.host) {
-#pragma unroll
-        for (int i = 0; i < JOB_SC_STAMP; ++i) a.host[i] = blk[i];
-        __threadfence_system();
-        a.host[JOB_SC_STAMP] = a.stamp;
-      }
-    }
-  }
-  double gam[WIDE_RPT];
-  if (a.skip >= 0) hadamard(gam, a.skip);
-  if (a.gate) {
-    __syncthreads();  // every thread has its Grams
-    if (threadIdx.x == 0) __hip_atomic_store(a.gate, a.gate_stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  if (a.skip < 0) return;
-  // Gamma waits in Winv for the ridge retry (each thread rereads its own entries)
-  double w[WIDE_RPT];
-  auto form = [&](double ridge) {
-#pragma unroll
-    for (int m = 0; m < WIDE_RPT; ++m) {
-      const int i = i0 + 8 * m;
-      const double g = a.Winv[i * WIDE_NE + j];
-      w[m] = (i < R && j < R) ? g + job_reg(a, i, j, ridge) : (i == j ? 1.0 : 0.0);
-    }
-  };
-#pragma unroll
-  for (int m = 0; m < WIDE_RPT; ++m) a.Winv[(i0 + 8 * m) * WIDE_NE + j] = gam[m];
-  form(0.0);
-  bool ok = wide_gauss_jordan(w, R, rowb, colb);
-  int path = 0;
-  if (!ok) {
-    form((double)FLT_EPSILON * (double)(10 * R));
-    ok = wide_gauss_jordan(w, R, rowb, colb);
-    path = ok ? 1 : 2;
-  }
-#pragma unroll
-  for (int m = 0; m < WIDE_RPT; ++m) a.Winv[(i0 + 8 * m) * WIDE_NE + j] = ok ? w[m] : 0.0;
-  if (threadIdx.x == 0 && a.scal) {
-    const double prev = a.scal[a.status_slot];
-    a.scal[a.status_slot] = a.status_reset ? (double)path : fmax(prev, (double)path);
-  }
+__global__ __launch_bounds__(WIDE_THREADS) void als_job_wide_kernel(AlsJob job) {
+  __shared__ __attribute__((aligned(16))) double lds[WIDE_LDS_BYTES / 8];
+  als_job_wide_run(job, lds);
 }
 
 int job_join(tenrso_ctx* ctx) {
@@ -566,30 +349,33 @@ int als_job_launch(tenrso_ctx* ctx, const AlsJob& job) {
 }
 
 // ---------------------------------------------------------------- row solve
-// grid: rows (one workgroup per row); 256 threads = 4 split quarters x 64
-// columns.  Each thread sums a quarter of the MTTKRP split partials of its
-// column (all loads in flight, FP64), the quarters are added in fixed order,
-// then A[i, c] = epi(sum_r M[i, r] Winv[r, c]) (the r-sum split over the same
-// four thread groups) and the block's <M, A> partial is written.
-constexpr int NE = JOB_NE;  // stride of Winv
+// grid: rows (one workgroup per row); 4 NC threads = 4 split quarters x NC columns
+// (NC = 64, or 128 above rank 64: the order and stride of Winv).  Each thread sums a
+// quarter of the MTTKRP split partials of its column (all loads in flight, FP64),
+// the quarters are added in fixed order, then A[i, c] = epi(sum_r M[i, r]
+// Winv[r, c]) (the r-sum split over the same four thread groups) and the block's
+// <M, A> partial is written.  A thread's quarter of its Winv column is loaded beside
+// the partials: one memory round trip (256 rows at rank 128: 13.6 us with the loads
+// behind the partials, in two halves).
 constexpr int SOLVE_RB = 1;
 
-__global__ __launch_bounds__(256) void solve_rows_kernel(const float* __restrict__ part, int splits,
-                                                         const double* __restrict__ M64, i64 rows, int R,
-                                                         const double* __restrict__ Winv, double l1, int nonneg,
-                                                         float* __restrict__ A, double* __restrict__ ip_part) {
-  __shared__ double sq[4 * NE];
-  __shared__ double sM[NE];
-  __shared__ double red[4];
-  const int c = threadIdx.x & 63, qd = threadIdx.x >> 6;
+template <int NC>
+__global__ __launch_bounds__(4 * NC) void solve_rows_kernel(const float* __restrict__ part, int splits,
+                                                            const double* __restrict__ M64, i64 rows, int R,
+                                                            const double* __restrict__ Winv, double l1, int nonneg,
+                                                            float* __restrict__ A, double* __restrict__ ip_part) {
+  __shared__ double sq[4 * NC];
+  __shared__ double sM[NC];
+  __shared__ double red[NC / 64];
+  const int c = threadIdx.x % NC, qd = threadIdx.x / NC;
   const i64 row = blockIdx.x;
   const bool colok = c < R;
   // this thread's quarter of Winv column c, loaded beside the partials (it does
-  // not depend on them): one memory round trip instead of two
+  // not depend on them)
   const int r0 = qd * R / 4, r1 = (qd + 1) * R / 4;
-  double w[NE / 4];
+  double w[NC / 4];
 #pragma unroll
-  for (int k = 0; k < NE / 4; ++k) w[k] = (colok && r0 + k < r1) ? Winv[(r0 + k) * NE + c] : 0.0;
+  for (int k = 0; k < NC / 4; ++k) w[k] = (colok && r0 + k < r1) ? Winv[(r0 + k) * NC + c] : 0.0;
   double m = 0.0;
   if (colok) {
     if (part) {
@@ -609,103 +395,41 @@ __global__ __launch_bounds__(256) void solve_rows_kernel(const float* __restrict
       m = M64[row * R + c];
     }
   }
-  sq[qd * NE + c] = m;
+  sq[qd * NC + c] = m;
   __syncthreads();
-  if (qd == 0) sM[c] = (sq[c] + sq[NE + c]) + (sq[2 * NE + c] + sq[3 * NE + c]);
+  if (qd == 0) sM[c] = (sq[c] + sq[NC + c]) + (sq[2 * NC + c] + sq[3 * NC + c]);
   __syncthreads();
-  // x[c] = sum_r M[r] Winv[r, c], r split over the four quarters (two
-  // alternating sums per thread, as before the prefetch)
+  // x[c] = sum_r M[r] Winv[r, c], r split over the four quarters (two alternating
+  // sums per thread)
   double x = 0.0;
   if (colok) {
     double x0 = 0, x1 = 0;
 #pragma unroll
-    for (int k = 0; k < NE / 4; k += 2) {
+    for (int k = 0; k < NC / 4; k += 2) {
       if (r0 + k < r1) x0 += sM[r0 + k] * w[k];
       if (r0 + k + 1 < r1) x1 += sM[r0 + k + 1] * w[k + 1];
     }
     x = x0 + x1;
   }
-  sq[qd * NE + c] = x;
+  sq[qd * NC + c] = x;
   __syncthreads();
   double ip = 0.0;
   if (qd == 0 && colok) {
-    double xv = (sq[c] + sq[NE + c]) + (sq[2 * NE + c] + sq[3 * NE + c]);
+    double xv = (sq[c] + sq[NC + c]) + (sq[2 * NC + c] + sq[3 * NC + c]);
     if (l1 > 0.0) xv = xv > l1 ? xv - l1 : (xv < -l1 ? xv + l1 : 0.0);  // soft_threshold (helpers.rs:610-623)
     if (nonneg) xv = xv > 0.0 ? xv : 0.0;                                  // core.rs:357-360
     const float x32 = (float)xv;
     A[row * R + c] = x32;
     ip = sM[c] * (double)x32;
   }
-  if (qd == 0) {
-    ip = wave_sum(ip);
-    if (c == 0 && ip_part) ip_part[blockIdx.x] = ip;
+  if (qd == 0) ip = wave_sum(ip);
+  if constexpr (NC == 64) {
+    if (threadIdx.x == 0 && ip_part) ip_part[blockIdx.x] = ip;
+  } else {
+    if (qd == 0 && (c & 63) == 0) red[c >> 6] = ip;
+    __syncthreads();
+    if (threadIdx.x == 0 && ip_part) ip_part[blockIdx.x] = red[0] + red[1];
   }
-  (void)red;
-}
-
-// Ranks SOLVE_RMAX + 1 .. WIDE_NE: the same row solve with Winv of stride
-// WIDE_NE; 256 threads = 2 halves x 128 columns (each half sums half of the
-// split partials, then half of the r-sum), one row per workgroup.
-__global__ __launch_bounds__(256) void solve_rows_wide_kernel(const float* __restrict__ part, int splits,
-                                                              const double* __restrict__ M64, i64 rows, int R,
-                                                              const double* __restrict__ Winv, double l1, int nonneg,
-                                                              float* __restrict__ A, double* __restrict__ ip_part) {
-  __shared__ double sq[2 * WIDE_NE];
-  __shared__ double sM[WIDE_NE];
-  __shared__ double red[2];
-  const int c = threadIdx.x & (WIDE_NE - 1), h = threadIdx.x >> 7;
-  const i64 row = blockIdx.x;
-  const bool colok = c < R;
-  double m = 0.0;
-  if (colok) {
-    if (part) {
-      const i64 n = rows * R, off = row * R + c;
-      const int s0 = h * splits / 2, s1 = (h + 1) * splits / 2;
-      double a0 = 0, a1 = 0;
-      int sp = s0;
-      for (; sp + 2 <= s1; sp += 2) {
-        a0 += (double)part[(i64)sp * n + off];
-        a1 += (double)part[(i64)(sp + 1) * n + off];
-      }
-      if (sp < s1) a0 += (double)part[(i64)sp * n + off];
-      m = a0 + a1;
-    } else if (h == 0) {
-      m = M64[row * R + c];
-    }
-  }
-  sq[h * WIDE_NE + c] = m;
-  __syncthreads();
-  if (h == 0) sM[c] = sq[c] + sq[WIDE_NE + c];
-  __syncthreads();
-  double x = 0.0;
-  if (colok) {
-    const int r0 = h * R / 2, r1 = (h + 1) * R / 2;
-    double x0 = 0, x1 = 0;
-    int r = r0;
-    for (; r + 2 <= r1; r += 2) {
-      x0 += sM[r] * Winv[(i64)r * WIDE_NE + c];
-      x1 += sM[r + 1] * Winv[(i64)(r + 1) * WIDE_NE + c];
-    }
-    if (r < r1) x0 += sM[r] * Winv[(i64)r * WIDE_NE + c];
-    x = x0 + x1;
-  }
-  sq[h * WIDE_NE + c] = x;  // the reads of sq above finished before the last barrier
-  __syncthreads();
-  double ip = 0.0;
-  if (h == 0 && colok) {
-    double xv = sq[c] + sq[WIDE_NE + c];
-    if (l1 > 0.0) xv = xv > l1 ? xv - l1 : (xv < -l1 ? xv + l1 : 0.0);  // soft_threshold (helpers.rs:610-623)
-    if (nonneg) xv = xv > 0.0 ? xv : 0.0;                                  // core.rs:357-360
-    const float x32 = (float)xv;
-    A[row * R + c] = x32;
-    ip = sM[c] * (double)x32;
-  }
-  if (h == 0) {
-    ip = wave_sum(ip);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ip;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0 && ip_part) ip_part[blockIdx.x] = red[0] + red[1];
 }
 
 int solve_rows(tenrso_ctx* ctx, const float* part, int splits, const double* M, i64 rows, i64 R,
@@ -719,10 +443,10 @@ int solve_rows(tenrso_ctx* ctx, const float* part, int splits, const double* M, 
   }
   TENRSO_TRY(job_join(ctx));  // Winv of a wide-rank job on the side stream
   if (R > SOLVE_RMAX)
-    hipLaunchKernelGGL(solve_rows_wide_kernel, dim3(nblk), dim3(256), 0, ctx->stream, part, splits, M, rows, (int)R,
+    hipLaunchKernelGGL(solve_rows_kernel<WIDE_NE>, dim3(nblk), dim3(4 * WIDE_NE), 0, ctx->stream, part, splits, M, rows, (int)R,
                        Winv, epi.l1, epi.nonneg, A, ip_part);
   else
-    hipLaunchKernelGGL(solve_rows_kernel, dim3(nblk), dim3(256), 0, ctx->stream, part, splits, M, rows, (int)R, Winv,
+    hipLaunchKernelGGL(solve_rows_kernel<JOB_NE>, dim3(nblk), dim3(4 * JOB_NE), 0, ctx->stream, part, splits, M, rows, (int)R, Winv,
                        epi.l1, epi.nonneg, A, ip_part);
   TENRSO_HIP_TRY(hipGetLastError());
   return TENRSO_OK;

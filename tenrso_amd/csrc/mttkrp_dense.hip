@@ -756,7 +756,11 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
 
   const i64 I = pl.I;
   const i64 nout = I * R;
-  const int RT = R <= 16 ? 16 : (R <= 32 ? 32 : 64);
+  // rank columns of a launch: up to 64, or 128 of an fp32 tensor (for ranks 65 to 128
+  // one pass over X, which can carry the wide-rank job: an ALS mode at 256^3 rank 128
+  // takes 48 us so, against two launches of 25 us beside the job on a side stream and
+  // about 28 us of waits between the streams)
+  const int RT = R <= 16 ? 16 : (R <= 32 ? 32 : (R <= 64 || (bf16 && !x3) ? 64 : 128));
   const int NT = RT / 16;
   const int rchunks = (int)((R + RT - 1) / RT);
 
@@ -901,12 +905,13 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
     // the job shares the launch it takes one of the resident slots, so every
     // workgroup is resident at once.
     int waves = 8, occ = 0;
-    const void* kern = fp32 ? mttkrp_x3_kernel_w8(NT, caseB, a.win_vec, XL)
-                            : mttkrp_bf16_kernel(NT, a.win_vec, KB / 32, XL);
+    const void* kern = !fp32 ? mttkrp_bf16_kernel(NT, a.win_vec, KB / 32, XL)
+                             : (NT == 8 ? mttkrp_x3_kernel_n8(caseB, a.win_vec, XL)
+                                        : mttkrp_x3_kernel_w8(NT, caseB, a.win_vec, XL));
     TENRSO_TRY(occupancy(kern, waves * 64, &occ));
     int wpc = bf16 ? ctx->wg_per_cu_bf16 : ctx->wg_per_cu_f32;  // TENRSO_WG_PER_CU_* override
     if (wpc <= 0) wpc = std::min(occ, 2);
-    const bool fuse_job = job != nullptr && rchunks == 1;
+    const bool fuse_job = job != nullptr && rchunks == 1 && (job->R <= JOB_NE || NT == 8);
     i64 target = (i64)wpc * ctx->num_cus - ((fuse_job && occ <= wpc) ? 1 : 0);
     // Splits of the slow range: the count with the least (rounds of resident
     // workgroups) x (blocks of its slowest wave + 3), a workgroup's start and end
@@ -927,7 +932,7 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
     // Several rounds and no job: 4-wave workgroups, as many splits as bring 1.5
     // times the resident ones while a wave keeps four blocks (9216 rows, 9216 j,
     // rank 32: 75 us with 576 workgroups, 70 with 1152, 69 with 1728).
-    if (fp32 && !fuse_job && wgs1 * ssp > target) {
+    if (fp32 && NT < 8 && !fuse_job && wgs1 * ssp > target) {
       kern = mttkrp_x3_kernel_w4(NT, caseB, a.win_vec, XL);
       waves = 4;
       TENRSO_TRY(occupancy(kern, waves * 64, &occ));

@@ -197,8 +197,9 @@ __device__ __forceinline__ i64 uniform_i64(i64 v) {
 
 // PRE row used when the MTTKRP has no PRE factor (a matrix): KR = FAST.
 #define TENRSO_ONES8 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f
-static __device__ float kPreOnes[64] = {TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8,
-                                       TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8};
+static __device__ float kPreOnes[128] = {
+    TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8,
+    TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8};
 #undef TENRSO_ONES8
 
 // Block schedule of one wave.  Block t of the wave is block kb = t % nkb of the

@@ -19,13 +19,17 @@
 // that is not finite; the largest magnitudes of every row and column, kept on the
 // way), and the workgroup then forms its tile again in plain fp32 arithmetic.
 #pragma once
+#include "als_job_wide.hpp"
 #include "mttkrp_tile.hpp"
 
 namespace tenrso {
 
 namespace {
 
-constexpr int X3_NBUF = 3;     // blocks of X in registers: two in flight (three more cost registers: 18.6 us)
+// blocks of X in registers: two in flight (three cost registers: 18.6 us against
+// 18.0 at 256^3 rank 64), one where eight rank tiles take the registers
+template <int NT>
+constexpr int X3_NBUF = NT == 8 ? 2 : 3;
 constexpr int X3_KWMAX = 128;  // rows of the LDS window
 
 // x - h of a pair, h the pair rounded to bf16: one v_dot2 each (h_0 -1 + h_1 0 + x_0),
@@ -101,34 +105,40 @@ __device__ __forceinline__ void x3_plain_tile(const float* X, const KernArgs& a,
 //    16-byte (8-byte in case B) vectors at any 4-byte alignment, which this
 //    hardware serves; elements past the window's end are read (they are the next
 //    row's) and zeroed, except where that would pass the end of X.
-// Two forms.  JOB: 8 waves and the inlined ALS job, whose registers (235) leave one
+// Forms.  JOB 1: 8 waves and the inlined ALS job, whose registers (235) leave one
 // workgroup a CU: the form of launches that carry the job or fill the GPU in one
-// round.  Without it, 4 waves: two (NT = 4) to four workgroups a CU, so that where
+// round.  JOB 2: the same with the job of ranks 65 to 128, for eight rank tiles (one
+// pass over X and one split of it instead of two).  JOB 0: 4 waves: two (NT = 4) to four workgroups a CU, so that where
 // a CU runs several one after another the end of one meets the loop of the next
 // (9216 rows x 9216 j at rank 32: 69-73 us against 77-85 us; one full round at
 // 256^3 rank 64: 19.1 us against 18.4 us).
-template <int NT, int WAVES, bool JOB, bool CASE_B, bool WV, int XL>
+template <int NT, int WAVES, int JOB, bool CASE_B, bool WV, int XL>
 __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __restrict__ X, KernArgs a,
                                                                 float* __restrict__ partial, AlsJob job,
                                                                 int has_job) {
-  constexpr int MT = 2, NBUF = X3_NBUF, KWMAX = X3_KWMAX;
+  constexpr int MT = 2, NBUF = X3_NBUF<NT>, KWMAX = X3_KWMAX;
   constexpr int KB = 32, PITCH = KWMAX + 8, RT = 16 * NT, NTH = WAVES * 64, ROWS = 16 * MT;
   constexpr int LDS_WIN = 3 * RT * PITCH * 2, LDS_RED = MT * NT * WAVES * 64 * 16;
   constexpr int LDS_B = LDS_WIN > LDS_RED ? LDS_WIN : LDS_RED;
-  constexpr int LDS_BYTES = !JOB || LDS_B > JOB_LDS_BYTES ? LDS_B : JOB_LDS_BYTES;
+  constexpr int LDS_JOB = JOB == 0 ? 0 : (JOB == 1 ? JOB_LDS_BYTES : WIDE_LDS_BYTES);
+  constexpr int LDS_BYTES = LDS_B > LDS_JOB ? LDS_B : LDS_JOB;
   __shared__ __attribute__((aligned(16))) float smem[LDS_BYTES / 4];
   __shared__ float colmax[WAVES][RT];  // largest magnitude of each window column, by staging wave
   __shared__ int plain;                // a wave asks for the plain form
-  if constexpr (JOB) {
-    static_assert(NTH % JOB_THREADS == 0, "the ALS job runs on the first 256 threads");
-    if (has_job && blockIdx.x == 0) {
-      // waves past the job's four end at once; one such workgroup a CU, so the job
-      // has its CU to itself
-      if (threadIdx.x < JOB_THREADS) als_job_run(job, reinterpret_cast<double*>(smem));
-      return;
+  if (JOB != 0 && has_job && blockIdx.x == 0) {
+    // one such workgroup a CU, so the job has its CU to itself; waves past the
+    // rank-64 job's four end at once
+    double* lds = reinterpret_cast<double*>(smem);
+    if constexpr (JOB == 1) {
+      static_assert(NTH % JOB_THREADS == 0, "the ALS job runs on the first 256 threads");
+      if (threadIdx.x < JOB_THREADS) als_job_run(job, lds);
+    } else if constexpr (JOB == 2) {
+      static_assert(NTH == WIDE_THREADS, "the wide-rank job runs on the whole workgroup");
+      als_job_wide_run(job, lds);
     }
+    return;
   }
-  const int tile = (int)blockIdx.x - (JOB && has_job ? 1 : 0);
+  const int tile = (int)blockIdx.x - (JOB != 0 && has_job ? 1 : 0);
   const int xt = tile % a.rtiles;
   uint16_t* sHi = reinterpret_cast<uint16_t*>(smem);
   uint16_t* sLo = sHi + RT * PITCH;
@@ -375,7 +385,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
   wg_reduce_store<MT, NT, WAVES, false>(acc, smem, wave, lane, out, a.I, a.R, a.r0, a.rcount, row_base, CASE_B);
 }
 
-template <int NT, int WAVES, bool JOB, bool CASE_B, bool WV>
+template <int NT, int WAVES, int JOB, bool CASE_B, bool WV>
 const void* x3_pick_xl(int xl) {
   if constexpr (!CASE_B) {
     if (xl == 4) return reinterpret_cast<const void*>(mttkrp_x3_mfma<NT, WAVES, JOB, CASE_B, WV, 4>);
@@ -384,7 +394,7 @@ const void* x3_pick_xl(int xl) {
   return reinterpret_cast<const void*>(mttkrp_x3_mfma<NT, WAVES, JOB, CASE_B, WV, 1>);
 }
 
-template <int NT, int WAVES, bool JOB>
+template <int NT, int WAVES, int JOB>
 const void* x3_pick(bool case_b, bool wv, int xl) {
   if (case_b) return wv ? x3_pick_xl<NT, WAVES, JOB, true, true>(xl) : x3_pick_xl<NT, WAVES, JOB, true, false>(xl);
   return wv ? x3_pick_xl<NT, WAVES, JOB, false, true>(xl) : x3_pick_xl<NT, WAVES, JOB, false, false>(xl);

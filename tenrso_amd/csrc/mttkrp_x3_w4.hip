@@ -5,9 +5,9 @@
 namespace tenrso {
 
 const void* mttkrp_x3_kernel_w4(int nt, bool case_b, bool wv, int xl) {
-  if (nt == 1) return x3_pick<1, 4, false>(case_b, wv, xl);
-  if (nt == 2) return x3_pick<2, 4, false>(case_b, wv, xl);
-  return x3_pick<4, 4, false>(case_b, wv, xl);
+  if (nt == 1) return x3_pick<1, 4, 0>(case_b, wv, xl);
+  if (nt == 2) return x3_pick<2, 4, 0>(case_b, wv, xl);
+  return x3_pick<4, 4, 0>(case_b, wv, xl);
 }
 
 }  // namespace tenrso

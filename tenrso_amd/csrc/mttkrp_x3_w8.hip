@@ -5,9 +5,9 @@
 namespace tenrso {
 
 const void* mttkrp_x3_kernel_w8(int nt, bool case_b, bool wv, int xl) {
-  if (nt == 1) return x3_pick<1, 8, true>(case_b, wv, xl);
-  if (nt == 2) return x3_pick<2, 8, true>(case_b, wv, xl);
-  return x3_pick<4, 8, true>(case_b, wv, xl);
+  if (nt == 1) return x3_pick<1, 8, 1>(case_b, wv, xl);
+  if (nt == 2) return x3_pick<2, 8, 1>(case_b, wv, xl);
+  return x3_pick<4, 8, 1>(case_b, wv, xl);
 }
 
 }  // namespace tenrso

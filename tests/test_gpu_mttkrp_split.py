@@ -46,7 +46,8 @@ def check(X, F, got):
 # block, two windows, tensors of fewer elements than a vector, more row tiles than the GPU holds at once
 SHAPES = [((1, 2), 1), ((3, 1), 2), ((2, 2, 1), 3), ((5, 7, 1), 16), ((1, 9, 33), 17), ((31, 4, 3), 4), ((33, 2, 31), 8),
           ((32, 2, 32), 64), ((34, 3, 63), 20), ((65, 2, 129), 33), ((3, 130, 35), 48), ((4, 3, 5, 67), 12),
-          ((9000, 2, 20), 8), ((2, 20, 9001), 5), ((3, 9004, 2), 36), ((2, 3, 161), 65)]
+          ((9000, 2, 20), 8), ((2, 20, 9001), 5), ((3, 9004, 2), 36), ((2, 3, 161), 65), ((33, 5, 40), 100),
+          ((35, 4, 33), 127), ((6, 20, 32), 128), ((34, 3, 35), 130)]
 
 
 @pytest.mark.parametrize("offset", [0, 1, 2])
