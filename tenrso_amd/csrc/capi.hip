@@ -361,7 +361,7 @@ int tenrso_cp_init_svd(tenrso_ctx* ctx, const float* X, int ndim, const int64_t*
     return TENRSO_ERR_INVALID_RANK;
   }
   TENRSO_TRY(set_device(ctx));
-  return cp_init_svd(ctx, X, ndim, shape, rank, kind, seed, factors, nullptr);
+  return cp_init_svd(ctx, X, ndim, shape, rank, kind, seed, factors);
 }
 
 int tenrso_cp_als_f32_host(tenrso_ctx* ctx, const float* X, int ndim, const int64_t* shape, float* const* factors,

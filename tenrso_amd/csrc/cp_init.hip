@@ -4,11 +4,12 @@
 // Per mode k (X viewed as [P, I, Q], I = I_k, J = P*Q columns of the unfolding):
 //   1. K = X_(k) X_(k)^T (I x I, FP64): the left singular vectors of X_(k) are the
 //      eigenvectors of K and its singular values the square roots of K's
-//      eigenvalues.  Split-K tiled kernel over the column range, FP64 sums, then a
-//      reduction that also mirrors the upper triangle.
-//   2. One workgroup: cyclic parallel Jacobi (round-robin pairing, all n/2
-//      rotations of a round applied at once: rows, barrier, columns and V) until
-//      the off-diagonal mass is below 1e-14 of the diagonal, then the top R
+//      eigenvalues.  Split-K tiles on the FP64 matrix cores, then a reduction that
+//      also mirrors the upper triangle.
+//   2. Two-sided block Jacobi, every mode at once: pairs of 32-wide blocks (circle
+//      method) are diagonalised by one workgroup each, their 64 x 64 rotations
+//      applied to K and to the eigenvectors by 64 x 64 tiles over the whole GPU,
+//      until the off-diagonal mass is below 1e-14 of the diagonal; then the top R
 //      eigenpairs in descending order.  The sign of each eigenvector is fixed so
 //      that its entry of largest magnitude is positive (an SVD's signs are
 //      arbitrary; the third-party SVD behind the reference does not document one).
@@ -34,18 +35,24 @@
 namespace tenrso {
 
 constexpr int INIT_RMAX = 128;  // rank bound of the SVD-based initialisations (that of the ALS)
+constexpr int JACOBI_SWEEPS = 16;
 
 namespace {
 
-constexpr int GT = 32;          // Gram tile
-constexpr int EIG_THREADS = 1024;
+typedef double doublex4 __attribute__((ext_vector_type(4)));
 
-// Gram partials: workgroup (tile pair, split) sums the columns [j0, j1) of its
-// split for a 32 x 32 tile (ti <= tj) of K.  Thread t computes row t / 8 and
-// columns 4 (t % 8) .. + 3 of the tile in FP64.
+constexpr int GT = 64;  // Gram tile
+constexpr int GK = 32;  // columns staged per step
+
+// Gram partials: workgroup (tile pair, split) sums the columns [j0, j1) of its split
+// for a 64 x 64 tile (ti <= tj) of K on the FP64 matrix cores; each of its 4 waves
+// owns 32 x 32 of it.  32 columns of both row tiles at a time go through LDS as fp32
+// (the next ones loaded meanwhile); element (i, j) of the unfolding is X[p, i, q]
+// with (p, q) = (j / Q, j % Q).  Bound: the FP64 matrix cores, 74 us at 256 rows of
+// 65536 columns at 73 TFLOP/s (32 x 32 tiles of VALU FMAs took 526 us).
 __global__ __launch_bounds__(256) void unfold_gram_partial_kernel(const float* __restrict__ X, i64 P, i64 I, i64 Q,
                                                                   int nt, int splits, double* __restrict__ part) {
-  __shared__ float sA[GT][GT + 1], sB[GT][GT + 1];
+  __shared__ float sA[GT][GK + 4], sB[GT][GK + 4];
   int t = blockIdx.x, ti = 0;
   while (t >= nt - ti) {
     t -= nt - ti;
@@ -55,172 +62,349 @@ __global__ __launch_bounds__(256) void unfold_gram_partial_kernel(const float* _
   const int split = blockIdx.y;
   const i64 J = P * Q;
   const i64 j0 = J * split / splits, j1 = J * (split + 1) / splits;
-  const int tid = threadIdx.x, r = tid >> 3, c4 = (tid & 7) * 4;
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  for (i64 jb = j0; jb < j1; jb += GT) {
-    // stage 32 rows x 32 columns of both row tiles: element (row, col) of the
-    // unfolding is X[p, i, q] with (p, q) = (j / Q, j % Q)
-    for (int e = tid; e < GT * GT; e += 256) {
-      const int rr = e / GT, cc = e % GT;
-      const i64 j = jb + cc;
-      float a = 0.f, b = 0.f;
-      if (j < j1) {
-        const i64 p = j / Q, q = j - (j / Q) * Q;
-        const i64 ia = (i64)ti * GT + rr, ib = (i64)tj * GT + rr;
-        if (ia < I) a = X[(p * I + ia) * Q + q];
-        if (ib < I) b = X[(p * I + ib) * Q + q];
-      }
-      sA[rr][cc] = a;
-      sB[rr][cc] = b;
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int cc = 0; cc < GT; ++cc) {
-      const double a = (double)sA[r][cc];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q4 = lane >> 4, l16 = lane & 15;
+  constexpr int PER = GT * GK / 256;
+  // a thread stages one column of a step: rows tid / 32 + 8 e, or (Q == 1, where
+  // consecutive rows are contiguous) one row: columns tid / 64 + 4 e
+  const bool rowwise = Q != 1;
+  float ra[PER], rb[PER];
+  auto load = [&](i64 jb) {
+    if (rowwise) {
+      const i64 j = jb + (tid & 31);
+      const bool ok = j < j1;
+      const i64 p = ok ? ((J >> 32) ? j / Q : (i64)((uint32_t)j / (uint32_t)Q)) : 0;
+      const float* x = X + (ok ? p * I * Q + (j - p * Q) : 0);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) acc[u] = fma(a, (double)sB[c4 + u][cc], acc[u]);
+      for (int e = 0; e < PER; ++e) {
+        const i64 ia = (i64)ti * GT + (tid >> 5) + 8 * e, ib = (i64)tj * GT + (tid >> 5) + 8 * e;
+        ra[e] = ok && ia < I ? x[ia * Q] : 0.f;
+        rb[e] = ok && ib < I ? x[ib * Q] : 0.f;
+      }
+    } else {
+      const i64 ia = (i64)ti * GT + lane, ib = (i64)tj * GT + lane;
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        const i64 j = jb + wave + 4 * e;
+        ra[e] = j < j1 && ia < I ? X[j * I + ia] : 0.f;
+        rb[e] = j < j1 && ib < I ? X[j * I + ib] : 0.f;
+      }
+    }
+  };
+  auto store = [&]() {
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      const int r = rowwise ? (tid >> 5) + 8 * e : lane, c = rowwise ? (tid & 31) : wave + 4 * e;
+      sA[r][c] = ra[e];
+      sB[r][c] = rb[e];
+    }
+  };
+  doublex4 acc[2][2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int v = 0; v < 2; ++v) acc[u][v] = doublex4{0.0, 0.0, 0.0, 0.0};
+  const int ar = 32 * (wave >> 1) + l16, br = 32 * (wave & 1) + l16;
+  load(j0);
+  for (i64 jb = j0; jb < j1; jb += GK) {
+    store();
+    __syncthreads();
+    if (jb + GK < j1) load(jb + GK);
+#pragma unroll
+    for (int kk = 0; kk < GK / 4; ++kk) {
+      double av[2], bv[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        av[u] = (double)sA[ar + 16 * u][4 * kk + q4];
+        bv[u] = (double)sB[br + 16 * u][4 * kk + q4];
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int v = 0; v < 2; ++v) acc[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u], bv[v], acc[u][v], 0, 0, 0);
     }
     __syncthreads();
   }
   double* out = part + (i64)split * I * I;
-  const i64 i = (i64)ti * GT + r;
-  if (i < I)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const i64 i2 = (i64)tj * GT + c4 + u;
-      if (i2 < I) out[i * I + i2] = acc[u];
-    }
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const i64 i = (i64)ti * GT + 32 * (wave >> 1) + 16 * u + 4 * e + q4;
+        const i64 i2 = (i64)tj * GT + 32 * (wave & 1) + 16 * v + l16;
+        if (i < I && i2 < I) out[i * I + i2] = acc[u][v][e];
+      }
 }
 
-// K[i][i2] = sum of the split partials, for tile(i) <= tile(i2), mirrored below.
-__global__ __launch_bounds__(256) void unfold_gram_reduce_kernel(const double* __restrict__ part, int splits, i64 I,
-                                                                 double* __restrict__ K) {
-  const i64 e = (i64)blockIdx.x * 256 + threadIdx.x;
-  if (e >= I * I) return;
-  const i64 i = e / I, i2 = e - (e / I) * I;
+// The eigenproblem of every mode (by value to the kernels below).  n is padded to a
+// multiple N of 64 with zero rows and columns, which no rotation touches.
+struct EigMode {
+  double* A;    // N x N: K, then diagonal
+  double* V;    // N x N: eigenvectors in columns
+  double* Q;    // [N / 64][64][64]: the rotations of a round
+  int* done;
+  double* U;    // n x R: eigenvectors of the top R, descending
+  double* lam;  // R
+  int n, N;
+};
+struct EigArgs {
+  EigMode m[MAXD];
+  int R;
+};
+
+// K[i][i2] = sum of the split partials, for tile(i) <= tile(i2), mirrored below; V = 1
+__global__ __launch_bounds__(256) void unfold_gram_reduce_kernel(const double* __restrict__ part, int splits,
+                                                                 EigMode m) {
+  const i64 e = (i64)blockIdx.x * 256 + threadIdx.x, I = m.n, N = m.N;
+  if (e == 0) *m.done = 0;
+  if (e >= N * N) return;
+  const i64 i = e / N, i2 = e - (e / N) * N;
+  m.V[e] = i == i2 ? 1.0 : 0.0;
+  if (i >= I || i2 >= I) {
+    m.A[e] = 0.0;
+    return;
+  }
   if (i / GT > i2 / GT) return;
   double s = 0.0;
-  for (int k = 0; k < splits; ++k) s += part[(i64)k * I * I + e];
-  K[i * I + i2] = s;
-  K[i2 * I + i] = s;
+  for (int k = 0; k < splits; ++k) s += part[(i64)k * I * I + i * I + i2];
+  m.A[i * N + i2] = s;
+  m.A[i2 * N + i] = s;
 }
 
-// One workgroup: eigen-decomposition of the symmetric n x n matrix A (in place,
-// global memory), eigenvectors in V; then the top `R` eigenpairs: U (n x R,
-// column r = eigenvector of the r-th largest eigenvalue, largest-magnitude entry
-// positive) and lam (R).  red: EIG_THREADS doubles of scratch is in LDS.
-__global__ __launch_bounds__(EIG_THREADS) void jacobi_eig_kernel(double* __restrict__ A, double* __restrict__ V,
-                                                                 int n, int R, int max_sweeps,
-                                                                 double* __restrict__ U, double* __restrict__ lam,
-                                                                 int* __restrict__ sweeps_out) {
-  __shared__ double cs[2 * 512];  // (c, s) of each pair of a round (n <= 1024)
-  __shared__ double red[EIG_THREADS / 64];
-  __shared__ int done;
-  const int tid = threadIdx.x;
-  const int m = n + (n & 1);  // even count; index n is a dummy when n is odd
-  const int half = m / 2;
-  for (i64 e = tid; e < (i64)n * n; e += EIG_THREADS) V[e] = (e / n == e % n) ? 1.0 : 0.0;
-  auto block_sum = [&](double v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    if ((tid & 63) == 0) red[tid >> 6] = v;
-    __syncthreads();
-    double s = 0.0;
-    for (int w = 0; w < EIG_THREADS / 64; ++w) s += red[w];
-    __syncthreads();
-    return s;
-  };
-  // pair k of round r (circle method): (r, m - 1) for k = 0, else (r + k, r - k) mod m - 1
-  auto pair_of = [&](int r, int k, int& a, int& b) {
-    if (k == 0) {
-      a = r;
-      b = m - 1;
-    } else {
-      a = (r + k) % (m - 1);
-      b = (r - k + (m - 1)) % (m - 1);
-    }
-  };
-  int sweep = 0;
-  for (; sweep < max_sweeps; ++sweep) {
-    double off = 0.0, dia = 0.0;
-    for (i64 e = tid; e < (i64)n * n; e += EIG_THREADS) {
-      const double v = A[e];
-      if (e / n == e % n) dia += v * v;
+// pair k of round r of the circle method over `count` (even) indices
+__device__ __forceinline__ void circle_pair(int count, int r, int k, int& a, int& b) {
+  a = k == 0 ? r : (r + k) % (count - 1);
+  b = k == 0 ? count - 1 : (r - k + (count - 1)) % (count - 1);
+}
+
+template <int THREADS>
+__device__ __forceinline__ double block_sum(double v, double* red) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double s = 0.0;
+  for (int w = 0; w < THREADS / 64; ++w) s += red[w];
+  __syncthreads();
+  return s;
+}
+
+// done once the off-diagonal mass is below 1e-28 of the diagonal's (squares); one
+// workgroup a mode
+__global__ __launch_bounds__(1024) void jacobi_check_kernel(EigArgs a) {
+  __shared__ double red[16];
+  const EigMode& m = a.m[blockIdx.x];
+  if (*m.done) return;
+  const i64 N = m.N;
+  double off = 0.0, dia = 0.0;
+  for (i64 i = threadIdx.x >> 6; i < N; i += 16)
+    for (i64 j = threadIdx.x & 63; j < N; j += 64) {
+      const double v = m.A[i * N + j];
+      if (i == j) dia += v * v;
       else off += v * v;
     }
-    off = block_sum(off);
-    dia = block_sum(dia);
-    if (tid == 0) done = off <= 1e-28 * dia || off == 0.0;
-    __syncthreads();
-    if (done) break;
-    for (int r = 0; r < m - 1; ++r) {
-      // rotation of every pair from the matrix before the round (NR jacobi form)
-      for (int k = tid; k < half; k += EIG_THREADS) {
-        int a, b;
-        pair_of(r, k, a, b);
+  off = block_sum<1024>(off, red);
+  dia = block_sum<1024>(dia, red);
+  if (threadIdx.x == 0 && (off <= 1e-28 * dia || off == 0.0)) *m.done = 1;
+}
+
+// The rotation of one pair of blocks of round r: cyclic parallel Jacobi on their
+// 64 x 64 submatrix in LDS (63 rounds of 32 disjoint rotations, rows and columns of
+// each 2 x 2 block by one thread), accumulated into Q.  One sweep where the matrix
+// has other blocks, which the next round brings; up to `inner` where it is the whole
+// matrix.
+constexpr int JB = 32;            // block width
+constexpr int JP = 2 * JB;        // order of a pair
+constexpr int JPITCH = JP + 1;    // doubles
+__global__ __launch_bounds__(1024) void jacobi_pair_kernel(EigArgs a, int r) {
+  __shared__ double S[JP * JPITCH], W[JP * JPITCH], cs[JP], red[16];
+  const EigMode& m = a.m[blockIdx.y];
+  const int blocks = m.N / JB;
+  if ((int)blockIdx.x >= blocks / 2 || r >= blocks - 1 || *m.done) return;
+  const int tid = threadIdx.x;
+  int p, q;
+  circle_pair(blocks, r, blockIdx.x, p, q);
+  const i64 N = m.N;
+  for (int e = tid; e < JP * JP; e += 1024) {
+    const int i = e / JP, j = e % JP;
+    const i64 gi = i < JB ? p * JB + i : q * JB + i - JB, gj = j < JB ? p * JB + j : q * JB + j - JB;
+    S[i * JPITCH + j] = m.A[gi * N + gj];
+    W[i * JPITCH + j] = i == j ? 1.0 : 0.0;
+  }
+  __syncthreads();
+  const int inner = blocks == 2 ? 30 : 1;
+  for (int sweep = 0; sweep < inner; ++sweep) {
+    if (sweep > 0) {
+      double off = 0.0, dia = 0.0;
+      for (int e = tid; e < JP * JP; e += 1024) {
+        const double v = S[(e / JP) * JPITCH + e % JP];
+        if (e / JP == e % JP) dia += v * v;
+        else off += v * v;
+      }
+      off = block_sum<1024>(off, red);
+      dia = block_sum<1024>(dia, red);
+      if (off <= 1e-28 * dia || off == 0.0) break;
+    }
+    for (int rr = 0; rr < JP - 1; ++rr) {
+      if (tid < JB) {
+        int i, j;
+        circle_pair(JP, rr, tid, i, j);
+        const double apq = S[i * JPITCH + j];
         double c = 1.0, s = 0.0;
-        if (a < n && b < n) {
-          const double apq = A[(i64)a * n + b];
-          if (apq != 0.0) {
-            const double th = (A[(i64)b * n + b] - A[(i64)a * n + a]) / (2.0 * apq);
-            const double t = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(fma(th, th, 1.0)));
-            c = 1.0 / sqrt(fma(t, t, 1.0));
-            s = t * c;
-          }
+        if (apq != 0.0) {
+          const double th = (S[j * JPITCH + j] - S[i * JPITCH + i]) / (2.0 * apq);
+          const double t = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(fma(th, th, 1.0)));
+          c = 1.0 / sqrt(fma(t, t, 1.0));
+          s = t * c;
         }
-        cs[2 * k] = c;
-        cs[2 * k + 1] = s;
+        cs[2 * tid] = c;
+        cs[2 * tid + 1] = s;
       }
       __syncthreads();
-      // rows: A[a][:], A[b][:] <- c A[a] - s A[b], s A[a] + c A[b]
-      for (i64 it = tid; it < (i64)half * n; it += EIG_THREADS) {
-        const int k = (int)(it / n), j = (int)(it - (it / n) * n);
-        int a, b;
-        pair_of(r, k, a, b);
-        if (a >= n || b >= n) continue;
-        const double c = cs[2 * k], s = cs[2 * k + 1];
-        const double xa = A[(i64)a * n + j], xb = A[(i64)b * n + j];
-        A[(i64)a * n + j] = c * xa - s * xb;
-        A[(i64)b * n + j] = s * xa + c * xb;
-      }
-      __syncthreads();
-      // columns of A and V
-      for (i64 it = tid; it < (i64)half * n; it += EIG_THREADS) {
-        const int k = (int)(it / n), i = (int)(it - (it / n) * n);
-        int a, b;
-        pair_of(r, k, a, b);
-        if (a >= n || b >= n) continue;
-        const double c = cs[2 * k], s = cs[2 * k + 1];
-        const double xa = A[(i64)i * n + a], xb = A[(i64)i * n + b];
-        A[(i64)i * n + a] = c * xa - s * xb;
-        A[(i64)i * n + b] = s * xa + c * xb;
-        const double va = V[(i64)i * n + a], vb = V[(i64)i * n + b];
-        V[(i64)i * n + a] = c * va - s * vb;
-        V[(i64)i * n + b] = s * va + c * vb;
+      {
+        const int ki = tid >> 5, kj = tid & 31;
+        int i0, i1, j0, j1;
+        circle_pair(JP, rr, ki, i0, i1);
+        circle_pair(JP, rr, kj, j0, j1);
+        const double ci = cs[2 * ki], si = cs[2 * ki + 1], cj = cs[2 * kj], sj = cs[2 * kj + 1];
+        const double x00 = S[i0 * JPITCH + j0], x01 = S[i0 * JPITCH + j1], x10 = S[i1 * JPITCH + j0],
+                     x11 = S[i1 * JPITCH + j1];
+        const double y00 = ci * x00 - si * x10, y01 = ci * x01 - si * x11;
+        const double y10 = si * x00 + ci * x10, y11 = si * x01 + ci * x11;
+        S[i0 * JPITCH + j0] = cj * y00 - sj * y01;
+        S[i0 * JPITCH + j1] = sj * y00 + cj * y01;
+        S[i1 * JPITCH + j0] = cj * y10 - sj * y11;
+        S[i1 * JPITCH + j1] = sj * y10 + cj * y11;
+        // columns j0, j1 of the accumulated rotation: rows ki and ki + 32
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          double* w = W + (ki + 32 * h) * JPITCH;
+          const double w0 = w[j0], w1 = w[j1];
+          w[j0] = cj * w0 - sj * w1;
+          w[j1] = sj * w0 + cj * w1;
+        }
       }
       __syncthreads();
     }
   }
-  // descending order: rank of i = #{j : lam_j > lam_i or (lam_j == lam_i and j < i)}
-  for (int i = tid; i < n; i += EIG_THREADS) {
-    const double li = A[(i64)i * n + i];
-    int rk = 0;
-    for (int j = 0; j < n; ++j) {
-      const double lj = A[(i64)j * n + j];
-      rk += (lj > li || (lj == li && j < i)) ? 1 : 0;
-    }
-    if (rk < R) {
-      lam[rk] = li;
-      // sign: largest-magnitude entry positive (first such entry)
-      double best = 0.0;
-      for (int row = 0; row < n; ++row) {
-        const double v = V[(i64)row * n + i];
-        if (fabs(v) > fabs(best)) best = v;
-      }
-      const double sg = best < 0.0 ? -1.0 : 1.0;
-      for (int row = 0; row < n; ++row) U[(i64)row * R + rk] = sg * V[(i64)row * n + i];
+  double* out = m.Q + (i64)blockIdx.x * JP * JP;
+  for (int e = tid; e < JP * JP; e += 1024) out[e] = W[(e / JP) * JPITCH + e % JP];
+}
+
+// A <- J^T A J and V <- V J for the rotations J of round r: workgroup (x, y) owns the
+// 64 x 64 tile of A of row pair and column pair (Q_I^T T Q_J), or of 64 rows of V and
+// a column pair (T Q_J); tiles are disjoint, so in place.  8 waves, each 16 rows x 32
+// columns of the tile, FP64 matrix cores.
+__global__ __launch_bounds__(512) void jacobi_update_kernel(EigArgs a, int r) {
+  __shared__ double sT[JP * JPITCH], sQ[JP * JPITCH];
+  const EigMode& m = a.m[blockIdx.y];
+  const int blocks = m.N / JB, pairs = blocks / 2;
+  if ((int)blockIdx.x >= 2 * pairs * pairs || r >= blocks - 1 || *m.done) return;
+  const bool isV = (int)blockIdx.x >= pairs * pairs;
+  const int t = (int)blockIdx.x - (isV ? pairs * pairs : 0), pi = t / pairs, pj = t % pairs;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q4 = lane >> 4, l16 = lane & 15;
+  int rp, rq, cp, cq;
+  circle_pair(blocks, r, pi, rp, rq);
+  circle_pair(blocks, r, pj, cp, cq);
+  if (isV) {  // 64 consecutive rows
+    rp = 2 * pi;
+    rq = 2 * pi + 1;
+  }
+  const i64 N = m.N;
+  double* M = isV ? m.V : m.A;
+  auto grow = [&](int i) { return (i64)(i < JB ? rp * JB + i : rq * JB + i - JB); };
+  auto gcol = [&](int j) { return (i64)(j < JB ? cp * JB + j : cq * JB + j - JB); };
+  for (int e = tid; e < JP * JP; e += 512) {
+    const int i = e / JP, j = e % JP;
+    sT[i * JPITCH + j] = M[grow(i) * N + gcol(j)];
+    sQ[i * JPITCH + j] = m.Q[(i64)pj * JP * JP + e];
+  }
+  __syncthreads();
+  const int r0 = 16 * (wave >> 1), c0 = 32 * (wave & 1);
+  doublex4 acc[2] = {doublex4{0.0, 0.0, 0.0, 0.0}, doublex4{0.0, 0.0, 0.0, 0.0}};
+#pragma unroll 4
+  for (int kk = 0; kk < JP / 4; ++kk) {
+    const double av = sT[(r0 + l16) * JPITCH + 4 * kk + q4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, sQ[(4 * kk + q4) * JPITCH + c0 + 16 * u + l16], acc[u], 0, 0, 0);
+  }
+  __syncthreads();
+  if (!isV) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sT[(r0 + 4 * e + q4) * JPITCH + c0 + 16 * u + l16] = acc[u][e];
+    for (int e = tid; e < JP * JP; e += 512) sQ[(e / JP) * JPITCH + e % JP] = m.Q[(i64)pi * JP * JP + e];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) acc[u] = doublex4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int kk = 0; kk < JP / 4; ++kk) {
+      const double av = sQ[(4 * kk + q4) * JPITCH + r0 + l16];  // Q_I^T
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        acc[u] =
+            __builtin_amdgcn_mfma_f64_16x16x4f64(av, sT[(4 * kk + q4) * JPITCH + c0 + 16 * u + l16], acc[u], 0, 0, 0);
     }
   }
-  if (tid == 0 && sweeps_out) *sweeps_out = sweep;
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) M[grow(r0 + 4 * e + q4) * N + gcol(c0 + 16 * u + l16)] = acc[u][e];
+}
+
+// Workgroup i: if eigenvalue i of the mode is among its top R (descending, ties by
+// index), its value and eigenvector, turned so that the first entry of largest
+// magnitude is positive.
+__global__ __launch_bounds__(256) void eig_select_kernel(EigArgs a) {
+  __shared__ int cnt[4];
+  __shared__ double bv[4];
+  __shared__ int bi[4];
+  const EigMode& m = a.m[blockIdx.y];
+  const int i = blockIdx.x, n = m.n, tid = threadIdx.x;
+  if (i >= n) return;
+  const i64 N = m.N;
+  const double li = m.A[i * N + i];
+  int rk = 0;
+  double best = 0.0;  // largest magnitude, its row
+  int row = n;
+  for (int j = tid; j < n; j += 256) {
+    const double lj = m.A[j * N + j];
+    rk += (lj > li || (lj == li && j < i)) ? 1 : 0;
+    const double v = m.V[j * N + i];
+    if (fabs(v) > fabs(best)) {
+      best = v;
+      row = j;
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    rk += __shfl_xor(rk, off, 64);
+    const double ov = __shfl_xor(best, off, 64);
+    const int orow = __shfl_xor(row, off, 64);
+    if (fabs(ov) > fabs(best) || (fabs(ov) == fabs(best) && orow < row)) {
+      best = ov;
+      row = orow;
+    }
+  }
+  if ((tid & 63) == 0) {
+    cnt[tid >> 6] = rk;
+    bv[tid >> 6] = best;
+    bi[tid >> 6] = row;
+  }
+  __syncthreads();
+  rk = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+  if (rk >= a.R) return;
+  best = bv[0];
+  row = bi[0];
+  for (int w = 1; w < 4; ++w)
+    if (fabs(bv[w]) > fabs(best) || (fabs(bv[w]) == fabs(best) && bi[w] < row)) {
+      best = bv[w];
+      row = bi[w];
+    }
+  const double sg = best < 0.0 ? -1.0 : 1.0;
+  if (tid == 0) m.lam[rk] = li;
+  for (int j = tid; j < n; j += 256) m.U[(i64)j * a.R + rk] = sg * m.V[j * N + i];
 }
 
 // Nnsvd: for columns j of X_(k) and rank columns r0 .. r0 + 16 of U (n x R):
@@ -377,7 +561,7 @@ __global__ __launch_bounds__(1024) void svd_init_finish_kernel(const double* __r
 }  // namespace
 
 int cp_init_svd(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, i64 R, int kind, uint64_t seed,
-                float* const* F, int* sweeps) {
+                float* const* F) {
   if (kind != TENRSO_INIT_SVD && kind != TENRSO_INIT_NNSVD && kind != TENRSO_INIT_LEVERAGE) {
     set_error("unknown initialisation kind %d", kind);
     return TENRSO_ERR_INVALID_ARGUMENT;
@@ -390,71 +574,114 @@ int cp_init_svd(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, i64 R
     set_error("rank %lld outside the on-device SVD initialisation bound 1..%d", (long long)R, INIT_RMAX);
     return TENRSO_ERR_UNSUPPORTED;
   }
-  i64 total = 1;
-  for (int k = 0; k < nd; ++k) total *= shape[k];
+  for (int k = 0; k < nd; ++k) {
+    if (shape[k] > 1024) {
+      set_error("mode %d of size %lld exceeds the on-device SVD initialisation bound 1024", k, (long long)shape[k]);
+      return TENRSO_ERR_UNSUPPORTED;
+    }
+    if (shape[k] <= 0) {
+      set_error("mode %d is empty", k);
+      return TENRSO_ERR_DEVICE;
+    }
+  }
+  // what depends on a mode: J columns of its unfolding, the splits of its Gram
+  // (about 1024 workgroups, at most 64 MiB of partials), the layout of its buffers
+  struct Mode {
+    i64 P, I, Q, J, nt, splits, nn_blk, oA, oQ, oU, oNN, oR;
+    int ar;
+  } md[MAXD];
+  i64 totA = 0, totQ = 0, totU = 0, totNN = 0, totR = 0, part = 0;
+  EigArgs ea{};
+  ea.R = (int)R;
+  for (int k = 0; k < nd; ++k) {
+    Mode& m = md[k];
+    m.P = m.Q = 1;
+    for (int j = 0; j < k; ++j) m.P *= shape[j];
+    for (int j = k + 1; j < nd; ++j) m.Q *= shape[j];
+    m.I = shape[k];
+    m.J = m.P * m.Q;
+    m.ar = (int)std::min<i64>(R, std::min<i64>(m.I, m.J));
+    m.nt = (m.I + GT - 1) / GT;
+    const i64 ntp = m.nt * (m.nt + 1) / 2;
+    m.splits = std::max<i64>(1, std::min<i64>((1024 + ntp - 1) / ntp, (m.J + 4 * GK - 1) / (4 * GK)));
+    m.splits = std::max<i64>(1, std::min<i64>(m.splits, (64ll << 20) / (m.I * m.I * 8)));
+    part = std::max(part, m.splits * m.I * m.I);
+    const i64 N = (m.I + JP - 1) / JP * JP;
+    ea.m[k].n = (int)m.I;
+    ea.m[k].N = (int)N;
+    m.oA = totA;
+    totA += N * N;
+    m.oQ = totQ;
+    totQ += N / JP * JP * JP;
+    m.oU = totU;
+    totU += m.I * R + R;
+    m.nn_blk = (m.J + 255) / 256;
+    m.oNN = totNN;
+    totNN += kind == TENRSO_INIT_NNSVD ? m.nn_blk * m.ar * 2 : 0;
+    m.oR = totR;
+    totR += m.I * (R - m.ar);
+  }
+  void *pA, *pV, *pPart, *pW;
+  TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_A, (size_t)(totA + totQ) * 8, &pA));
+  TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_V, (size_t)totA * 8 + MAXD * sizeof(int), &pV));
+  TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_PART, (size_t)part * 8, &pPart));
+  TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_W, (size_t)(totU + totNN) * 8 + (size_t)totR * 4 + 16, &pW));
+  float* rnd = (float*)((double*)pW + totU + totNN);
+  int maxN = 0;
+  for (int k = 0; k < nd; ++k) {
+    const Mode& m = md[k];
+    EigMode& e = ea.m[k];
+    e.A = (double*)pA + m.oA;
+    e.Q = (double*)pA + totA + m.oQ;
+    e.V = (double*)pV + m.oA;
+    e.done = (int*)((double*)pV + totA) + k;
+    e.U = (double*)pW + m.oU;
+    e.lam = e.U + m.I * R;
+    maxN = std::max(maxN, e.N);
+    hipLaunchKernelGGL(unfold_gram_partial_kernel, dim3((unsigned)(m.nt * (m.nt + 1) / 2), (unsigned)m.splits),
+                       dim3(256), 0, ctx->stream, X, m.P, m.I, m.Q, (int)m.nt, (int)m.splits, (double*)pPart);
+    TENRSO_HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(unfold_gram_reduce_kernel, dim3((unsigned)((i64)e.N * e.N / 256)), dim3(256), 0, ctx->stream,
+                       (const double*)pPart, (int)m.splits, e);
+    TENRSO_HIP_TRY(hipGetLastError());
+  }
+  // Every sweep is queued without a host round trip; a mode that has converged
+  // (5 to 8 sweeps; quadratically at the end) skips the rest, 2-3 us a launch.
+  const int pairs = maxN / JP, rounds = maxN / JB - 1;
+  for (int sweep = 0; sweep < JACOBI_SWEEPS; ++sweep) {
+    hipLaunchKernelGGL(jacobi_check_kernel, dim3((unsigned)nd), dim3(1024), 0, ctx->stream, ea);
+    for (int r = 0; r < rounds; ++r) {
+      hipLaunchKernelGGL(jacobi_pair_kernel, dim3((unsigned)pairs, (unsigned)nd), dim3(1024), 0, ctx->stream, ea, r);
+      hipLaunchKernelGGL(jacobi_update_kernel, dim3((unsigned)(2 * pairs * pairs), (unsigned)nd), dim3(512), 0,
+                         ctx->stream, ea, r);
+    }
+    TENRSO_HIP_TRY(hipGetLastError());
+  }
+  hipLaunchKernelGGL(eig_select_kernel, dim3((unsigned)maxN, (unsigned)nd), dim3(256), 0, ctx->stream, ea);
+  TENRSO_HIP_TRY(hipGetLastError());
   std::mt19937_64 rng(seed);
   std::normal_distribution<double> noise(0.0, 0.01);  // helpers.rs: Normal::new(0.0, 0.01)
   for (int k = 0; k < nd; ++k) {
-    const i64 I = shape[k];
-    if (I > 1024) {
-      set_error("mode %d of size %lld exceeds the on-device SVD initialisation bound 1024", k, (long long)I);
-      return TENRSO_ERR_UNSUPPORTED;
-    }
-    i64 P = 1, Q = 1;
-    for (int m = 0; m < k; ++m) P *= shape[m];
-    for (int m = k + 1; m < nd; ++m) Q *= shape[m];
-    const i64 J = P * Q;
-    const int ar = (int)std::min<i64>(R, std::min<i64>(I, J));
-    const int nt = (int)((I + GT - 1) / GT);
-    const int ntp = nt * (nt + 1) / 2;
-    int splits = (int)std::max<i64>(1, std::min<i64>(64, 512 / ntp));
-    splits = (int)std::max<i64>(1, std::min<i64>(splits, (64ll << 20) / (I * I * 8)));
-    void *pK, *pV, *pPart, *pW;
-    TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_A, (size_t)I * I * 8, &pK));
-    TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_V, (size_t)I * I * 8, &pV));
-    TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_PART, (size_t)splits * I * I * 8, &pPart));
-    // U (I x R doubles), lam (R), the Nnsvd partials, the draws (I x (R - ar) floats), sweeps
-    const i64 nn_blk = (J + 255) / 256;
-    const size_t u_bytes = (size_t)I * R * 8, lam_bytes = (size_t)R * 8;
-    const size_t nn_bytes = kind == TENRSO_INIT_NNSVD ? (size_t)nn_blk * ar * 2 * 8 : 0;
-    const size_t rnd_bytes = (size_t)I * (R - ar) * 4 + 16;
-    TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_W, u_bytes + lam_bytes + nn_bytes + rnd_bytes + 16, &pW));
-    double* K = (double*)pK;
-    double* U = (double*)pW;
-    double* lam = U + (size_t)I * R;
-    double* nn = lam + R;
-    float* rnd = (float*)((char*)nn + nn_bytes);
-    hipLaunchKernelGGL(unfold_gram_partial_kernel, dim3((unsigned)ntp, (unsigned)splits), dim3(256), 0, ctx->stream, X,
-                       P, I, Q, nt, splits, (double*)pPart);
-    TENRSO_HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(unfold_gram_reduce_kernel, dim3((unsigned)((I * I + 255) / 256)), dim3(256), 0, ctx->stream,
-                       (const double*)pPart, splits, I, K);
-    TENRSO_HIP_TRY(hipGetLastError());
-    int* dsweeps = (int*)ctx->pinned_dev + 64;  // scratch int in mapped host memory
-    hipLaunchKernelGGL(jacobi_eig_kernel, dim3(1), dim3(EIG_THREADS), 0, ctx->stream, K, (double*)pV, (int)I,
-                       (int)R, 60, U, lam, dsweeps);
-    TENRSO_HIP_TRY(hipGetLastError());
-    if (kind == TENRSO_INIT_NNSVD && ar > 0) {
-      hipLaunchKernelGGL(nnsvd_norms_kernel, dim3((unsigned)nn_blk, (unsigned)((ar + NN_RC - 1) / NN_RC)), dim3(256),
-                         0, ctx->stream, X, P, I, Q, (const double*)U, (int)R, ar, nn);
+    const Mode& m = md[k];
+    const EigMode& e = ea.m[k];
+    double* nn = (double*)pW + totU + m.oNN;
+    float* draws = rnd + m.oR;
+    if (kind == TENRSO_INIT_NNSVD && m.ar > 0) {
+      hipLaunchKernelGGL(nnsvd_norms_kernel, dim3((unsigned)m.nn_blk, (unsigned)((m.ar + NN_RC - 1) / NN_RC)), dim3(256),
+                         0, ctx->stream, X, m.P, m.I, m.Q, (const double*)e.U, (int)R, m.ar, nn);
       TENRSO_HIP_TRY(hipGetLastError());
     }
-    if (ar < R) {
-      std::vector<float> h((size_t)I * (R - ar));
+    if (m.ar < R) {
+      std::vector<float> h((size_t)m.I * (R - m.ar));
       for (auto& v : h) v = (float)noise(rng);
-      TENRSO_HIP_TRY(hipMemcpyAsync(rnd, h.data(), h.size() * 4, hipMemcpyHostToDevice, ctx->stream));
+      TENRSO_HIP_TRY(hipMemcpyAsync(draws, h.data(), h.size() * 4, hipMemcpyHostToDevice, ctx->stream));
       TENRSO_HIP_TRY(hipStreamSynchronize(ctx->stream));  // h leaves scope
     }
-    hipLaunchKernelGGL(svd_init_finish_kernel, dim3(1), dim3(1024), 0, ctx->stream, (const double*)U,
-                       (const double*)lam, (int)I, (int)R, ar, kind, (const double*)nn, (int)nn_blk,
-                       (const float*)rnd, F[k]);
+    hipLaunchKernelGGL(svd_init_finish_kernel, dim3(1), dim3(1024), 0, ctx->stream, (const double*)e.U,
+                       (const double*)e.lam, (int)m.I, (int)R, m.ar, kind, (const double*)nn, (int)m.nn_blk,
+                       (const float*)draws, F[k]);
     TENRSO_HIP_TRY(hipGetLastError());
-    if (sweeps) {
-      TENRSO_HIP_TRY(hipStreamSynchronize(ctx->stream));
-      sweeps[k] = ((volatile int*)ctx->pinned)[64];
-    }
   }
-  (void)total;
   return TENRSO_OK;
 }
 
