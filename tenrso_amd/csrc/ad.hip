@@ -162,6 +162,7 @@ __global__ __launch_bounds__(GR_T) void grad_rows_kernel(const float* __restrict
   }
 }
 
+// xpart (or null): npx partial sums of ||X||^2, added here instead of scal's value
 // loss = 0.5 (||X||^2 - 2 sum(part) + sum_rs prod_k G_k[r,s]) into out[0] and, when
 // hist is not null, into *hist (the device-side loss history of a descent)
 __device__ void gamma_norm_block(const double* __restrict__ G, int nd, int R, int n, double* __restrict__ out);
@@ -170,8 +171,9 @@ __device__ void gamma_norm_block(const double* __restrict__ G, int nd, int R, in
 // mode n = blockIdx.x - 1 into gnorm[n] (the step size of a descent step).
 __global__ __launch_bounds__(256) void loss_kernel(const double* __restrict__ G, int nd, int R,
                                                    const double* __restrict__ part, int npart,
-                                                   const double* __restrict__ scal, double* __restrict__ out,
-                                                   double* __restrict__ hist, double* __restrict__ gnorm) {
+                                                   const double* __restrict__ scal, const double* __restrict__ xpart,
+                                                   int npx, double* __restrict__ out, double* __restrict__ hist,
+                                                   double* __restrict__ gnorm) {
   if (blockIdx.x > 0) {
     gamma_norm_block(G, nd, R, (int)blockIdx.x - 1, gnorm);
     return;
@@ -191,6 +193,28 @@ __global__ __launch_bounds__(256) void loss_kernel(const double* __restrict__ G,
   }
   const double recon = red[0];
   __syncthreads();
+  double nx = 0.0;
+  if (xpart) {
+    double x0 = 0.0, x1 = 0.0, x2 = 0.0, x3 = 0.0;
+    int b = threadIdx.x;
+    for (; b + 768 < npx; b += 1024) {
+      x0 += xpart[b];
+      x1 += xpart[b + 256];
+      x2 += xpart[b + 512];
+      x3 += xpart[b + 768];
+    }
+    for (; b < npx; b += 256) x0 += xpart[b];
+    red[threadIdx.x] = (x0 + x1) + (x2 + x3);
+    __syncthreads();
+    for (int k = 128; k > 0; k >>= 1) {
+      if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
+      __syncthreads();
+    }
+    nx = red[0];
+    __syncthreads();
+  } else {
+    nx = scal[SC_NORM_X];
+  }
   double ip = 0.0;
   for (int b = threadIdx.x; b < npart; b += 256) ip += part[b];
   red[threadIdx.x] = ip;
@@ -200,7 +224,7 @@ __global__ __launch_bounds__(256) void loss_kernel(const double* __restrict__ G,
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    const double loss = 0.5 * (scal[SC_NORM_X] - 2.0 * red[0] + recon);
+    const double loss = 0.5 * (nx - 2.0 * red[0] + recon);
     out[0] = loss;
     out[1] = red[0];
     out[2] = recon;
@@ -319,13 +343,28 @@ int loss_work(tenrso_ctx* ctx, int nd, const i64* shape, i64 R, LossWork* w) {
 }  // namespace
 
 // grads[n] = A_n Gamma_n - mttkrp(X, A, n); loss into w.out[0] (device, and into
-// *hist when not null), with ||X||^2 already in w.scal[SC_NORM_X].  Per mode: the
-// MTTKRP as split partials, then one fused row kernel; modes without a gradient
-// to form are skipped except the last, whose MTTKRP gives <X, Xhat>.  With `tree`
-// (four modes) two partial MTTKRPs serve all four modes instead.
+// *hist when not null), with ||X||^2 already in w.scal[SC_NORM_X], or (with_norm)
+// formed here: by the last mode's MTTKRP (a tree's first pass) as it reads X,
+// else by a pass of its own.  Per mode: the MTTKRP as split partials, then one
+// fused row kernel; modes without a gradient to form are skipped except the
+// last, whose MTTKRP gives <X, Xhat>.  With `tree` (four modes) two partial
+// MTTKRPs serve all four modes instead.
 static int loss_grad_device(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, const float* const* F, i64 R,
                             float* const* grads, LossWork& w, double* hist, const float* Xt = nullptr,
-                            double* gnorm = nullptr, bool tree = false) {
+                            double* gnorm = nullptr, bool tree = false, bool with_norm = false) {
+  const double* xpart = nullptr;
+  int npx = 0;
+  // the norm of a launch that left none: one pass over X
+  auto take_norm = [&](const MttkrpResult* mr) -> int {
+    if (mr && mr->norm) {
+      xpart = mr->norm;
+      npx = mr->nnorm;
+      return TENRSO_OK;
+    }
+    i64 total = 1;
+    for (int k = 0; k < nd; ++k) total *= shape[k];
+    return tensor_norm_min(ctx, X, total, w.part, w.scal);
+  };
   TENRSO_TRY(gram_f64_many(ctx, nd, F, shape, R, w.G));
   if (tree) {
     // 4-way dimension tree: two passes over X instead of four.
@@ -341,7 +380,9 @@ static int loss_grad_device(tenrso_ctx* ctx, const float* X, int nd, const i64* 
       const float* Fv[3] = {half == 0 ? F[0] : F[0], half == 0 ? F[2] : F[1], half == 0 ? F[3] : F[2]};
       MttkrpResult mr;
       TENRSO_TRY(mttkrp_dense(ctx, TENRSO_PREC_FP32, X, nullptr, 3, v, Fv, R, half == 0 ? 0 : 2,
-                              MttkrpOut::PARTIAL, nullptr, &mr));
+                              MttkrpOut::PARTIAL, nullptr, &mr, nullptr, false, nullptr, 0, 0, nullptr,
+                              with_norm && half == 0));
+      if (with_norm && half == 0) TENRSO_TRY(take_norm(&mr));
       const i64 ya = half == 0 ? I0 : I2, yb = half == 0 ? I1 : I3;  // Y rows = ya x yb
       // both modes of the pass in one launch (the first: M[i] sums over the
       // second index of Y; the second: over the first)
@@ -363,7 +404,7 @@ static int loss_grad_device(tenrso_ctx* ctx, const float* X, int nd, const i64* 
       }
     }
     hipLaunchKernelGGL(loss_kernel, dim3(gnorm ? 1 + nd : 1), dim3(256), 0, ctx->stream, w.G, nd, (int)R, w.part,
-                       (int)shape[nd - 1], w.scal, w.out, hist, gnorm);
+                       (int)shape[nd - 1], w.scal, xpart, npx, w.out, hist, gnorm);
     TENRSO_HIP_TRY(hipGetLastError());
     return TENRSO_OK;
   }
@@ -380,7 +421,10 @@ static int loss_grad_device(tenrso_ctx* ctx, const float* X, int nd, const i64* 
     if (!gn && !last) continue;
     MttkrpResult mr;
     TENRSO_TRY(mttkrp_dense(ctx, TENRSO_PREC_FP32, X, Xt, nd, shape, F, R, n, MttkrpOut::PARTIAL, nullptr, &mr,
-                            nullptr, false, nullptr, 0, 0, pre[n]));
+                            nullptr, false, nullptr, 0, 0, pre[n], with_norm && last));
+    // with the last mode, which always runs: every mode takes the same kernel
+    // whichever gradients are asked for
+    if (with_norm && last) TENRSO_TRY(take_norm(&mr));
     if (shape[n] == 0) continue;
     hipLaunchKernelGGL(grad_rows_kernel<false>, dim3((unsigned)shape[n]), dim3(GR_T), 0, ctx->stream, mr.partial,
                        mr.splits, (int)R, w.G, nd, GradRows{n, shape[n], F[n], gn, last ? w.part : nullptr, {}},
@@ -388,7 +432,7 @@ static int loss_grad_device(tenrso_ctx* ctx, const float* X, int nd, const i64* 
     TENRSO_HIP_TRY(hipGetLastError());
   }
   hipLaunchKernelGGL(loss_kernel, dim3(gnorm ? 1 + nd : 1), dim3(256), 0, ctx->stream, w.G, nd, (int)R, w.part,
-                     (int)shape[nd - 1], w.scal, w.out, hist, gnorm);
+                     (int)shape[nd - 1], w.scal, xpart, npx, w.out, hist, gnorm);
   TENRSO_HIP_TRY(hipGetLastError());
   return TENRSO_OK;
 }
@@ -403,9 +447,8 @@ int cp_loss_grad_dev(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, 
   TENRSO_TRY(loss_work(ctx, nd, shape, R, &w));
   i64 total = 1;
   for (int k = 0; k < nd; ++k) total *= shape[k];
-  TENRSO_TRY(fill_f64(ctx, w.scal, 64, 0.0));
-  TENRSO_TRY(tensor_norm_min(ctx, X, total, w.part, w.scal));
-  TENRSO_TRY(loss_grad_device(ctx, X, nd, shape, F, R, grads, w, nullptr, nullptr, nullptr, nd == 4 && total > 0));
+  TENRSO_TRY(loss_grad_device(ctx, X, nd, shape, F, R, grads, w, nullptr, nullptr, nullptr, nd == 4 && total > 0,
+                              true));
   if (loss_dev) *loss_dev = w.out;
   return TENRSO_OK;
 }

@@ -104,6 +104,7 @@ enum BufSlot : int {
   SLOT_GATE,
   SLOT_GRAM_CHUNKS,
   SLOT_XPAD,
+  SLOT_NORM,
   SLOT_COUNT
 };
 

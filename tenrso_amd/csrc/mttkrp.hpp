@@ -18,6 +18,8 @@ enum class MttkrpOut {
 struct MttkrpResult {
   const float* partial = nullptr;  // [splits, I, R]
   int splits = 0;
+  const double* norm = nullptr;    // with want_norm: partial sums of ||X||^2, or null
+  int nnorm = 0;                   //   where the kernel of this shape leaves none
 };
 
 // Caller-provided device workspace for the PRE Khatri-Rao rows and the split
@@ -37,12 +39,14 @@ struct MttkrpScratch {
 // MTTKRP launch (or, where it cannot, as its own kernel just before it).
 // x_pad / xt_pad (BF16 only, 0 = none): the memory extent of the last mode of X
 // and of X_t when those copies have it padded with zeros.
+// want_norm: also leave FP64 partial sums of ||X||^2 in res->norm (FP32 calls whose
+// ranks fit one launch of the MFMA kernel; null otherwise).
 // pre_rows (optional, tensors of order >= 4): the PRE Khatri-Rao rows of this
 // mode already formed (mttkrp_pre_batch), instead of a launch that forms them.
 int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int nd, const i64* shape,
                  const float* const* F, i64 R, int mode, MttkrpOut outk, void* out, MttkrpResult* res,
                  const AlsJob* job = nullptr, bool xt_f32 = false, const MttkrpScratch* scratch = nullptr,
-                 i64 x_pad = 0, i64 xt_pad = 0, const float* pre_rows = nullptr);
+                 i64 x_pad = 0, i64 xt_pad = 0, const float* pre_rows = nullptr, bool want_norm = false);
 
 // The PRE Khatri-Rao rows of the MTTKRPs of several modes of one tensor (order
 // >= 4) in one launch: pre[i] receives the rows the MFMA MTTKRP of modes[i]

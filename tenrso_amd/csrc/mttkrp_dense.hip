@@ -722,7 +722,7 @@ Plan make_plan(int nd, const i64* shape, int mode) {
 int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int nd, const i64* shape,
                  const float* const* F, i64 R, int mode, MttkrpOut outk, void* out, MttkrpResult* res,
                  const AlsJob* job, bool xt_f32, const MttkrpScratch* scratch, i64 x_pad, i64 xt_pad,
-                 const float* pre_rows) {
+                 const float* pre_rows, bool want_norm) {
   Plan pl = make_plan(nd, shape, mode);
   const bool bf16 = prec == TENRSO_PREC_BF16;
   const float* Fv[MAXD];
@@ -872,6 +872,8 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
 
   float* partial = nullptr;
   int splits = 1;
+  const double* norm = nullptr;
+  int nnorm = 0;
   if (mfma_ok) {
     constexpr i64 rows_per_wg = 32;
     const i64 rtiles = (i64)cdiv(I, rows_per_wg);
@@ -932,8 +934,9 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
     // Several rounds and no job: 4-wave workgroups, as many splits as bring 1.5
     // times the resident ones while a wave keeps four blocks (9216 rows, 9216 j,
     // rank 32: 75 us with 576 workgroups, 70 with 1152, 69 with 1728).
-    if (fp32 && NT < 8 && !fuse_job && wgs1 * ssp > target) {
-      kern = mttkrp_x3_kernel_w4(NT, caseB, a.win_vec, XL);
+    const bool with_norm = want_norm && fp32 && !bf16 && pad == 0 && !job && rchunks == 1 && NT < 8;
+    if (fp32 && NT < 8 && !fuse_job && (wgs1 * ssp > target || with_norm)) {
+      kern = with_norm ? mttkrp_x3_kernel_norm(NT, caseB, a.win_vec, XL) : mttkrp_x3_kernel_w4(NT, caseB, a.win_vec, XL);
       waves = 4;
       TENRSO_TRY(occupancy(kern, waves * 64, &occ));
       target = (i64)(ctx->wg_per_cu_f32 > 0 ? ctx->wg_per_cu_f32 : occ) * ctx->num_cus;
@@ -949,6 +952,13 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
     a.slow_rem = a.n_slow % a.slow_splits;
     splits = a.nwin * a.slow_splits;
     TENRSO_TRY(partial_buffer(splits, &partial));
+    if (with_norm) {
+      void* np = nullptr;
+      nnorm = (int)(rtiles * splits * waves);
+      TENRSO_TRY(ctx_buffer(ctx, SLOT_NORM, (size_t)nnorm * sizeof(double), &np));
+      a.norm = (double*)np;
+      norm = a.norm;
+    }
     if (job && !fuse_job) TENRSO_TRY(als_job_launch(ctx, *job));
     const dim3 block(waves * 64);
     // BF16 with the job fused: the MTTKRP workgroups wait for the job's Gram loads
@@ -1029,6 +1039,8 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
   if (res) {
     res->partial = partial;
     res->splits = splits;
+    res->norm = norm;
+    res->nnorm = nnorm;
   }
   if (outk == MttkrpOut::F32) return reduce_partials(ctx, partial, splits, nout, (float*)out, nullptr);
   if (outk == MttkrpOut::F64) return reduce_partials(ctx, partial, splits, nout, nullptr, (double*)out);

@@ -10,6 +10,8 @@ namespace tenrso {
 // 8 waves, able to run the ALS job as workgroup 0, or 4 waves without it.
 const void* mttkrp_x3_kernel_w8(int nt, bool case_b, bool wv, int xl);
 const void* mttkrp_x3_kernel_w4(int nt, bool case_b, bool wv, int xl);
+// The 4-wave instances that also leave the sum of squares of X (KernArgs::norm).
+const void* mttkrp_x3_kernel_norm(int nt, bool case_b, bool wv, int xl);
 // Eight rank tiles, 8 waves, able to run the wide-rank job.
 const void* mttkrp_x3_kernel_n8(bool case_b, bool wv, int xl);
 

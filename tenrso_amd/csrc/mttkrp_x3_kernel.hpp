@@ -112,7 +112,10 @@ __device__ __forceinline__ void x3_plain_tile(const float* X, const KernArgs& a,
 // a CU runs several one after another the end of one meets the loop of the next
 // (9216 rows x 9216 j at rank 32: 69-73 us against 77-85 us; one full round at
 // 256^3 rank 64: 19.1 us against 18.4 us).
-template <int NT, int WAVES, int JOB, bool CASE_B, bool WV, int XL>
+// NORM: the sum of squares of X as well (FP64; every element of X is read by exactly
+// one lane), a partial per wave in a.norm.  In the memory-bound loop it is nearly
+// free, where a pass of its own over X takes as long as the MTTKRP.
+template <int NT, int WAVES, int JOB, bool CASE_B, bool WV, int XL, bool NORM>
 __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __restrict__ X, KernArgs a,
                                                                 float* __restrict__ partial, AlsJob job,
                                                                 int has_job) {
@@ -172,6 +175,9 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
       acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
       Tacc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
+  double sumsq[MT];  // sum of squares of the lane's rows (NORM)
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) sumsq[mt] = 0.0;
   float rmax[MT];  // largest |x| of the lane's row(s) in this wave's blocks
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) rmax[mt] = 0.f;
@@ -288,6 +294,10 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
       }
 #pragma unroll
       for (int e = 0; e < 8; e += 2) x3_max3(rmax[mt], x[e], x[e + 1]);
+      if constexpr (NORM) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sumsq[mt] = fma((double)x[e], (double)x[e], sumsq[mt]);
+      }
       x3_split(x, xh[mt], xl[mt], xl2[mt]);
     }
     // Two rank tiles at a time, term by term (smallest first): consecutive MFMAs
@@ -350,6 +360,19 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
     }
   }
 
+  if constexpr (NORM) {
+    // rows past I repeat the last one (case B: the last pair)
+    double v = 0.0;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const i64 row = CASE_B ? row_base + MT * c + mt : row_base + 16 * mt + c;
+      v += row < a.I ? sumsq[mt] : 0.0;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if (lane == 0) a.norm[(i64)blockIdx.x * WAVES + wave] = v;
+  }
+
   // not finite, or small enough for the low parts (2^-16 of the products) to leave
   // the exponent range: all of it again in fp32
   float z = 0.f;
@@ -385,19 +408,20 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
   wg_reduce_store<MT, NT, WAVES, false>(acc, smem, wave, lane, out, a.I, a.R, a.r0, a.rcount, row_base, CASE_B);
 }
 
-template <int NT, int WAVES, int JOB, bool CASE_B, bool WV>
+template <int NT, int WAVES, int JOB, bool CASE_B, bool WV, bool NORM>
 const void* x3_pick_xl(int xl) {
   if constexpr (!CASE_B) {
-    if (xl == 4) return reinterpret_cast<const void*>(mttkrp_x3_mfma<NT, WAVES, JOB, CASE_B, WV, 4>);
+    if (xl == 4) return reinterpret_cast<const void*>(mttkrp_x3_mfma<NT, WAVES, JOB, CASE_B, WV, 4, NORM>);
   }
-  if (xl == 0) return reinterpret_cast<const void*>(mttkrp_x3_mfma<NT, WAVES, JOB, CASE_B, WV, 0>);
-  return reinterpret_cast<const void*>(mttkrp_x3_mfma<NT, WAVES, JOB, CASE_B, WV, 1>);
+  if (xl == 0) return reinterpret_cast<const void*>(mttkrp_x3_mfma<NT, WAVES, JOB, CASE_B, WV, 0, NORM>);
+  return reinterpret_cast<const void*>(mttkrp_x3_mfma<NT, WAVES, JOB, CASE_B, WV, 1, NORM>);
 }
 
-template <int NT, int WAVES, int JOB>
+template <int NT, int WAVES, int JOB, bool NORM = false>
 const void* x3_pick(bool case_b, bool wv, int xl) {
-  if (case_b) return wv ? x3_pick_xl<NT, WAVES, JOB, true, true>(xl) : x3_pick_xl<NT, WAVES, JOB, true, false>(xl);
-  return wv ? x3_pick_xl<NT, WAVES, JOB, false, true>(xl) : x3_pick_xl<NT, WAVES, JOB, false, false>(xl);
+  if (case_b)
+    return wv ? x3_pick_xl<NT, WAVES, JOB, true, true, NORM>(xl) : x3_pick_xl<NT, WAVES, JOB, true, false, NORM>(xl);
+  return wv ? x3_pick_xl<NT, WAVES, JOB, false, true, NORM>(xl) : x3_pick_xl<NT, WAVES, JOB, false, false, NORM>(xl);
 }
 
 }  // namespace
