@@ -380,7 +380,7 @@ static int loss_grad_device(tenrso_ctx* ctx, const float* X, int nd, const i64* 
       const float* Fv[3] = {half == 0 ? F[0] : F[0], half == 0 ? F[2] : F[1], half == 0 ? F[3] : F[2]};
       MttkrpResult mr;
       TENRSO_TRY(mttkrp_dense(ctx, TENRSO_PREC_FP32, X, nullptr, 3, v, Fv, R, half == 0 ? 0 : 2,
-                              MttkrpOut::PARTIAL, nullptr, &mr, nullptr, false, nullptr, 0, 0, nullptr,
+                              MttkrpOut::PARTIAL, nullptr, &mr, nullptr, nullptr, 0, 0, nullptr,
                               with_norm && half == 0));
       if (with_norm && half == 0) TENRSO_TRY(take_norm(&mr));
       const i64 ya = half == 0 ? I0 : I2, yb = half == 0 ? I1 : I3;  // Y rows = ya x yb
@@ -421,7 +421,7 @@ static int loss_grad_device(tenrso_ctx* ctx, const float* X, int nd, const i64* 
     if (!gn && !last) continue;
     MttkrpResult mr;
     TENRSO_TRY(mttkrp_dense(ctx, TENRSO_PREC_FP32, X, Xt, nd, shape, F, R, n, MttkrpOut::PARTIAL, nullptr, &mr,
-                            nullptr, false, nullptr, 0, 0, pre[n], with_norm && last));
+                            nullptr, nullptr, 0, 0, pre[n], with_norm && last));
     // with the last mode, which always runs: every mode takes the same kernel
     // whichever gradients are asked for
     if (with_norm && last) TENRSO_TRY(take_norm(&mr));

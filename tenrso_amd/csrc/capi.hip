@@ -170,17 +170,8 @@ int tenrso_mttkrp_bf16(tenrso_ctx* ctx, const uint16_t* X_bf16, int ndim, const 
   TENRSO_TRY(check_mttkrp_basic(ndim, shape, rank, mode));
   if (rank == 0 || shape[mode] == 0) return TENRSO_OK;
   TENRSO_TRY(set_device(ctx));
-  const void* Xt = nullptr;
-  if (mode == ndim - 1) {
-    // last mode: move it to the front once (bf16 -> bf16 transpose)
-    const i64 total = prod(shape, ndim);
-    void* pt = nullptr;
-    TENRSO_TRY(ctx_buffer(ctx, SLOT_XBF16_T, (size_t)total * 2 + 16, &pt));
-    TENRSO_TRY(transpose_last_to_front_u16(ctx, X_bf16, ndim, shape, (uint16_t*)pt));
-    Xt = pt;
-  }
   TENRSO_TRY(timed_begin(ctx));
-  TENRSO_TRY(mttkrp_dense(ctx, TENRSO_PREC_BF16, X_bf16, Xt, ndim, shape, factors, rank, mode, MttkrpOut::F32, out,
+  TENRSO_TRY(mttkrp_dense(ctx, TENRSO_PREC_BF16, X_bf16, nullptr, ndim, shape, factors, rank, mode, MttkrpOut::F32, out,
                           nullptr));
   return timed_end(ctx);
 }
@@ -207,17 +198,15 @@ int tenrso_mttkrp_profile(tenrso_ctx* ctx, int precision, const void* X, int ndi
   }
   const bool bf16 = precision == TENRSO_PREC_BF16 || x3;
   const void* Xt = nullptr;
-  if (bf16 && mode == ndim - 1) {
-    const i64 total = prod(shape, ndim);
+  if (x3) {
     void* pt = nullptr;
-    TENRSO_TRY(ctx_buffer(ctx, SLOT_XBF16_T, (size_t)total * (x3 ? 4 : 2) + 16, &pt));
-    if (x3) TENRSO_TRY(transpose_last_to_front_f32(ctx, (const float*)X, ndim, shape, (float*)pt));
-    else TENRSO_TRY(transpose_last_to_front_u16(ctx, (const uint16_t*)X, ndim, shape, (uint16_t*)pt));
+    TENRSO_TRY(ctx_buffer(ctx, SLOT_XBF16_T, (size_t)prod(shape, ndim) * 4 + 16, &pt));
+    TENRSO_TRY(transpose_last_to_front_f32(ctx, (const float*)X, ndim, shape, (float*)pt));
     Xt = pt;
   }
   ctx->profile_reps = reps;
   int rc = mttkrp_dense(ctx, bf16 ? TENRSO_PREC_BF16 : TENRSO_PREC_FP32, X, Xt, ndim, shape, factors, rank, mode,
-                        MttkrpOut::PARTIAL, nullptr, nullptr, nullptr, x3);
+                        MttkrpOut::PARTIAL, nullptr, nullptr);
   ctx->profile_reps = 0;
   if (rc != TENRSO_OK) return rc;
   *ms = ctx->last_kernel_ms;

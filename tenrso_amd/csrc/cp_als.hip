@@ -395,7 +395,7 @@ int cp_als_device(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, flo
   const i64 x_pad = padded ? Kxp : (fpad ? Kx32 : 0), xt_pad = padded ? Btp : (fpad ? Bt32 : 0);
   pb.mttkrp = [&](int mode, const float* const* Fc, const AlsJob* job, MttkrpResult* mr) {
     return mttkrp_dense(ctx, bf16 ? TENRSO_PREC_BF16 : TENRSO_PREC_FP32, Xk, Xt, nd, shape, Fc, R, mode,
-                        MttkrpOut::PARTIAL, nullptr, mr, job, /*xt_f32=*/true, nullptr, x_pad, xt_pad);
+                        MttkrpOut::PARTIAL, nullptr, mr, job, nullptr, x_pad, xt_pad);
   };
   return cp_als_run(ctx, pb, F, o, res, hist);
 }

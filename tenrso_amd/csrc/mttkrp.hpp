@@ -31,10 +31,9 @@ struct MttkrpScratch {
   size_t bytes = 0;
 };
 
-// X: fp32 tensor (prec FP32) or bf16 tensor (prec BF16, uint16 storage).  For BF16
-// and mode == ndim-1 the caller passes X_t, the tensor with the last mode moved
-// to the front: bf16 (xt_f32 false), or the exact fp32 tensor (xt_f32 true), which
-// the MFMA kernel contracts with a three-way bf16 split at FP32 accuracy.
+// X: fp32 tensor (prec FP32) or bf16 tensor (prec BF16, uint16 storage).
+// X_t (optional): the fp32 tensor with the last mode moved to the front, which the
+// last mode's MTTKRP contracts instead of X, at FP32 accuracy also in a BF16 call.
 // job (optional): the ALS linear algebra of this mode; it runs as workgroup 0 of the
 // MTTKRP launch (or, where it cannot, as its own kernel just before it).
 // x_pad / xt_pad (BF16 only, 0 = none): the memory extent of the last mode of X
@@ -45,7 +44,7 @@ struct MttkrpScratch {
 // mode already formed (mttkrp_pre_batch), instead of a launch that forms them.
 int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int nd, const i64* shape,
                  const float* const* F, i64 R, int mode, MttkrpOut outk, void* out, MttkrpResult* res,
-                 const AlsJob* job = nullptr, bool xt_f32 = false, const MttkrpScratch* scratch = nullptr,
+                 const AlsJob* job = nullptr, const MttkrpScratch* scratch = nullptr,
                  i64 x_pad = 0, i64 xt_pad = 0, const float* pre_rows = nullptr, bool want_norm = false);
 
 // The PRE Khatri-Rao rows of the MTTKRPs of several modes of one tensor (order
@@ -83,8 +82,7 @@ int convert_bf16(tenrso_ctx* ctx, const float* src, int nd, const i64* shape, bo
 int prepare_bf16_als(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, uint16_t* dst, float* dstT,
                      double* tmp, int* nblk_out);
 
-// [.., I_{N-1}] -> [I_{N-1}, ..] (last mode moved to the front), plain copies.
-int transpose_last_to_front_u16(tenrso_ctx* ctx, const uint16_t* src, int nd, const i64* shape, uint16_t* dst);
+// [.., I_{N-1}] -> [I_{N-1}, ..] (last mode moved to the front), a plain copy.
 int transpose_last_to_front_f32(tenrso_ctx* ctx, const float* src, int nd, const i64* shape, float* dst);
 // Padded layouts for the BF16 ALS of tensors with ragged last modes: the bf16
 // copy with its last mode padded to Kp, and the fp32 last-to-front copy with

@@ -21,8 +21,8 @@
 //     dimension, in v_mfma_f32_16x16x32_bf16: an fp32 tensor as exact triples of
 //     bf16 (mttkrp_x3_kernel.hpp), a bf16 tensor as it is (here).  For q-contiguous X
 //     (mode < N-1, "case A") each lane loads 8 consecutive j straight from HBM; for
-//     the last mode (Q == 1, "case B", fp32 only) lanes run along i, which is
-//     contiguous, and each lane loads its 8 j of two rows.
+//     the last mode (Q == 1, "case B") lanes run along i, which is contiguous, and
+//     each lane loads its 8 j of two rows (bf16: four).
 //   * Workgroups split j; each writes an [I_tile x R] fp32 partial, summed in a
 //     fixed order (FP64) by reduce_partials or by the ALS solve kernel.  No float
 //     atomics: results are run-to-run deterministic.
@@ -34,43 +34,63 @@
 namespace tenrso {
 
 // ---------------------------------------------------------------------------
-// BF16 MFMA kernel (v_mfma_f32_16x16x32_bf16), case A only (q-contiguous X; the
-// last mode runs on the last-to-front copy).  The work split and the T-then-PRE
-// contraction of the fp32 kernel (mttkrp_x3_kernel.hpp), FP32 accumulation.  X enters as
-// bf16 (one 16-byte load of 8 consecutive j per lane and k-step); the FAST window
-// enters as an exact bf16 hi + lo pair (two MFMAs per step), so the input tensor
-// is the only operand rounded to bf16.
+// BF16 MFMA kernel (v_mfma_f32_16x16x32_bf16).  The work split and the T-then-PRE
+// contraction of the fp32 kernel (mttkrp_x3_kernel.hpp), FP32 accumulation.  X
+// enters as it is.
+//   XL 0, 1, 4 (16-byte aligned rows; case A): whole windows, masked windows, a
+// zero-padded copy.  One 16-byte load of 8 consecutive j per lane, row and k-step; the
+// FAST window enters as a bf16 hi + lo pair (two MFMAs per step).
+//   XL 3 (any size and alignment; both cases) and case B (the last mode; XL 0 for I a
+// multiple of 4 and an 8-byte aligned X): the FAST window as the exact triple of each
+// fp32 value, so the products are those of fp32 arithmetic, as they are in the
+// one-thread-an-output kernel that served such calls (2000 us at 19x69x32x75 rank 21;
+// 70 us here).  Vectors are loaded unaligned, elements past the window's end (the next
+// row's) are masked, except where the load would pass the end of X.  As in the fp32
+// kernel a tile that is not finite, or whose values are too small for their low parts,
+// is formed again in plain fp32.
+//   Case B: 64 rows a workgroup, lanes along i; each lane loads four rows (8 bytes) of
+// its 8 j, a full 128-byte line per j and 16 lanes, and byte permutes turn the 8 x 4
+// block into four A operands.  (A copy of X with the last mode in front took 43 us of
+// the 64 of a 512x256x256 rank 64 last mode; this form takes 19.)
 // ---------------------------------------------------------------------------
-template <int NT, int WAVES, int MT, int KS, int KWMAX, bool WV, int XL>
+template <int NT, int WAVES, int KS, int KWMAX, bool CASE_B, bool WV, int XL>
 __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* __restrict__ X, KernArgs a,
                                                                float* __restrict__ partial, AlsJob job, int has_job) {
+  constexpr int MT = CASE_B ? 4 : 2, NBUF = CASE_B ? 3 : 4;
+  constexpr bool EXACT = CASE_B || XL == 3;  // FAST as triples
   constexpr int KB = 32 * KS, PITCH = KWMAX + 8, RT = 16 * NT, NTH = WAVES * 64, ROWS = 16 * MT;
-  constexpr int LDS_WIN_U16 = 2 * RT * PITCH, LDS_RED_F = MT * NT * WAVES * 64 * 4;
-  constexpr int LDS_B = (LDS_WIN_U16 * 2 > LDS_RED_F * 4) ? LDS_WIN_U16 * 2 : LDS_RED_F * 4;
-  constexpr int LDS_BYTES = LDS_B > JOB_LDS_BYTES ? LDS_B : JOB_LDS_BYTES;
+  constexpr int LDS_WIN = (EXACT ? 3 : 2) * RT * PITCH * 2, LDS_RED = MT * NT * WAVES * 64 * 16;
+  constexpr int LDS_B = LDS_WIN > LDS_RED ? LDS_WIN : LDS_RED;
+  constexpr int LDS_BYTES = CASE_B || LDS_B > JOB_LDS_BYTES ? LDS_B : JOB_LDS_BYTES;
+  static_assert(!CASE_B || KS == 1, "case B takes blocks of 32");
   __shared__ __attribute__((aligned(16))) float smem[LDS_BYTES / 4];
-  static_assert(NTH % JOB_THREADS == 0, "the ALS job runs on the first 256 threads");
-  if (has_job && blockIdx.x == 0) {
-    // the job's workgroup: waves past the job's four end at once (a barrier
-    // no longer waits for an ended wave); with one such workgroup per CU the
-    // job has its CU to itself
-    if (threadIdx.x < JOB_THREADS) als_job_run(job, reinterpret_cast<double*>(smem));
-    return;
-  }
-  if (has_job && job.gate) {
-    // start gate: wait (a bounded number of polls) until the job has its Grams
-    if (threadIdx.x == 0) {
-      for (int it = 0; it < JOB_GATE_POLLS; ++it) {
-        if (__hip_atomic_load(job.gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == job.gate_stamp) break;
-        __builtin_amdgcn_s_sleep(8);
-      }
+  __shared__ float colmax[WAVES][RT];  // largest magnitude of each window column, by staging wave
+  __shared__ int plain;                // a wave asks for the plain form
+  if constexpr (!CASE_B) {  // the BF16 ALS contracts its last mode in fp32
+    static_assert(NTH % JOB_THREADS == 0, "the ALS job runs on the first 256 threads");
+    if (has_job && blockIdx.x == 0) {
+      // the job's workgroup: waves past the job's four end at once (a barrier
+      // no longer waits for an ended wave); with one such workgroup per CU the
+      // job has its CU to itself
+      if (threadIdx.x < JOB_THREADS) als_job_run(job, reinterpret_cast<double*>(smem));
+      return;
     }
-    __syncthreads();
+    if (has_job && job.gate) {
+      // start gate: wait (a bounded number of polls) until the job has its Grams
+      if (threadIdx.x == 0) {
+        for (int it = 0; it < JOB_GATE_POLLS; ++it) {
+          if (__hip_atomic_load(job.gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == job.gate_stamp) break;
+          __builtin_amdgcn_s_sleep(8);
+        }
+      }
+      __syncthreads();
+    }
   }
-  const int tile = (int)blockIdx.x - (has_job ? 1 : 0);
+  const int tile = (int)blockIdx.x - (!CASE_B && has_job ? 1 : 0);
   const int xt = tile % a.rtiles;
   uint16_t* sHi = reinterpret_cast<uint16_t*>(smem);
   uint16_t* sLo = sHi + RT * PITCH;
+  uint16_t* sLo2 = sLo + RT * PITCH;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar schedule and addresses
   const int g = lane >> 4, c = lane & 15;
@@ -80,8 +100,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
   // balanced split of the slow range: the first slow_rem splits take one more
   const i64 s_lo = uniform_i64((i64)ss * a.slow_q + (ss < a.slow_rem ? ss : a.slow_rem));
   const i64 s_hi = s_lo + a.slow_q + (ss < a.slow_rem ? 1 : 0);
-  // rows of this window that exist (XL == 1: a ragged fastest mode, whose loads
-  // are masked past kv; kv is a multiple of the 8-element load vector)
+  // rows of this window that exist
   const int kv = XL == 0 ? a.kw : (int)min((i64)a.kw, a.fast_size - (i64)w * a.kw);
   const int nkb = XL == 0 ? a.kw / KB : (kv + KB - 1) / KB;
   // the workgroup's blocks (slow index, then block within it) in WAVES contiguous,
@@ -91,16 +110,11 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
   const i64 wb0 = uniform_i64(wave * nblk_wg / WAVES), wb1 = (wave + 1) * nblk_wg / WAVES;
   const int T = __builtin_amdgcn_readfirstlane((int)(wb1 - wb0));  // blocks of this wave
   const i64 row_base = (i64)xt * ROWS;
+  if (tid == 0) plain = 0;
 
   FastWindow<RT, NTH, KWMAX> fw;  // window loads before the X blocks
   stage_window_load<WV>(fw, a, w, kv);
 
-  i64 rowc[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const i64 rr = row_base + 16 * mt + c;
-    rowc[mt] = rr < a.I ? rr : a.I - 1;
-  }
   floatx4 acc[MT][NT], Tacc[MT][NT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
@@ -110,18 +124,35 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
       Tacc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
 
+  // case A: x[mt][ks], 8 j of a row; case B: the 8 j, four rows each
   struct Buf {
-    bf16x8 x[MT][KS];
+    uint32x4 x[CASE_B ? 4 : MT][KS];
     float pre[NT];
     int kb;
-    uint32_t okm;  // XL == 1: bit ks set where the vector of k-step ks lies below kv
+    uint32_t okm;  // XL 1: bit ks set where the vector of k-step ks lies below kv
   };
 
   // per-lane element offsets, fixed for the whole loop; the per-block part of
   // every address is wave-uniform
   i64 loff[MT];
+  int shift = 0;  // case B: bits by which the lane's rows lie above the loaded four
+  if constexpr (!CASE_B) {
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) loff[mt] = rowc[mt] * a.Q + 8 * g;
+    for (int mt = 0; mt < MT; ++mt) {
+      const i64 rr = row_base + 16 * mt + c;
+      loff[mt] = (rr < a.I ? rr : a.I - 1) * a.Q + 8 * g;
+    }
+  } else {
+    const i64 rr = row_base + MT * c, top = a.I > MT ? a.I - MT : 0;
+    loff[0] = (i64)(8 * g) * a.I + (rr < top ? rr : top);
+    if (XL != 0 && rr > top && rr < a.I) shift = 16 * (int)(rr - top);
+  }
+  // XL 3: a block starting past `lim` would read past the end of X
+  i64 lim = 0;
+  if constexpr (XL == 3) {
+    const i64 last = (row_base + ROWS < a.I ? row_base + ROWS : a.I) - 1;
+    lim = uniform_i64(CASE_B ? a.total - (i64)(KB - 1) * a.I - (a.I > MT ? a.I : MT) : a.total - last * a.Q - KB);
+  }
   // PRE column of each lane: columns past rcount read column r0 (those
   // accumulator columns are never stored)
   const bool has_pre = a.pre != nullptr;
@@ -131,95 +162,202 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) poff[nt] = (has_pre ? a.r0 : 0) + (16 * nt + c < a.rcount ? 16 * nt + c : 0);
 
-  BlockCursor<1, KB, false> cur(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
+  BlockCursor<1, KB, CASE_B> cur(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
 
   auto load = [&](int t, Buf& b) {
     b.kb = cur.kb;
     const float* prow = pre_base + cur.slow * pre_stride;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) b.pre[nt] = prow[poff[nt]];
-    const bool live = t < T;  // past the end: one cache line at X (see the FP32 kernel)
-    const uint16_t* ubase = X + (live ? cur.offset(a) : 0);
-    // XL == 1: vectors at k >= kv are loaded from X instead and zeroed in compute();
-    // XL == 4 (a zero-padded copy): no masks
-    uint32_t okm = 0xffu;
-    if constexpr (XL > 0 && XL != 4) {
-      okm = 0;
+    const bool live = t < T;  // past the end: one cache line at X (see the fp32 kernel)
+    const i64 off = live ? cur.offset(a) : 0;
+    const uint16_t* ubase = X + off;
+    bool inside = true;  // uniform
+    if constexpr (XL == 3) inside = live ? off <= lim : a.total >= 8;
+    // XL 1: vectors at k >= kv (a multiple of 8) are loaded from X instead and zeroed
+    b.okm = 0xffu;
+    if constexpr (XL == 1) {
+      b.okm = 0;
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) okm |= (live && b.kb * KB + 32 * ks + 8 * g < kv) ? 1u << ks : 0u;
+      for (int ks = 0; ks < KS; ++ks) b.okm |= (live && b.kb * KB + 32 * ks + 8 * g < kv) ? 1u << ks : 0u;
     }
-    b.okm = okm;
+    if constexpr (!CASE_B) {
+      if (XL != 3 || inside) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const uint16_t* base = ubase + (live ? loff[mt] : 0);
+        for (int mt = 0; mt < MT; ++mt) {
+          const uint16_t* base = ubase + (live ? loff[mt] : 0);
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        b.x[mt][ks] = *reinterpret_cast<const bf16x8*>(((okm >> ks) & 1u) ? base + 32 * ks : X);
+          for (int ks = 0; ks < KS; ++ks) {
+            if constexpr (XL == 3) __builtin_memcpy(&b.x[mt][ks], __builtin_assume_aligned(base + 32 * ks, 2), 16);
+            else b.x[mt][ks] = *reinterpret_cast<const uint32x4*>(((b.okm >> ks) & 1u) ? base + 32 * ks : X);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) {
+            const int k = b.kb * KB + 8 * g + e;
+            const uint32_t lo = *(live && k < kv ? ubase + loff[mt] + e : X);
+            const uint32_t hi = *(live && k + 1 < kv ? ubase + loff[mt] + e + 1 : X);
+            b.x[mt][0][e / 2] = lo | hi << 16;
+          }
+      }
+    } else {
+      const uint16_t* base = ubase + (live ? loff[0] : 0);
+      const i64 stride = live ? a.I : 0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint16_t* p = base + e * stride;
+        uint32x2 v;
+        if constexpr (XL == 3) {
+          if (inside) {
+            __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 8);
+          } else {
+            const uint16_t* q = live && b.kb * KB + 8 * g + e < kv ? p : X;
+            const i64 room = X + a.total - q;  // at least 1
+            uint32_t h[4];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) h[m] = q[m < room ? m : 0];
+            v = uint32x2{h[0] | h[1] << 16, h[2] | h[3] << 16};
+          }
+        } else {
+          v = *reinterpret_cast<const uint32x2*>(p);
+        }
+        b.x[e / 2][0][2 * (e % 2)] = v[0];
+        b.x[e / 2][0][2 * (e % 2) + 1] = v[1];
       }
     }
     if (t + 1 < T) cur.step(a);
   };
 
+  uint32_t rmax[MT];  // largest |x| of the lane's rows in this wave's blocks: even j, odd j
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) rmax[mt] = 0;
   auto compute = [&](int t, const Buf& b) {
     if (t >= T) return;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      bf16x8 xv[MT];
+      uint32x4 xw[MT];
+      if constexpr (!CASE_B) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        xv[mt] = b.x[mt][ks];
-        if constexpr (XL > 0 && XL != 4) {
-          if (!((b.okm >> ks) & 1u)) xv[mt] = bf16x8{};
+        for (int mt = 0; mt < MT; ++mt) {
+          xw[mt] = b.x[mt][ks];
+          if constexpr (XL == 1) {
+            if (!((b.okm >> ks) & 1u)) xw[mt] = uint32x4{};
+          }
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          uint32x2 j0 = {b.x[e / 2][0][0], b.x[e / 2][0][1]}, j1 = {b.x[e / 2][0][2], b.x[e / 2][0][3]};
+          if constexpr (XL == 3) {
+            j0 = __builtin_bit_cast(uint32x2, __builtin_bit_cast(uint64_t, j0) >> shift);
+            j1 = __builtin_bit_cast(uint32x2, __builtin_bit_cast(uint64_t, j1) >> shift);
+          }
+          // low halves of (j0, j1), then high halves
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            xw[2 * h][e / 2] = __builtin_amdgcn_perm(j1[h], j0[h], 0x05040100u);
+            xw[2 * h + 1][e / 2] = __builtin_amdgcn_perm(j1[h], j0[h], 0x07060302u);
+          }
         }
       }
-      // two rank tiles at a time, the hi term of all four accumulators before
-      // their lo term (no MFMA waits for the one just issued)
-      constexpr int NG = NT >= 2 ? 2 : 1;
+      if constexpr (XL == 3) {
+        if (b.kb * KB + KB > kv) {  // the window's partly filled last block
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) {
+            const int k = b.kb * KB + 8 * g + e;
+            const uint32_t mask = (k < kv ? 0xffffu : 0u) | (k + 1 < kv ? 0xffff0000u : 0u);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) xw[mt][e / 2] &= mask;
+          }
+        }
+      }
+      if constexpr (EXACT)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) rmax[mt] = max_u16x2(rmax[mt], xw[mt][q] & 0x7fff7fffu);
+      bf16x8 xv[MT];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) xv[mt] = __builtin_bit_cast(bf16x8, xw[mt]);
+      // at least four accumulators between two products of one (no MFMA waits
+      // for the one just issued), smallest term first
+      constexpr int NG = NT >= 2 && !CASE_B ? 2 : 1;
 #pragma unroll
       for (int n0 = 0; n0 < NT; n0 += NG) {
-        bf16x8 bh[NG], bl[NG];
+        bf16x8 bh[NG], bl[NG], bl2[NG];
 #pragma unroll
         for (int u = 0; u < NG; ++u) {
           const int off = (16 * (n0 + u) + c) * PITCH + b.kb * KB + 32 * ks + 8 * g;
           bh[u] = *reinterpret_cast<const bf16x8*>(&sHi[off]);
           bl[u] = *reinterpret_cast<const bf16x8*>(&sLo[off]);
+          if constexpr (EXACT) bl2[u] = *reinterpret_cast<const bf16x8*>(&sLo2[off]);
         }
-#pragma unroll
-        for (int u = 0; u < NG; ++u)
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt)
-            Tacc[mt][n0 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv[mt], bh[u], Tacc[mt][n0 + u], 0, 0, 0);
-#pragma unroll
-        for (int u = 0; u < NG; ++u)
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt)
-            Tacc[mt][n0 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv[mt], bl[u], Tacc[mt][n0 + u], 0, 0, 0);
+#define TENRSO_BF16_TERM(XB)                                                                       \
+  _Pragma("unroll") for (int u = 0; u < NG; ++u) _Pragma("unroll") for (int mt = 0; mt < MT; ++mt) \
+      Tacc[mt][n0 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv[mt], XB[u], Tacc[mt][n0 + u], 0, 0, 0);
+        if constexpr (EXACT) {
+          TENRSO_BF16_TERM(bl2)
+          TENRSO_BF16_TERM(bl)
+          TENRSO_BF16_TERM(bh)
+        } else {
+          TENRSO_BF16_TERM(bh)
+          TENRSO_BF16_TERM(bl)
+        }
+#undef TENRSO_BF16_TERM
       }
     }
     // a slow index ends, or this wave's range does (it may end inside one)
     if (b.kb == nkb - 1 || t == T - 1) fold_slow<MT, NT>(acc, Tacc, b.pre);
   };
 
-  Buf b0, b1, b2, b3;
-  load(0, b0);
-  load(1, b1);
-  load(2, b2);
+  Buf b[NBUF];
+#pragma unroll
+  for (int i = 0; i < NBUF - 1; ++i) load(i, b[i]);
   if constexpr (XL > 0) window_zero_tail(fw, kv);
-  stage_window_store_bf16x2<RT, PITCH, NTH, KWMAX>(sHi, sLo, fw);
+  if constexpr (EXACT) {
+    window_colmax(fw, lane, colmax[wave]);
+    stage_window_store_bf16x3<RT, PITCH, NTH, KWMAX>(sHi, sLo, sLo2, fw);
+  } else {
+    stage_window_store_bf16x2<RT, PITCH, NTH, KWMAX>(sHi, sLo, fw);
+  }
   __syncthreads();  // LDS window staged
-  for (int t = 0; t < T; t += 4) {
-    load(t + 3, b3);
-    compute(t, b0);
-    load(t + 4, b0);
-    compute(t + 1, b1);
-    load(t + 5, b1);
-    compute(t + 2, b2);
-    load(t + 6, b2);
-    compute(t + 3, b3);
+  for (int t = 0; t < T; t += NBUF) {
+#pragma unroll
+    for (int i = 0; i < NBUF; ++i) {
+      load(t + i + NBUF - 1, b[(i + NBUF - 1) % NBUF]);
+      compute(t + i, b[i]);
+    }
   }
 
-  wg_reduce_store<MT, NT, WAVES>(acc, smem, wave, lane, partial + (i64)split * a.I * a.R, a.I, a.R, a.r0, a.rcount,
-                                 row_base, false);
+  float* out = partial + (i64)split * a.I * a.R;
+  if constexpr (EXACT) {
+    // not finite, or small enough for the low parts (2^-16 of the products) to leave
+    // the exponent range: all of it again in fp32
+    float cm = 0.f;
+#pragma unroll
+    for (int v = 0; v < WAVES; ++v) cm = fmaxf(cm, colmax[v][lane % RT]);
+    const float cmin = wave_min(cm > 0.f ? cm : 0x1p126f);
+    float xmin = 0x1p126f;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      float m = fmaxf(__uint_as_float(rmax[mt] << 16), __uint_as_float(rmax[mt] & 0xffff0000u));
+      m = fmaxf(m, __shfl_xor(m, 16, 64));
+      m = fmaxf(m, __shfl_xor(m, 32, 64));
+      xmin = m > 0.f ? fminf(xmin, m) : xmin;
+    }
+    xmin = wave_min(xmin);
+    const bool small = xmin < 0x1p-110f || cmin < 0x1p-96f || xmin * cmin < 0x1p-90f;
+    if (__any(!(sum_of_zeros<MT, NT>(acc) == 0.f)) || small) plain = 1;
+    __syncthreads();
+    if (plain) {
+      plain_tile<CASE_B>(X, a, out, row_base, ROWS, w, kv, s_lo, s_hi, NTH);
+      return;
+    }
+  }
+  wg_reduce_store<MT, NT, WAVES, !EXACT>(acc, smem, wave, lane, out, a.I, a.R, a.r0, a.rcount, row_base, CASE_B);
 }
 
 // ---------------------------------------------------------------------------
@@ -326,10 +464,9 @@ __global__ __launch_bounds__(256) void f32_to_bf16_kernel(const float* __restric
   }
 }
 
-// [rows, K] -> [K, rows] transpose through a 32x32 LDS tile: fp32 -> bf16 (RNE),
-// bf16 -> bf16 or fp32 -> fp32.
+// [rows, K] -> [K, rows] transpose through a 32x32 LDS tile: fp32 -> bf16 (RNE)
+// or fp32 -> fp32.
 __device__ __forceinline__ uint16_t to_out(float v, uint16_t*) { return f32_to_bf16_rne(v); }
-__device__ __forceinline__ uint16_t to_out(uint16_t v, uint16_t*) { return v; }
 __device__ __forceinline__ float to_out(float v, float*) { return v; }
 
 // With B < Bp the output rows are padded: input row r = a*B + b lands at
@@ -663,34 +800,33 @@ int prepare_bf16_als(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, 
   return TENRSO_OK;
 }
 
-int transpose_last_to_front_u16(tenrso_ctx* ctx, const uint16_t* src, int nd, const i64* shape, uint16_t* dst) {
-  i64 total = 1;
-  for (int k = 0; k < nd; ++k) total *= shape[k];
-  if (total == 0) return TENRSO_OK;
-  const i64 K = shape[nd - 1], rows = total / K;
-  hipLaunchKernelGGL((transpose_kernel<uint16_t, uint16_t>), dim3(cdiv(K, 32), cdiv(rows, 32)), dim3(256), 0,
-                     ctx->stream, src, rows, K, dst);
-  TENRSO_HIP_TRY(hipGetLastError());
-  return TENRSO_OK;
-}
-
 namespace {
 
 // The bf16 instance for nt rank tiles of 16, blocks of 32 ks elements, wv (16-byte
-// window loads) and the load form xl: 0 whole windows, 1 masked, 4 a zero-padded
-// copy.  ks = 2 only with xl 0 (a fastest mode divisible by 64 is never ragged).
+// window loads) and the load form xl.  ks = 2 only in case A with xl 0 (a fastest
+// mode divisible by 64 is never ragged).
 constexpr int BF16_WAVES = 8, BF16_KWMAX = 128;
-template <int NT, bool WV>
+template <int NT, bool CASE_B, bool WV>
 const void* bf16_pick(int ks, int xl) {
-  if (ks == 2) return reinterpret_cast<const void*>(mttkrp_bf16_mfma<NT, BF16_WAVES, 2, 2, BF16_KWMAX, WV, 0>);
-  if (xl == 0) return reinterpret_cast<const void*>(mttkrp_bf16_mfma<NT, BF16_WAVES, 2, 1, BF16_KWMAX, WV, 0>);
-  if (xl == 4) return reinterpret_cast<const void*>(mttkrp_bf16_mfma<NT, BF16_WAVES, 2, 1, BF16_KWMAX, WV, 4>);
-  return reinterpret_cast<const void*>(mttkrp_bf16_mfma<NT, BF16_WAVES, 2, 1, BF16_KWMAX, WV, 1>);
+  constexpr int W = BF16_WAVES, K = BF16_KWMAX;
+  if constexpr (!CASE_B) {
+    if (ks == 2) return reinterpret_cast<const void*>(mttkrp_bf16_mfma<NT, W, 2, K, CASE_B, WV, 0>);
+    if (xl == 4) return reinterpret_cast<const void*>(mttkrp_bf16_mfma<NT, W, 1, K, CASE_B, WV, 4>);
+  }
+  if (xl == 0) return reinterpret_cast<const void*>(mttkrp_bf16_mfma<NT, W, 1, K, CASE_B, WV, 0>);
+  if constexpr (!CASE_B) {
+    if (xl == 1) return reinterpret_cast<const void*>(mttkrp_bf16_mfma<NT, W, 1, K, CASE_B, WV, 1>);
+  }
+  return reinterpret_cast<const void*>(mttkrp_bf16_mfma<NT, W, 1, K, CASE_B, WV, 3>);
 }
-const void* mttkrp_bf16_kernel(int nt, bool wv, int ks, int xl) {
-  if (nt == 1) return wv ? bf16_pick<1, true>(ks, xl) : bf16_pick<1, false>(ks, xl);
-  if (nt == 2) return wv ? bf16_pick<2, true>(ks, xl) : bf16_pick<2, false>(ks, xl);
-  return wv ? bf16_pick<4, true>(ks, xl) : bf16_pick<4, false>(ks, xl);
+template <int NT>
+const void* bf16_pick(bool case_b, bool wv, int ks, int xl) {
+  if (case_b) return wv ? bf16_pick<NT, true, true>(ks, xl) : bf16_pick<NT, true, false>(ks, xl);
+  return wv ? bf16_pick<NT, false, true>(ks, xl) : bf16_pick<NT, false, false>(ks, xl);
+}
+const void* mttkrp_bf16_kernel(int nt, bool case_b, bool wv, int ks, int xl) {
+  return nt == 1 ? bf16_pick<1>(case_b, wv, ks, xl)
+                 : (nt == 2 ? bf16_pick<2>(case_b, wv, ks, xl) : bf16_pick<4>(case_b, wv, ks, xl));
 }
 
 struct Plan {
@@ -721,7 +857,7 @@ Plan make_plan(int nd, const i64* shape, int mode) {
 
 int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int nd, const i64* shape,
                  const float* const* F, i64 R, int mode, MttkrpOut outk, void* out, MttkrpResult* res,
-                 const AlsJob* job, bool xt_f32, const MttkrpScratch* scratch, i64 x_pad, i64 xt_pad,
+                 const AlsJob* job, const MttkrpScratch* scratch, i64 x_pad, i64 xt_pad,
                  const float* pre_rows, bool want_norm) {
   Plan pl = make_plan(nd, shape, mode);
   const bool bf16 = prec == TENRSO_PREC_BF16;
@@ -732,17 +868,11 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
   i64 shape_use[MAXD];
   for (int k = 0; k < nd; ++k) shape_use[k] = shape[k];
 
-  // BF16 last mode: run mode 0 of the last-to-front copy (same j order); an
-  // fp32 copy is contracted exactly (bf16x3 split).  FP32 with a last-to-front
-  // fp32 copy given: its last mode also runs as mode 0 of the copy (q-contiguous
-  // 16-byte loads instead of the last mode's i-contiguous ones).
+  // With a last-to-front copy given (fp32, also of a BF16 call), the last mode runs
+  // as mode 0 of the copy (same j order).
   bool x3 = false;
-  if ((bf16 || X_t) && mode == nd - 1 && nd >= 2) {
-    x3 = bf16 && xt_f32;
-    if (!X_t) {
-      set_error("internal: bf16 last-mode MTTKRP needs the last-to-front copy");
-      return TENRSO_ERR_INVALID_ARGUMENT;
-    }
+  if (X_t && mode == nd - 1 && nd >= 2) {
+    x3 = bf16;
     Xuse = X_t;
     mode_use = 0;
     shape_use[0] = shape[nd - 1];
@@ -837,8 +967,9 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
   a.pre = pre;
   a.fast = fastf;
 
-  const int KB = (bf16 && !x3) ? ((pl.fast_size % 64 == 0) ? 64 : 32) : 32;
-  constexpr int KWMAX = 128;  // LDS window bound (64 x 136 bf16, three or two planes)
+  const bool fp32 = !bf16 || x3;
+  const int KB = !fp32 && !caseB && pl.fast_size % 64 == 0 && (uintptr_t)Xuse % 16 == 0 ? 64 : 32;
+  constexpr int KWMAX = 128;  // LDS window bound (64 x 136 bf16, three planes)
   // LDS window of the fastest mode: the largest multiple of KB that divides it.
   // A fastest mode no such window divides ("ragged", e.g. 100 or 250) takes
   // windows of a multiple of 32 rows covering it as evenly as possible, the last
@@ -849,7 +980,6 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
       kw = (int)cand;
       break;
     }
-  const bool fp32 = !bf16 || x3;
   const uintptr_t xaddr = (uintptr_t)Xuse;
   int XL = 0;
   if (kw == 0 && pl.fast_size > 0) {
@@ -862,20 +992,19 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
   // (the pads are zero, and window rows past kv are staged as zeros); only the
   // window load keeps kv (XL 4)
   if (!caseB && pad > 0 && XL == 1 && xaddr % 16 == 0 && fast_stride >= (pl.fast_size + 31) / 32 * 32) XL = 4;
-  // The fp32 kernel's unmasked forms read aligned vectors (16 bytes of a row; 8
-  // bytes of two rows in case B); every other tensor, at any 4-byte alignment,
-  // takes XL 1.  The bf16 kernel needs 16-byte aligned rows, else the generic one
-  // runs.
-  if (fp32 && XL == 0 && (caseB ? I % 2 != 0 || xaddr % 8 != 0 : xaddr % 16 != 0)) XL = 1;
-  const bool mfma_ok = pl.n_oth >= 1 && pl.J > 0 && kw > 0 && I > 0 &&
-                       (fp32 ? xaddr % 4 == 0 : !caseB && xaddr % 16 == 0 && (XL != 1 || fast_stride % 8 == 0));
+  // The unmasked forms read aligned vectors: 16 bytes of a row; in case B 8 bytes of
+  // two (fp32) or four (bf16) rows.  Every other tensor, at any alignment of its
+  // type, takes XL 1 (fp32) or, unless its rows are 16-byte aligned, XL 3 (bf16).
+  if (XL == 0 && (caseB ? I % (fp32 ? 2 : 4) != 0 || xaddr % 8 != 0 : xaddr % 16 != 0)) XL = 1;
+  if (!fp32 && XL == 1 && (caseB || fast_stride % 8 != 0 || xaddr % 16 != 0)) XL = 3;
+  const bool mfma_ok = pl.n_oth >= 1 && pl.J > 0 && kw > 0 && I > 0 && xaddr % (fp32 ? 4 : 2) == 0;
 
   float* partial = nullptr;
   int splits = 1;
   const double* norm = nullptr;
   int nnorm = 0;
   if (mfma_ok) {
-    constexpr i64 rows_per_wg = 32;
+    const i64 rows_per_wg = !fp32 && caseB ? 64 : 32;
     const i64 rtiles = (i64)cdiv(I, rows_per_wg);
     const i64 tiles = rtiles * rchunks;
     a.kw = kw;
@@ -907,13 +1036,13 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
     // the job shares the launch it takes one of the resident slots, so every
     // workgroup is resident at once.
     int waves = 8, occ = 0;
-    const void* kern = !fp32 ? mttkrp_bf16_kernel(NT, a.win_vec, KB / 32, XL)
+    const void* kern = !fp32 ? mttkrp_bf16_kernel(NT, caseB, a.win_vec, KB / 32, XL)
                              : (NT == 8 ? mttkrp_x3_kernel_n8(caseB, a.win_vec, XL)
                                         : mttkrp_x3_kernel_w8(NT, caseB, a.win_vec, XL));
     TENRSO_TRY(occupancy(kern, waves * 64, &occ));
     int wpc = bf16 ? ctx->wg_per_cu_bf16 : ctx->wg_per_cu_f32;  // TENRSO_WG_PER_CU_* override
     if (wpc <= 0) wpc = std::min(occ, 2);
-    const bool fuse_job = job != nullptr && rchunks == 1 && (job->R <= JOB_NE || NT == 8);
+    const bool fuse_job = job != nullptr && rchunks == 1 && (job->R <= JOB_NE || NT == 8) && (fp32 || !caseB);
     i64 target = (i64)wpc * ctx->num_cus - ((fuse_job && occ <= wpc) ? 1 : 0);
     // Splits of the slow range: the count with the least (rounds of resident
     // workgroups) x (blocks of its slowest wave + 3), a workgroup's start and end

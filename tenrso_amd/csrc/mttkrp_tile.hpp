@@ -12,6 +12,8 @@ namespace tenrso {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx8 __attribute__((ext_vector_type(8)));
+typedef uint32_t uint32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t uint32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 
@@ -110,21 +112,46 @@ __device__ __forceinline__ void window_zero_tail(FastWindow<RT, NTH, KWMAX>& fw,
   }
 }
 
-template <int RT, int PITCH, int NTH, int KWMAX>
-__device__ __forceinline__ void stage_window_store(float* __restrict__ s, const FastWindow<RT, NTH, KWMAX>& fw) {
-  static_assert(PITCH % 2 == 0, "pairs of window rows are stored as 8-byte words");
-#pragma unroll
-  for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e) {
-    const int u = threadIdx.x + e * NTH;
-    const int r4 = 4 * (u % (RT / 4)), kk = 2 * (u / (RT / 4));
-    if (!FastWindow<RT, NTH, KWMAX>::live(u)) continue;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      *reinterpret_cast<float2*>(&s[(r4 + q) * PITCH + kk]) = float2{fw.v[e][0][q], fw.v[e][1][q]};
-  }
+// m = max(m, |a|, |b|)
+__device__ __forceinline__ void max3_abs(float& m, float a, float b) {
+  asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b));
 }
 
-// Same window as an exact bf16 pair: FAST = hi + lo with hi = bf16(FAST) and
+// maxima of two unsigned 16-bit halves
+__device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b) {
+  typedef unsigned short ushortx2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(
+      uint32_t, __builtin_elementwise_max(__builtin_bit_cast(ushortx2, a), __builtin_bit_cast(ushortx2, b)));
+}
+
+// smallest over the wave
+__device__ __forceinline__ float wave_min(float v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
+  return v;
+}
+
+// Largest magnitudes of the window's columns among the rows a wave stages, into its
+// colmax[RT].  A thread's units are all of the same four ranks (NTH is a multiple of
+// RT / 4), and the lanes RT / 4 apart hold them too.  Ranks past rcount repeat a
+// valid column.
+template <int RT, int NTH, int KWMAX>
+__device__ __forceinline__ void window_colmax(const FastWindow<RT, NTH, KWMAX>& fw, int lane, float* colmax) {
+  float m[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) max3_abs(m[q], fw.v[e][0][q], fw.v[e][1][q]);
+#pragma unroll
+  for (int o = RT / 4; o < 64; o <<= 1)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) m[q] = fmaxf(m[q], __shfl_xor(m[q], o, 64));
+  if (lane < RT / 4)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) colmax[4 * lane + q] = m[q];
+}
+
+// The window in LDS as a bf16 pair: FAST = hi + lo with hi = bf16(FAST) and
 // lo = bf16(FAST - hi), so hi + lo carries 16 significant bits.
 template <int RT, int PITCH, int NTH, int KWMAX>
 __device__ __forceinline__ void stage_window_store_bf16x2(uint16_t* __restrict__ shi, uint16_t* __restrict__ slo,
@@ -150,7 +177,7 @@ __device__ __forceinline__ void stage_window_store_bf16x2(uint16_t* __restrict__
   }
 }
 
-// Same window as an exact bf16 triple: FAST = hi + lo + lo2 (hi = bf16(FAST),
+// The same as an exact bf16 triple: FAST = hi + lo + lo2 (hi = bf16(FAST),
 // lo = bf16(FAST - hi), lo2 = bf16(FAST - hi - lo)); each residual is exact in
 // fp32 and the last one has at most 8 significant bits, so for every normal
 // fp32 value hi + lo + lo2 equals FAST exactly.
@@ -178,15 +205,6 @@ __device__ __forceinline__ void stage_window_store_bf16x3(uint16_t* __restrict__
       *reinterpret_cast<uint32_t*>(&slo2[o]) = l2w;
     }
   }
-}
-
-// Exact three-way bf16 split of 8 fp32 values (see stage_window_store_bf16x3).
-__device__ __forceinline__ void split_bf16x3(const floatx8& x, bf16x8& h, bf16x8& l, bf16x8& l2) {
-  h = __builtin_convertvector(x, bf16x8);
-  const floatx8 r = x - __builtin_convertvector(h, floatx8);
-  l = __builtin_convertvector(r, bf16x8);
-  const floatx8 r2 = r - __builtin_convertvector(l, floatx8);
-  l2 = __builtin_convertvector(r2, bf16x8);
 }
 
 // A value the compiler cannot prove uniform but that is: move it to scalar registers.
@@ -309,6 +327,44 @@ __device__ __forceinline__ void fold_slow(floatx4 (&acc)[MT][NT], floatx4 (&T)[M
       acc[mt][nt] += T[mt][nt] * pre[nt];
       T[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
+}
+
+// Zero if every accumulator is finite, else NaN.
+template <int MT, int NT>
+__device__ __forceinline__ float sum_of_zeros(const floatx4 (&acc)[MT][NT]) {
+  float z = 0.f;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) z = fmaf(acc[mt][nt][v], 0.f, z);
+  return z;
+}
+
+__device__ __forceinline__ float to_f32(float x) { return x; }
+__device__ __forceinline__ float to_f32(uint16_t x) { return __uint_as_float((uint32_t)x << 16); }
+
+// The tile of one workgroup in plain fp32: acc = fma(x, pre * fast, acc) over its
+// slow range and window, one thread an output.
+template <bool CASE_B, typename TX>
+__device__ __forceinline__ void plain_tile(const TX* X, const KernArgs& a, float* out, i64 row_base, int rows, int w,
+                                           int kv, i64 s_lo, i64 s_hi, int nth) {
+  for (int e = threadIdx.x; e < rows * a.rcount; e += nth) {
+    const i64 row = row_base + e / a.rcount;
+    const int r = a.r0 + e % a.rcount;
+    if (row >= a.I) continue;
+    float acc = 0.f;
+    for (i64 slow = s_lo; slow < s_hi; ++slow) {
+      const float pre = a.pre ? a.pre[slow * a.R + r] : 1.f;
+      const i64 p = CASE_B ? 0 : slow / a.qs;
+      const TX* x = CASE_B ? X + (slow * a.fast_size + (i64)w * a.kw) * a.I + row
+                           : X + (p * a.I + row) * a.Q + (slow - p * a.qs) * a.fast_stride + (i64)w * a.kw;
+      const float* f = a.fast + (i64)w * a.kw * a.R + r;
+      for (int k = 0; k < kv; ++k) acc = fmaf(to_f32(x[CASE_B ? (i64)k * a.I : k]), pre * f[(i64)k * a.R], acc);
+    }
+    out[row * a.R + r] = acc;
+  }
 }
 
 }  // namespace tenrso

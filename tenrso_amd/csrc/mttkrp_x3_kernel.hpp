@@ -61,41 +61,7 @@ __device__ __forceinline__ void x3_split(const floatx8& x, bf16x8& h, bf16x8& l,
   }
 }
 
-// m = max(m, |a|, |b|)
-__device__ __forceinline__ void x3_max3(float& m, float a, float b) {
-  asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b));
-}
-
-// smallest over the wave
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
-  return v;
-}
-
-// The tile of one workgroup in plain fp32: acc = fma(x, pre * fast, acc) over its
-// slow range and window, one thread an output.
-template <bool CASE_B>
-__device__ __forceinline__ void x3_plain_tile(const float* X, const KernArgs& a, float* out, i64 row_base, int rows,
-                                           int w, int kv, i64 s_lo, i64 s_hi, int nth) {
-  for (int e = threadIdx.x; e < rows * a.rcount; e += nth) {
-    const i64 row = row_base + e / a.rcount;
-    const int r = a.r0 + e % a.rcount;
-    if (row >= a.I) continue;
-    float acc = 0.f;
-    for (i64 slow = s_lo; slow < s_hi; ++slow) {
-      const float pre = a.pre ? a.pre[slow * a.R + r] : 1.f;
-      const i64 p = CASE_B ? 0 : slow / a.qs;
-      const float* x = CASE_B ? X + (slow * a.fast_size + (i64)w * a.kw) * a.I + row
-                              : X + (p * a.I + row) * a.Q + (slow - p * a.qs) * a.fast_stride + (i64)w * a.kw;
-      const float* f = a.fast + (i64)w * a.kw * a.R + r;
-      for (int k = 0; k < kv; ++k) acc = fmaf(x[CASE_B ? (i64)k * a.I : k], pre * f[(i64)k * a.R], acc);
-    }
-    out[row * a.R + r] = acc;
-  }
-}
-
-// The work split of the other MFMA kernels: a workgroup owns 32 rows and one LDS
+// The work split: a workgroup owns 32 rows and one LDS
 // window (up to 128 rows) of the fastest mode, its waves contiguous ranges of its
 // blocks (32 consecutive j).  T = X FAST is contracted per slow index and folded
 // into the accumulator with PRE[slow].  The FAST window is split once, when it
@@ -293,7 +259,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
         }
       }
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) x3_max3(rmax[mt], x[e], x[e + 1]);
+      for (int e = 0; e < 8; e += 2) max3_abs(rmax[mt], x[e], x[e + 1]);
       if constexpr (NORM) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) sumsq[mt] = fma((double)x[e], (double)x[e], sumsq[mt]);
@@ -333,23 +299,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
 #pragma unroll
   for (int i = 0; i < NBUF - 1; ++i) load(i, b[i]);
   if constexpr (XL > 0) window_zero_tail(fw, kv);
-  {
-    // column maxima: a thread's units are all of the same four ranks (NTH is a
-    // multiple of RT / 4), and the lanes RT / 4 apart hold them too.  Ranks past
-    // rcount repeat a valid column.
-    float m[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) x3_max3(m[q], fw.v[e][0][q], fw.v[e][1][q]);
-#pragma unroll
-    for (int o = RT / 4; o < 64; o <<= 1)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) m[q] = fmaxf(m[q], __shfl_xor(m[q], o, 64));
-    if (lane < RT / 4)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) colmax[wave][4 * lane + q] = m[q];
-  }
+  window_colmax(fw, lane, colmax[wave]);
   stage_window_store_bf16x3<RT, PITCH, NTH, KWMAX>(sHi, sLo, sLo2, fw);
   __syncthreads();  // LDS window staged
   for (int t = 0; t < T; t += NBUF) {
@@ -375,13 +325,6 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
 
   // not finite, or small enough for the low parts (2^-16 of the products) to leave
   // the exponent range: all of it again in fp32
-  float z = 0.f;
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) z = fmaf(acc[mt][nt][v], 0.f, z);
   float rmin = 0x1p126f, cmin = 0x1p126f;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
@@ -398,11 +341,11 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
   rmin = wave_min(rmin);
   cmin = wave_min(cmin);
   const bool small = rmin < 0x1p-96f || cmin < 0x1p-96f || rmin * cmin < 0x1p-90f;
-  if (__any(!(z == 0.f)) || small) plain = 1;
+  if (__any(!(sum_of_zeros<MT, NT>(acc) == 0.f)) || small) plain = 1;
   __syncthreads();
   float* out = partial + (i64)split * a.I * a.R;
   if (plain) {
-    x3_plain_tile<CASE_B>(X, a, out, row_base, ROWS, w, kv, s_lo, s_hi, NTH);
+    plain_tile<CASE_B>(X, a, out, row_base, ROWS, w, kv, s_lo, s_hi, NTH);
     return;
   }
   wg_reduce_store<MT, NT, WAVES, false>(acc, smem, wave, lane, out, a.I, a.R, a.r0, a.rcount, row_base, CASE_B);

@@ -81,5 +81,5 @@ extern "C" int tenrso_mttkrp_f32_noalloc(tenrso_ctx* ctx, const float* X, int nd
   ws.base = base;
   ws.bytes = NOALLOC_SCRATCH_BYTES;
   return mttkrp_dense(ctx, TENRSO_PREC_FP32, X, nullptr, ndim, shape, factors, rank, mode, MttkrpOut::F32, out,
-                      nullptr, nullptr, false, &ws);
+                      nullptr, nullptr, &ws);
 }
