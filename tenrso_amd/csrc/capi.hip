@@ -215,8 +215,17 @@ int tenrso_mttkrp_profile(tenrso_ctx* ctx, int precision, const void* X, int ndi
 
 int tenrso_mttkrp_all_modes_f32(tenrso_ctx* ctx, const float* X, int ndim, const int64_t* shape,
                                 const float* const* factors, int64_t rank, float* const* outs) {
-  for (int m = 0; m < ndim; ++m) TENRSO_TRY(tenrso_mttkrp_f32(ctx, X, ndim, shape, factors, rank, m, outs[m]));
-  return TENRSO_OK;
+  clear_error();
+  if (ndim <= 0) return TENRSO_OK;
+  if (bad_ctx(ctx)) return TENRSO_ERR_INVALID_ARGUMENT;
+  TENRSO_TRY(check_mttkrp_basic(ndim, shape, rank, 0));
+  if (rank == 0) return TENRSO_OK;
+  if (ctx->timing || prod(shape, ndim) == 0) {  // (the time kept is that of the last mode)
+    for (int m = 0; m < ndim; ++m) TENRSO_TRY(tenrso_mttkrp_f32(ctx, X, ndim, shape, factors, rank, m, outs[m]));
+    return TENRSO_OK;
+  }
+  TENRSO_TRY(set_device(ctx));
+  return mttkrp_all_modes(ctx, X, ndim, shape, factors, rank, outs);
 }
 
 int tenrso_mttkrp_f32_host(tenrso_ctx* ctx, const float* X, int ndim, const int64_t* shape,

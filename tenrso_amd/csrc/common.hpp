@@ -105,6 +105,8 @@ enum BufSlot : int {
   SLOT_GRAM_CHUNKS,
   SLOT_XPAD,
   SLOT_NORM,
+  SLOT_PARTIAL_MODE,  // MAXD of them: split partials of each mode
+  SLOT_PARTIAL_MODE_END = SLOT_PARTIAL_MODE + 7,
   SLOT_COUNT
 };
 

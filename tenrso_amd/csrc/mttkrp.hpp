@@ -40,12 +40,18 @@ struct MttkrpScratch {
 // and of X_t when those copies have it padded with zeros.
 // want_norm: also leave FP64 partial sums of ||X||^2 in res->norm (FP32 calls whose
 // ranks fit one launch of the MFMA kernel; null otherwise).
+// slot: the context buffer of the split partials.
 // pre_rows (optional, tensors of order >= 4): the PRE Khatri-Rao rows of this
 // mode already formed (mttkrp_pre_batch), instead of a launch that forms them.
 int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int nd, const i64* shape,
                  const float* const* F, i64 R, int mode, MttkrpOut outk, void* out, MttkrpResult* res,
                  const AlsJob* job = nullptr, const MttkrpScratch* scratch = nullptr,
-                 i64 x_pad = 0, i64 xt_pad = 0, const float* pre_rows = nullptr, bool want_norm = false);
+                 i64 x_pad = 0, i64 xt_pad = 0, const float* pre_rows = nullptr, bool want_norm = false,
+                 int slot = SLOT_PARTIAL);
+
+// The fp32 MTTKRPs of every mode of one tensor that has elements.
+int mttkrp_all_modes(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, const float* const* F, i64 R,
+                     float* const* outs);
 
 // The PRE Khatri-Rao rows of the MTTKRPs of several modes of one tensor (order
 // >= 4) in one launch: pre[i] receives the rows the MFMA MTTKRP of modes[i]

@@ -28,6 +28,9 @@ __all__ = [
 ]
 
 
+_MAX_MODES = 8  # tensors of a higher order are refused by the library
+
+
 def _is_torch(x) -> bool:
     return type(x).__module__.startswith("torch")
 
@@ -48,6 +51,8 @@ def _dev_f32(t, device):
     reference's usual T = f64, CPU tensors) are converted, never reinterpreted."""
     import torch
     if _is_torch(t):
+        if t.dtype == torch.float32 and t.device == device and t.is_contiguous() and not t.requires_grad:
+            return t  # as it is: the conversions below cost 2 us of host time each
         if t.is_complex():
             raise TypeError("complex factors are not supported")
         return t.detach().to(device=device, dtype=torch.float32).contiguous()
@@ -61,6 +66,13 @@ def _i64s(vals):
 def _check_mttkrp(shape, factors, mode):
     """mttkrp.rs:85-122 validation (same order, same messages) via tenrso_mttkrp_check."""
     nf = len(factors)
+    # the usual, valid call needs no trip to the library (4 us)
+    if 2 <= nf == len(shape) <= _MAX_MODES and 0 <= mode < nf:
+        s0 = factors[0].shape
+        if len(s0) == 2:
+            R = int(s0[1])
+            if all(f.shape == (n, R) for f, n in zip(factors, shape)):
+                return R
     if nf == 0:
         raise ValueError(f"Number of factor matrices (0) must match tensor rank ({len(shape)})")
     rows = [int(f.shape[0]) for f in factors]
@@ -137,6 +149,22 @@ def mttkrp_fused_parallel(tensor, factors, mode: int):
 
 def mttkrp_all_modes(tensor, factors):
     """mttkrp_all_modes (utils.rs:282-311)."""
+    nd = len(tensor.shape)
+    if nd >= 2 and _is_cuda(tensor):
+        import torch
+        shape = tuple(tensor.shape)
+        R = _check_mttkrp(shape, factors, 0)
+        X = tensor.contiguous()
+        if X.dtype != torch.float32:
+            raise TypeError("device mttkrp expects a float32 CUDA tensor (the library computes in f32)")
+        F = [_dev_f32(f, X.device) for f in factors]
+        outs = [X.new_empty((n, R)) for n in shape]
+        ctx = _lib.torch_context(X)
+        ptrs = C.c_void_p * nd
+        check(lib().tenrso_mttkrp_all_modes_f32(ctx.ptr, X.data_ptr(), nd, _i64s(shape),
+                                                ptrs(*[f.data_ptr() for f in F]), R,
+                                                ptrs(*[o.data_ptr() for o in outs])))
+        return outs
     return [mttkrp(tensor, factors, m) for m in range(len(tensor.shape))]
 
 
