@@ -146,7 +146,10 @@ __device__ __forceinline__ int job_col(int t) { return 16 * t + (threadIdx.x & 1
 // and tile) and 16 of its lanes invert the next P (adjugate, below) while the
 // remaining MFMAs run.  LDS is double-buffered: one barrier per step.  Returns
 // false if a pivot block is not positive definite.
-__device__ __forceinline__ bool job_block_gj(doublex4 (&acc)[4], double* lds) {
+// Only the ceil(R / 4) steps of the matrix proper are taken: outside R x R it is the
+// identity, whose steps would change nothing (0.45 us each; all 16 at every rank left
+// the launches of small ALS problems at 13.8 us, the job's own time).
+__device__ __forceinline__ bool job_block_gj(doublex4 (&acc)[4], double* lds, int R) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int q = lane >> 4, j = lane & 15;
   int* flag = reinterpret_cast<int*>(lds + JOB_GJ_FLAG);
@@ -203,6 +206,7 @@ __device__ __forceinline__ bool job_block_gj(doublex4 (&acc)[4], double* lds) {
   }
 #pragma unroll
   for (int s = 0; s < 16; ++s) {
+    if (4 * s >= R) break;
     const int b = s & 1, T = s >> 2, e = s & 3;
     const double* Rw = lds + JOB_GJ_ROW + b * 4 * JOB_NE;
     const double* Pi = lds + JOB_GJ_PINV + b * 16;
@@ -407,7 +411,7 @@ __device__ __forceinline__ void als_job_run(const AlsJob& a, double* lds) {
     for (int e = 0; e < 4; ++e) acc[t][e] = gam[t][e];
   pad_and_band(0.0);
   TENRSO_JOB_MARK(3);
-  ok = job_block_gj(acc, lds);
+  ok = job_block_gj(acc, lds, R);
   TENRSO_JOB_MARK(4);
   if (!ok) {
     // ridge retry (cp/helpers.rs:477-490): Gamma + eps 10R I
@@ -416,7 +420,7 @@ __device__ __forceinline__ void als_job_run(const AlsJob& a, double* lds) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[t][e] = a.Winv[job_row(e) * JOB_NE + job_col(t)];
     pad_and_band((double)FLT_EPSILON * (double)(10 * R));
-    ok = job_block_gj(acc, lds);
+    ok = job_block_gj(acc, lds, R);
     path = 1;
   }
   if (!ok) path = 2;

@@ -159,8 +159,7 @@ int tenrso_convert_f32_to_bf16(tenrso_ctx* ctx, const float* src, int64_t n, uin
     return TENRSO_ERR_INVALID_ARGUMENT;
   }
   TENRSO_TRY(set_device(ctx));
-  const i64 shape1[1] = {n};
-  return convert_bf16(ctx, src, 1, shape1, false, dst);
+  return convert_bf16(ctx, src, n, dst);
 }
 
 int tenrso_mttkrp_bf16(tenrso_ctx* ctx, const uint16_t* X_bf16, int ndim, const int64_t* shape,

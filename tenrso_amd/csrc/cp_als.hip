@@ -319,11 +319,10 @@ int cp_als_device(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, flo
   pb.nd = nd;
   pb.shape = shape;
   // BF16: modes 0..N-2 contract the bf16 copy of X; the last mode, whose <M, A>
-  // gives the fit, contracts the exact fp32 tensor through its last-to-front copy
-  // (bf16x3 split on the MFMA path), so the fit is the fit to X itself.  The bf16
-  // copy, the fp32 last-to-front copy and ||X||^2 come from one pass over X when
-  // the shape allows it (prepare_bf16_als); otherwise norm, copy and transposed
-  // copy are three passes
+  // gives the fit, contracts the exact fp32 tensor, so the fit is the fit to X
+  // itself.  The bf16 copy and ||X||^2 come from one pass over X (13 us at 256^3, where
+  // a last-to-front copy in the same pass took 29 and gained the last mode nothing:
+  // 19.1 us in place, 19.5 from the copy).
   bool prepared = false;
   // A last mode that is no multiple of 8 (bf16 copy) or a mode N-2 that is no
   // multiple of 4 (the fp32 last-to-front copy, whose last mode it is) would
@@ -336,21 +335,17 @@ int cp_als_device(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, flo
   const i64 Kxp = (Kx + 7) / 8 * 8, Bt32a = (Bt + 31) / 32 * 32;
   const i64 Btp = Bt32a * 8 <= Bt * 9 ? Bt32a : (Bt + 3) / 4 * 4;
   const bool padded = bf16 && nd >= 2 && total > 0 && (Kxp != Kx || Btp != Bt);
-  auto bf16_buffers = [&](void** pb16, void** pt) -> int {
+  auto bf16_buffer = [&](void** pb16) -> int {
     const size_t nb = padded ? (size_t)(total / Kx * Kxp) : (size_t)total;
-    const size_t nt = padded ? (size_t)(total / Bt * Btp) : (size_t)total;
-    TENRSO_TRY(ctx_buffer(ctx, SLOT_XBF16, nb * 2, pb16));
-    TENRSO_TRY(ctx_buffer(ctx, SLOT_XBF16_T, nt * sizeof(float), pt));
-    return TENRSO_OK;
+    return ctx_buffer(ctx, SLOT_XBF16, nb * 2, pb16);
   };
   pb.norm_min = [&](double* tmp, double* scal) -> int {
     if (bf16 && !padded) {
-      void *pb16, *pt;
-      TENRSO_TRY(bf16_buffers(&pb16, &pt));
+      void* pb16;
+      TENRSO_TRY(bf16_buffer(&pb16));
       int nblk = 0;
-      if (prepare_bf16_als(ctx, X, nd, shape, (uint16_t*)pb16, (float*)pt, tmp, &nblk) == TENRSO_OK) {
+      if (convert_bf16_norm(ctx, X, total, (uint16_t*)pb16, tmp, &nblk) == TENRSO_OK) {
         Xk = pb16;
-        Xt = pt;
         prepared = true;
         return norm_min_finish(ctx, tmp, nblk, scal, SC_COUNT);
       }
@@ -359,17 +354,18 @@ int cp_als_device(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, flo
   };
   pb.prepare = [&]() -> int {
     if (!bf16 || prepared) return TENRSO_OK;
-    void *pb16, *pt;
-    TENRSO_TRY(bf16_buffers(&pb16, &pt));
+    void* pb16;
+    TENRSO_TRY(bf16_buffer(&pb16));
     if (padded) {
+      void* pt;
+      TENRSO_TRY(ctx_buffer(ctx, SLOT_XBF16_T, (size_t)(total / Bt * Btp) * sizeof(float), &pt));
       TENRSO_TRY(convert_bf16_padded(ctx, X, nd, shape, Kxp, (uint16_t*)pb16));
       TENRSO_TRY(transpose_last_to_front_f32_padded(ctx, X, nd, shape, Btp, (float*)pt));
+      Xt = pt;
     } else {
-      TENRSO_TRY(convert_bf16(ctx, X, nd, shape, false, (uint16_t*)pb16));
-      TENRSO_TRY(transpose_last_to_front_f32(ctx, X, nd, shape, (float*)pt));
+      TENRSO_TRY(convert_bf16(ctx, X, total, (uint16_t*)pb16));
     }
     Xk = pb16;
-    Xt = pt;
     return TENRSO_OK;
   };
   // FP32 with a last mode of no multiple of 32 floats (250^3, say): its rows are
@@ -394,6 +390,9 @@ int cp_als_device(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, flo
   }
   const i64 x_pad = padded ? Kxp : (fpad ? Kx32 : 0), xt_pad = padded ? Btp : (fpad ? Bt32 : 0);
   pb.mttkrp = [&](int mode, const float* const* Fc, const AlsJob* job, MttkrpResult* mr) {
+    if (bf16 && mode == nd - 1 && !Xt)  // the fp32 tensor in place
+      return mttkrp_dense(ctx, TENRSO_PREC_FP32, X, nullptr, nd, shape, Fc, R, mode, MttkrpOut::PARTIAL, nullptr, mr,
+                          job);
     return mttkrp_dense(ctx, bf16 ? TENRSO_PREC_BF16 : TENRSO_PREC_FP32, Xk, Xt, nd, shape, Fc, R, mode,
                         MttkrpOut::PARTIAL, nullptr, mr, job, nullptr, x_pad, xt_pad);
   };

@@ -78,15 +78,12 @@ int als_job_launch(tenrso_ctx* ctx, const AlsJob& job);
 // Sum split partials [splits, n] in FP64 into out (fp32 or fp64).
 int reduce_partials(tenrso_ctx* ctx, const float* partial, int splits, i64 n, float* out32, double* out64);
 
-// fp32 -> bf16 (RNE) copy; when `last_to_front` the output is the tensor with its
-// last mode moved to the front ([I_{N-1}, I_0, ..., I_{N-2}]).
-int convert_bf16(tenrso_ctx* ctx, const float* src, int nd, const i64* shape, bool last_to_front, uint16_t* dst);
-// BF16 ALS input in one pass: dst = bf16(X), dstT = the fp32 tensor with its last
-// mode moved to the front, and (sum of squares, min) partials in tmp[0, 2 * nblk).
-// TENRSO_ERR_UNSUPPORTED (nothing launched) unless the last mode is a multiple of
-// 4 and X is 16-byte aligned.  dst may be null: then only dstT and the partials.
-int prepare_bf16_als(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, uint16_t* dst, float* dstT,
-                     double* tmp, int* nblk_out);
+// fp32 -> bf16 (RNE) copy of n elements.
+int convert_bf16(tenrso_ctx* ctx, const float* src, i64 n, uint16_t* dst);
+// bf16 copy and the (sum of squares, min) partials of X in one pass: tmp[0, 2 * nblk).
+// TENRSO_ERR_UNSUPPORTED (nothing launched) unless total is a positive multiple of 4
+// and X is 16-byte aligned.
+int convert_bf16_norm(tenrso_ctx* ctx, const float* X, i64 total, uint16_t* dst, double* tmp, int* nblk_out);
 
 // [.., I_{N-1}] -> [I_{N-1}, ..] (last mode moved to the front), a plain copy.
 int transpose_last_to_front_f32(tenrso_ctx* ctx, const float* src, int nd, const i64* shape, float* dst);

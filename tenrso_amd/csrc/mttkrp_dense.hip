@@ -483,30 +483,25 @@ __global__ __launch_bounds__(256) void f32_to_bf16_kernel(const float* __restric
   }
 }
 
-// [rows, K] -> [K, rows] transpose through a 32x32 LDS tile: fp32 -> bf16 (RNE)
-// or fp32 -> fp32.
-__device__ __forceinline__ uint16_t to_out(float v, uint16_t*) { return f32_to_bf16_rne(v); }
-__device__ __forceinline__ float to_out(float v, float*) { return v; }
-
+// [rows, K] -> [K, rows] transpose through a 32x32 LDS tile.
 // With B < Bp the output rows are padded: input row r = a*B + b lands at
 // a*Bp + b of an output row of extent (rows / B) * Bp (the pad entries are
 // zero-filled beforehand); B = Bp leaves the layout plain.
-template <typename TIN, typename TOUT>
-__global__ __launch_bounds__(256) void transpose_kernel(const TIN* __restrict__ src, i64 rows, i64 K,
-                                                        TOUT* __restrict__ dst, i64 B = 1, i64 Bp = 1) {
-  __shared__ TIN tile[32][33];
+__global__ __launch_bounds__(256) void transpose_kernel(const float* __restrict__ src, i64 rows, i64 K,
+                                                        float* __restrict__ dst, i64 B = 1, i64 Bp = 1) {
+  __shared__ float tile[32][33];
   const i64 r0 = (i64)blockIdx.y * 32, k0 = (i64)blockIdx.x * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
   for (int yy = ty; yy < 32; yy += 8) {
     const i64 r = r0 + yy, k = k0 + tx;
-    tile[yy][tx] = (r < rows && k < K) ? src[r * K + k] : (TIN)0;
+    tile[yy][tx] = (r < rows && k < K) ? src[r * K + k] : 0.f;
   }
   __syncthreads();
   for (int yy = ty; yy < 32; yy += 8) {
     const i64 k = k0 + yy, r = r0 + tx;
     if (k < K && r < rows) {
       const i64 o = B == Bp ? k * rows + r : k * (rows / B * Bp) + (r / B) * Bp + r % B;
-      dst[o] = to_out(tile[tx][yy], dst);
+      dst[o] = tile[tx][yy];
     }
   }
 }
@@ -629,19 +624,10 @@ int khatri_rao_many(tenrso_ctx* ctx, int n, const float* const* F, const i64* si
   return TENRSO_OK;
 }
 
-int convert_bf16(tenrso_ctx* ctx, const float* src, int nd, const i64* shape, bool last_to_front, uint16_t* dst) {
-  i64 total = 1;
-  for (int k = 0; k < nd; ++k) total *= shape[k];
-  if (total == 0) return TENRSO_OK;
-  if (!last_to_front || nd < 2) {
-    const int vec = (uintptr_t)src % 16 == 0 && (uintptr_t)dst % 8 == 0;
-    hipLaunchKernelGGL(f32_to_bf16_kernel, dim3(cdiv(cdiv(total, 4), 256)), dim3(256), 0, ctx->stream, src, total,
-                       dst, vec);
-  } else {
-    const i64 K = shape[nd - 1], rows = total / K;
-    hipLaunchKernelGGL((transpose_kernel<float, uint16_t>), dim3(cdiv(K, 32), cdiv(rows, 32)), dim3(256), 0,
-                       ctx->stream, src, rows, K, dst);
-  }
+int convert_bf16(tenrso_ctx* ctx, const float* src, i64 n, uint16_t* dst) {
+  if (n == 0) return TENRSO_OK;
+  const int vec = (uintptr_t)src % 16 == 0 && (uintptr_t)dst % 8 == 0;
+  hipLaunchKernelGGL(f32_to_bf16_kernel, dim3(cdiv(cdiv(n, 4), 256)), dim3(256), 0, ctx->stream, src, n, dst, vec);
   TENRSO_HIP_TRY(hipGetLastError());
   return TENRSO_OK;
 }
@@ -702,7 +688,7 @@ int transpose_last_to_front_f32_padded(tenrso_ctx* ctx, const float* src, int nd
   if (Bp != B)
     hipLaunchKernelGGL(zero_pads_kernel, dim3(cdiv(nrow * (Bp - B), 256)), dim3(256), 0, ctx->stream, dst, nrow, B,
                        Bp);
-  hipLaunchKernelGGL((transpose_kernel<float, float>), dim3(cdiv(K, 32), cdiv(rows, 32)), dim3(256), 0, ctx->stream,
+  hipLaunchKernelGGL(transpose_kernel, dim3(cdiv(K, 32), cdiv(rows, 32)), dim3(256), 0, ctx->stream,
                      src, rows, K, dst, B, Bp);
   TENRSO_HIP_TRY(hipGetLastError());
   return TENRSO_OK;
@@ -713,78 +699,46 @@ int transpose_last_to_front_f32(tenrso_ctx* ctx, const float* src, int nd, const
   for (int k = 0; k < nd; ++k) total *= shape[k];
   if (total == 0) return TENRSO_OK;
   const i64 K = shape[nd - 1], rows = total / K;
-  hipLaunchKernelGGL((transpose_kernel<float, float>), dim3(cdiv(K, 32), cdiv(rows, 32)), dim3(256), 0, ctx->stream,
+  hipLaunchKernelGGL(transpose_kernel, dim3(cdiv(K, 32), cdiv(rows, 32)), dim3(256), 0, ctx->stream,
                      src, rows, K, dst);
   TENRSO_HIP_TRY(hipGetLastError());
   return TENRSO_OK;
 }
 
-// One pass over an fp32 tensor viewed as [rows, K] (K = last mode) for the BF16
-// ALS: the bf16 copy (same layout), the last-to-front fp32 copy ([K, rows]; the
-// last mode's MTTKRP contracts the exact tensor, see mttkrp_bf16_mfma) and
-// per-workgroup (sum of squares, min) partials, instead of three passes.  64 x 64
-// tiles, grid-stride over tiles; each thread loads 4 x 16 bytes (K % 4 == 0, X
-// 16-byte aligned), writes its bf16 quads straight out and through an LDS tile
-// the transposed fp32 quads.  The bf16 values are f32_to_bf16_rne, as in the
-// separate conversion kernel.
-__global__ __launch_bounds__(256) void prepare_bf16_kernel(const float* __restrict__ X, i64 rows, i64 K,
-                                                           uint16_t* __restrict__ dst, float* __restrict__ dstT,
-                                                           double* __restrict__ part) {
-  __shared__ float tile[64][64 + 1];
+// bf16 copy of an fp32 tensor (RNE, as f32_to_bf16_kernel) and per-workgroup (sum of
+// squares, min) partials in one pass: 16-byte loads, grid-stride.
+__global__ __launch_bounds__(256) void convert_bf16_norm_kernel(const float* __restrict__ X, i64 n4,
+                                                                uint16_t* __restrict__ dst,
+                                                                double* __restrict__ part) {
   __shared__ double red[256];
   const int tid = threadIdx.x;
-  const i64 tr_n = (rows + 63) / 64, tk_n = (K + 63) / 64;
+  const floatx4* X4 = reinterpret_cast<const floatx4*>(X);
+  ushort4* d4 = reinterpret_cast<ushort4*>(dst);
+  const i64 stride = (i64)gridDim.x * 256;
   double ss = 0.0;
   float mn = FLT_MAX;
-  for (i64 t = blockIdx.x; t < tr_n * tk_n; t += gridDim.x) {
-    const i64 r0 = (t / tk_n) * 64, k0 = (t % tk_n) * 64;
-    // load + direct copy: thread -> (row tid / 16 + 16 j, columns 4 (tid % 16) ..)
-    const int c4 = 4 * (tid & 15);
+  auto one = [&](i64 i, const floatx4& v) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int rr = (tid >> 4) + 16 * j;
-      const i64 r = r0 + rr, k = k0 + c4;
-      floatx4 v = {0.f, 0.f, 0.f, 0.f};
-      if (r < rows && k < K) {
-        v = *reinterpret_cast<const floatx4*>(X + r * K + k);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          ss = fma((double)v[q], (double)v[q], ss);
-          mn = fminf(mn, v[q]);
-        }
-        if (dst) {  // null: the transposed copy and the norm only
-          ushort4 o;
-          o.x = f32_to_bf16_rne(v[0]);
-          o.y = f32_to_bf16_rne(v[1]);
-          o.z = f32_to_bf16_rne(v[2]);
-          o.w = f32_to_bf16_rne(v[3]);
-          *reinterpret_cast<ushort4*>(dst + r * K + k) = o;
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) tile[rr][c4 + q] = v[q];
+    for (int q = 0; q < 4; ++q) {
+      ss = fma((double)v[q], (double)v[q], ss);
+      mn = fminf(mn, v[q]);
     }
-    __syncthreads();
-    // transposed quads: thread -> (column kk = tid / 16 + 16 j, rows 4 (tid % 16) ..)
+    ushort4 o;
+    o.x = f32_to_bf16_rne(v[0]);
+    o.y = f32_to_bf16_rne(v[1]);
+    o.z = f32_to_bf16_rne(v[2]);
+    o.w = f32_to_bf16_rne(v[3]);
+    d4[i] = o;
+  };
+  i64 i = (i64)blockIdx.x * 256 + tid;
+  for (; i + 3 * stride < n4; i += 4 * stride) {
+    floatx4 v[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int kk = (tid >> 4) + 16 * j, r4 = 4 * (tid & 15);
-      const i64 k = k0 + kk, r = r0 + r4;
-      if (k < K && r < rows) {
-        const floatx4 o = {tile[r4][kk], tile[r4 + 1][kk], tile[r4 + 2][kk], tile[r4 + 3][kk]};
-        float* d = dstT + k * rows + r;
-        if (r + 3 < rows && rows % 4 == 0) {
-          *reinterpret_cast<floatx4*>(d) = o;
-        } else {
-          d[0] = o[0];
-          if (r + 1 < rows) d[1] = o[1];
-          if (r + 2 < rows) d[2] = o[2];
-          if (r + 3 < rows) d[3] = o[3];
-        }
-      }
-    }
-    __syncthreads();  // tile reused by the next tile of this workgroup
+    for (int u = 0; u < 4; ++u) v[u] = X4[i + u * stride];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) one(i + u * stride, v[u]);
   }
+  for (; i < n4; i += stride) one(i, X4[i]);
   // (sum, min) partial of the workgroup
   double v = ss;
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
@@ -804,16 +758,11 @@ __global__ __launch_bounds__(256) void prepare_bf16_kernel(const float* __restri
   }
 }
 
-int prepare_bf16_als(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, uint16_t* dst, float* dstT,
-                     double* tmp, int* nblk_out) {
-  i64 total = 1;
-  for (int k = 0; k < nd; ++k) total *= shape[k];
-  const i64 K = nd >= 1 ? shape[nd - 1] : 1, rows = K ? total / K : 0;
+int convert_bf16_norm(tenrso_ctx* ctx, const float* X, i64 total, uint16_t* dst, double* tmp, int* nblk_out) {
   *nblk_out = 0;
-  if (total == 0 || nd < 2 || K % 4 != 0 || (uintptr_t)X % 16 != 0) return TENRSO_ERR_UNSUPPORTED;
-  const i64 tiles = cdiv(rows, 64) * cdiv(K, 64);
-  const int nblk = (int)std::min<i64>(1024, tiles);
-  hipLaunchKernelGGL(prepare_bf16_kernel, dim3(nblk), dim3(256), 0, ctx->stream, X, rows, K, dst, dstT, tmp);
+  if (total == 0 || total % 4 != 0 || (uintptr_t)X % 16 != 0) return TENRSO_ERR_UNSUPPORTED;
+  const int nblk = (int)std::min<i64>(1024, cdiv(total / 4, 256 * 4));
+  hipLaunchKernelGGL(convert_bf16_norm_kernel, dim3(nblk), dim3(256), 0, ctx->stream, X, total / 4, dst, tmp);
   TENRSO_HIP_TRY(hipGetLastError());
   *nblk_out = nblk;
   return TENRSO_OK;
@@ -1085,6 +1034,10 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
         ssp = s;
       }
     }
+    // With the job fused a launch of few blocks lasts as long as the job, and fewer
+    // splits leave the row solve less to add: one round, and a slow index a wave
+    // (224x96x128 rank 5: solve 4.5 us behind 12 splits, 5.1 behind 36).
+    if (fuse_job) ssp = std::max<i64>(1, std::min<i64>(target / wgs1, a.n_slow / waves));
     // Several rounds and no job: 4-wave workgroups, as many splits as bring 1.5
     // times the resident ones while a wave keeps four blocks (9216 rows, 9216 j,
     // rank 32: 75 us with 576 workgroups, 70 with 1152, 69 with 1728).
