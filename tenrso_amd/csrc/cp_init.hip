@@ -35,7 +35,7 @@
 namespace tenrso {
 
 constexpr int INIT_RMAX = 128;  // rank bound of the SVD-based initialisations (that of the ALS)
-constexpr int JACOBI_SWEEPS = 16;
+constexpr int JACOBI_SWEEPS = 18;
 
 namespace {
 
@@ -178,6 +178,36 @@ __device__ __forceinline__ void circle_pair(int count, int r, int k, int& a, int
   b = k == 0 ? count - 1 : (r - k + (count - 1)) % (count - 1);
 }
 
+// 1 / sqrt(x), two Newton steps
+__device__ __forceinline__ double rsqrt_newton(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+  return y;
+}
+
+// The Jacobi rotation (c, s) of a = a_qq - a_pp and b = 2 a_pq != 0:
+// t = b / (a + sign(a) sqrt(a^2 + b^2)), c = 1 / sqrt(1 + t^2), s = t c.  By
+// approximate reciprocals refined to full precision, a third of the chain of two
+// divisions and two square roots; those where a^2 + b^2 leaves the exponent range.
+__device__ __forceinline__ void rotation(double a, double b, double& c, double& s) {
+  const double h2 = fma(a, a, b * b);
+  double t;
+  if (h2 > 0x1p-900 && h2 < 0x1p900) {
+    const double den = fma(h2, rsqrt_newton(h2), fabs(a));
+    double r = __builtin_amdgcn_rcp(den);
+    r = fma(r, fma(-den, r, 1.0), r);
+    r = fma(r, fma(-den, r, 1.0), r);
+    t = (a >= 0.0 ? b : -b) * r;
+    c = rsqrt_newton(fma(t, t, 1.0));
+  } else {
+    const double th = a / b;
+    t = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(fma(th, th, 1.0)));
+    c = 1.0 / sqrt(fma(t, t, 1.0));
+  }
+  s = t * c;
+}
+
 template <int THREADS>
 __device__ __forceinline__ double block_sum(double v, double* red) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
@@ -197,22 +227,31 @@ __global__ __launch_bounds__(1024) void jacobi_check_kernel(EigArgs a) {
   if (*m.done) return;
   const i64 N = m.N;
   double off = 0.0, dia = 0.0;
-  for (i64 i = threadIdx.x >> 6; i < N; i += 16)
+  // four rows in flight (N is a multiple of 64)
+  for (i64 i = threadIdx.x >> 6; i < N; i += 64)
     for (i64 j = threadIdx.x & 63; j < N; j += 64) {
-      const double v = m.A[i * N + j];
-      if (i == j) dia += v * v;
-      else off += v * v;
+      double v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = m.A[(i + 16 * u) * N + j];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (i + 16 * u == j) dia += v[u] * v[u];
+        else off += v[u] * v[u];
+      }
     }
   off = block_sum<1024>(off, red);
   dia = block_sum<1024>(dia, red);
   if (threadIdx.x == 0 && (off <= 1e-28 * dia || off == 0.0)) *m.done = 1;
 }
 
-// The rotation of one pair of blocks of round r: cyclic parallel Jacobi on their
-// 64 x 64 submatrix in LDS (63 rounds of 32 disjoint rotations, rows and columns of
-// each 2 x 2 block by one thread), accumulated into Q.  One sweep where the matrix
-// has other blocks, which the next round brings; up to `inner` where it is the whole
-// matrix.
+// The rotation of one pair of blocks of round r, accumulated into Q: Jacobi on their
+// 64 x 64 submatrix in LDS, 32 disjoint rotations at a time, rows and columns of each
+// 2 x 2 block by one thread.  A sweep's first round takes all pairs of the submatrix
+// (63 steps), the others only those across the two blocks (32 steps): a sweep then
+// takes every pair of the matrix once.  (All pairs in every round: one sweep less of
+// 12 at 256 rows, but 441 steps a sweep instead of 255.)  Where the two blocks are the
+// whole matrix, up to 30 sweeps at once.  A step is bound by LDS (131 KB of S and W)
+// and the chain of the 32 rotations.
 constexpr int JB = 32;            // block width
 constexpr int JP = 2 * JB;        // order of a pair
 constexpr int JPITCH = JP + 1;    // doubles
@@ -233,6 +272,15 @@ __global__ __launch_bounds__(1024) void jacobi_pair_kernel(EigArgs a, int r) {
   }
   __syncthreads();
   const int inner = blocks == 2 ? 30 : 1;
+  const bool all = r == 0;  // (two blocks have no other round)
+  auto pair_of = [&](int rr, int k, int& i, int& j) {
+    if (all) {
+      circle_pair(JP, rr, k, i, j);
+    } else {
+      i = k;
+      j = JB + ((k + rr) & (JB - 1));
+    }
+  };
   for (int sweep = 0; sweep < inner; ++sweep) {
     if (sweep > 0) {
       double off = 0.0, dia = 0.0;
@@ -245,18 +293,13 @@ __global__ __launch_bounds__(1024) void jacobi_pair_kernel(EigArgs a, int r) {
       dia = block_sum<1024>(dia, red);
       if (off <= 1e-28 * dia || off == 0.0) break;
     }
-    for (int rr = 0; rr < JP - 1; ++rr) {
+    for (int rr = 0; rr < (all ? JP - 1 : JB); ++rr) {
       if (tid < JB) {
         int i, j;
-        circle_pair(JP, rr, tid, i, j);
+        pair_of(rr, tid, i, j);
         const double apq = S[i * JPITCH + j];
         double c = 1.0, s = 0.0;
-        if (apq != 0.0) {
-          const double th = (S[j * JPITCH + j] - S[i * JPITCH + i]) / (2.0 * apq);
-          const double t = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(fma(th, th, 1.0)));
-          c = 1.0 / sqrt(fma(t, t, 1.0));
-          s = t * c;
-        }
+        if (apq != 0.0) rotation(S[j * JPITCH + j] - S[i * JPITCH + i], 2.0 * apq, c, s);
         cs[2 * tid] = c;
         cs[2 * tid + 1] = s;
       }
@@ -264,8 +307,8 @@ __global__ __launch_bounds__(1024) void jacobi_pair_kernel(EigArgs a, int r) {
       {
         const int ki = tid >> 5, kj = tid & 31;
         int i0, i1, j0, j1;
-        circle_pair(JP, rr, ki, i0, i1);
-        circle_pair(JP, rr, kj, j0, j1);
+        pair_of(rr, ki, i0, i1);
+        pair_of(rr, kj, j0, j1);
         const double ci = cs[2 * ki], si = cs[2 * ki + 1], cj = cs[2 * kj], sj = cs[2 * kj + 1];
         const double x00 = S[i0 * JPITCH + j0], x01 = S[i0 * JPITCH + j1], x10 = S[i1 * JPITCH + j0],
                      x11 = S[i1 * JPITCH + j1];
@@ -296,7 +339,7 @@ __global__ __launch_bounds__(1024) void jacobi_pair_kernel(EigArgs a, int r) {
 // a column pair (T Q_J); tiles are disjoint, so in place.  8 waves, each 16 rows x 32
 // columns of the tile, FP64 matrix cores.
 __global__ __launch_bounds__(512) void jacobi_update_kernel(EigArgs a, int r) {
-  __shared__ double sT[JP * JPITCH], sQ[JP * JPITCH];
+  __shared__ double sT[JP * JPITCH], sQ[JP * JPITCH], sP[JP * JPITCH];
   const EigMode& m = a.m[blockIdx.y];
   const int blocks = m.N / JB, pairs = blocks / 2;
   if ((int)blockIdx.x >= 2 * pairs * pairs || r >= blocks - 1 || *m.done) return;
@@ -318,6 +361,7 @@ __global__ __launch_bounds__(512) void jacobi_update_kernel(EigArgs a, int r) {
     const int i = e / JP, j = e % JP;
     sT[i * JPITCH + j] = M[grow(i) * N + gcol(j)];
     sQ[i * JPITCH + j] = m.Q[(i64)pj * JP * JP + e];
+    if (!isV) sP[i * JPITCH + j] = m.Q[(i64)pi * JP * JP + e];
   }
   __syncthreads();
   const int r0 = 16 * (wave >> 1), c0 = 32 * (wave & 1);
@@ -335,13 +379,12 @@ __global__ __launch_bounds__(512) void jacobi_update_kernel(EigArgs a, int r) {
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int e = 0; e < 4; ++e) sT[(r0 + 4 * e + q4) * JPITCH + c0 + 16 * u + l16] = acc[u][e];
-    for (int e = tid; e < JP * JP; e += 512) sQ[(e / JP) * JPITCH + e % JP] = m.Q[(i64)pi * JP * JP + e];
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < 2; ++u) acc[u] = doublex4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll 4
     for (int kk = 0; kk < JP / 4; ++kk) {
-      const double av = sQ[(4 * kk + q4) * JPITCH + r0 + l16];  // Q_I^T
+      const double av = sP[(4 * kk + q4) * JPITCH + r0 + l16];  // Q_I^T
 #pragma unroll
       for (int u = 0; u < 2; ++u)
         acc[u] =
