@@ -40,14 +40,15 @@ struct MttkrpScratch {
 // and of X_t when those copies have it padded with zeros.
 // want_norm: also leave FP64 partial sums of ||X||^2 in res->norm (FP32 calls whose
 // ranks fit one launch of the MFMA kernel; null otherwise).
-// slot: the context buffer of the split partials.
+// slot: the context buffer of the split partials.  plan: only fill it, launch nothing
+// (from four modes on with pre_rows).
 // pre_rows (optional, tensors of order >= 4): the PRE Khatri-Rao rows of this
 // mode already formed (mttkrp_pre_batch), instead of a launch that forms them.
 int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int nd, const i64* shape,
                  const float* const* F, i64 R, int mode, MttkrpOut outk, void* out, MttkrpResult* res,
                  const AlsJob* job = nullptr, const MttkrpScratch* scratch = nullptr,
                  i64 x_pad = 0, i64 xt_pad = 0, const float* pre_rows = nullptr, bool want_norm = false,
-                 int slot = SLOT_PARTIAL);
+                 int slot = SLOT_PARTIAL, struct X3Plan* plan = nullptr);
 
 // The fp32 MTTKRPs of every mode of one tensor that has elements.
 int mttkrp_all_modes(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, const float* const* F, i64 R,

@@ -823,10 +823,42 @@ Plan make_plan(int nd, const i64* shape, int mode) {
 
 }  // namespace
 
+// How a mode runs in the fp32 MFMA kernel (ok: it can, in one launch of up to 64 rank
+// columns); its splits are still to be chosen.
+struct X3Plan {
+  bool ok = false, case_b = false;
+  int nt = 0, xl = 0;
+  KernArgs a;
+};
+
+// resident workgroups of a kernel on one CU (occupancy query, cached)
+static int occupancy(tenrso_ctx* ctx, const void* kern, int threads, int* occ) {
+  for (int i = 0; i < ctx->occ_n; ++i)
+    if (ctx->occ_kern[i] == kern) {
+      *occ = ctx->occ_val[i];
+      return TENRSO_OK;
+    }
+  int nb = 0;
+  TENRSO_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, threads, 0));
+  *occ = std::max(1, nb);
+  if (ctx->occ_n < 64) {
+    ctx->occ_kern[ctx->occ_n] = kern;
+    ctx->occ_val[ctx->occ_n++] = *occ;
+  }
+  return TENRSO_OK;
+}
+
+// a.slow_splits splits of the slow range, balanced
+static void set_splits(KernArgs& a, i64 ssp) {
+  a.slow_splits = (int)std::max<i64>(1, ssp);
+  a.slow_q = a.n_slow / a.slow_splits;
+  a.slow_rem = a.n_slow % a.slow_splits;
+}
+
 int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int nd, const i64* shape,
                  const float* const* F, i64 R, int mode, MttkrpOut outk, void* out, MttkrpResult* res,
                  const AlsJob* job, const MttkrpScratch* scratch, i64 x_pad, i64 xt_pad,
-                 const float* pre_rows, bool want_norm, int slot) {
+                 const float* pre_rows, bool want_norm, int slot, X3Plan* plan) {
   Plan pl = make_plan(nd, shape, mode);
   const bool bf16 = prec == TENRSO_PREC_BF16;
   const float* Fv[MAXD];
@@ -982,22 +1014,15 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
     a.total = caseB ? pl.J * I : pl.J / Qcon * I * Qmem;
     a.rtiles = (int)rtiles;
     a.win_vec = (R % 4 == 0) && ((uintptr_t)fastf % 16 == 0);
-    // resident workgroups of a kernel on one CU (occupancy query, cached)
-    auto occupancy = [&](const void* kern, int threads, int* occ) -> int {
-      for (int i = 0; i < ctx->occ_n; ++i)
-        if (ctx->occ_kern[i] == kern) {
-          *occ = ctx->occ_val[i];
-          return TENRSO_OK;
-        }
-      int nb = 0;
-      TENRSO_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, threads, 0));
-      *occ = std::max(1, nb);
-      if (ctx->occ_n < 64) {
-        ctx->occ_kern[ctx->occ_n] = kern;
-        ctx->occ_val[ctx->occ_n++] = *occ;
-      }
+    if (plan) {
+      plan->ok = fp32 && NT < 8 && rchunks == 1;
+      plan->a = a;
+      plan->a.rcount = (int)R;
+      plan->case_b = caseB;
+      plan->nt = NT;
+      plan->xl = XL;
       return TENRSO_OK;
-    };
+    }
     // 8-wave workgroups, one per CU (the register budget admits one), so a fused
     // ALS job gets a CU of its own instead of sharing one with an MTTKRP workgroup
     // (measured: the job at ~22 us beside the MTTKRP against ~14 us alone).  When
@@ -1007,7 +1032,7 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
     const void* kern = !fp32 ? mttkrp_bf16_kernel(NT, caseB, a.win_vec, KB / 32, XL)
                              : (NT == 8 ? mttkrp_x3_kernel_n8(caseB, a.win_vec, XL)
                                         : mttkrp_x3_kernel_w8(NT, caseB, a.win_vec, XL));
-    TENRSO_TRY(occupancy(kern, waves * 64, &occ));
+    TENRSO_TRY(occupancy(ctx, kern, waves * 64, &occ));
     int wpc = bf16 ? ctx->wg_per_cu_bf16 : ctx->wg_per_cu_f32;  // TENRSO_WG_PER_CU_* override
     if (wpc <= 0) wpc = std::min(occ, 2);
     const bool fuse_job = job != nullptr && rchunks == 1 && (job->R <= JOB_NE || NT == 8) && (fp32 || !caseB);
@@ -1045,7 +1070,7 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
     if (fp32 && NT < 8 && !fuse_job && (wgs1 * ssp > target || with_norm)) {
       kern = with_norm ? mttkrp_x3_kernel_norm(NT, caseB, a.win_vec, XL) : mttkrp_x3_kernel_w4(NT, caseB, a.win_vec, XL);
       waves = 4;
-      TENRSO_TRY(occupancy(kern, waves * 64, &occ));
+      TENRSO_TRY(occupancy(ctx, kern, waves * 64, &occ));
       target = (i64)(ctx->wg_per_cu_f32 > 0 ? ctx->wg_per_cu_f32 : occ) * ctx->num_cus;
       ssp = std::min<i64>((3 * target / 2 + wgs1 - 1) / wgs1, a.n_slow * nkb / (4 * waves));
       ssp = std::max<i64>(1, std::min<i64>(ssp, a.n_slow));
@@ -1054,9 +1079,7 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
     // a caller's workspace bounds the partials: fewer splits, or refuse
     if (max_splits() < a.nwin) return too_small(a.nwin);
     ssp = std::min<i64>(ssp, max_splits() / a.nwin);
-    a.slow_splits = (int)std::max<i64>(1, ssp);
-    a.slow_q = a.n_slow / a.slow_splits;
-    a.slow_rem = a.n_slow % a.slow_splits;
+    set_splits(a, ssp);
     splits = a.nwin * a.slow_splits;
     TENRSO_TRY(partial_buffer(splits, &partial));
     if (with_norm) {
@@ -1111,6 +1134,7 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
       TENRSO_TRY(launch_main(true));
     }
   } else {
+    if (plan) return TENRSO_OK;
     if (pad > 0 && fast_stride != pl.fast_size) {
       set_error("internal: a padded tensor copy reached the generic MTTKRP");
       return TENRSO_ERR_UNSUPPORTED;
@@ -1154,10 +1178,12 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
   return TENRSO_OK;
 }
 
-// One reduction (and, from four modes on, one launch for the Khatri-Rao rows) for all
-// the modes.  Small tensors are bound by the host and the gaps between launches: all
-// modes of 64^3 rank 8 take 22 us so, against 49 us as three calls of two launches; at
-// 256^3 rank 64 58.4 us against 61.5, at 96^4 rank 32 248 us against 260.
+// All modes in one launch of the fp32 MFMA kernel and one reduction (from four modes on
+// one launch for the Khatri-Rao rows before); where a mode cannot run so (rank above
+// 64, a last mode of one row), a launch a mode and one reduction.  Small tensors are
+// bound by the host and the gaps between launches.  All modes of 64^3 rank 8: 49 us as
+// three calls of two launches, 22 with a launch a mode, 15 so; 256^3 rank 64: 61.5,
+// 58.4 and 44 us (250^3: 73.5, 70.7, 51; 96^4 rank 32: 260, 248, 202).
 int mttkrp_all_modes(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, const float* const* F, i64 R,
                      float* const* outs) {
   static_assert(SLOT_PARTIAL_MODE_END - SLOT_PARTIAL_MODE + 1 == MAXD, "a buffer of partials per mode");
@@ -1170,19 +1196,60 @@ int mttkrp_all_modes(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, 
     rows += total / (shape[m] * shape[m == nd - 1 ? nd - 2 : nd - 1]) * R;
   }
   // (rows far larger than X, as many small modes have, are formed a mode at a time)
-  if (nd >= 4 && rows <= 2 * total) TENRSO_TRY(mttkrp_pre_batch(ctx, nd, shape, F, R, nd, modes, false, pre));
+  const bool batch = nd >= 4 && rows <= 2 * total;
+  if (batch) TENRSO_TRY(mttkrp_pre_batch(ctx, nd, shape, F, R, nd, modes, false, pre));
   ReduceMany r{};
-  for (int m = 0; m < nd; ++m) {
-    MttkrpResult res;
-    TENRSO_TRY(mttkrp_dense(ctx, TENRSO_PREC_FP32, X, nullptr, nd, shape, F, R, m, MttkrpOut::PARTIAL, nullptr, &res,
-                            nullptr, nullptr, 0, 0, pre[m], false, SLOT_PARTIAL_MODE + m));
-    const i64 n = shape[m] * R;
-    r.part[r.count] = res.partial;
-    r.splits[r.count] = res.splits;
-    r.n[r.count] = n;
-    r.out[r.count] = outs[m];
-    r.first[r.count + 1] = r.first[r.count] + cdiv(n, 64);
-    ++r.count;
+  auto add = [&](int m, const float* partial, int splits) {
+    r.part[m] = partial;
+    r.splits[m] = splits;
+    r.n[m] = shape[m] * R;
+    r.out[m] = outs[m];
+    r.first[m + 1] = r.first[m] + cdiv(shape[m] * R, 64);
+    r.count = m + 1;
+  };
+  X3Plan plan[MAXD];
+  bool one = nd < 4 || batch, wv = true;
+  for (int m = 0; one && m < nd; ++m) {
+    one = nd < 4 || pre[m] != nullptr;
+    if (!one) break;
+    TENRSO_TRY(mttkrp_dense(ctx, TENRSO_PREC_FP32, X, nullptr, nd, shape, F, R, m, MttkrpOut::PARTIAL, nullptr, nullptr,
+                            nullptr, nullptr, 0, 0, pre[m], false, SLOT_PARTIAL, &plan[m]));
+    one = plan[m].ok && plan[m].case_b == (m == nd - 1) && plan[m].xl == plan[m < nd - 1 ? 0 : m].xl;
+    wv = wv && plan[m].a.win_vec;
+  }
+  if (one) {
+    const void* kern = mttkrp_x3_kernel_all(plan[0].nt, wv, plan[0].xl, plan[nd - 1].xl);
+    int occ = 0;
+    TENRSO_TRY(occupancy(ctx, kern, 256, &occ));
+    // Splits: the resident workgroups of one round shared between the modes, at least a
+    // block a wave (256^3 rank 64: 43.9 us in one round, 48.7 in two, 54.6 in three,
+    // 61.4 in one with a few workgroups over).
+    const i64 target = (i64)(ctx->wg_per_cu_f32 > 0 ? ctx->wg_per_cu_f32 : occ) * ctx->num_cus;
+    AllModesArgs p{};
+    p.nd = nd;
+    for (int m = 0; m < nd; ++m) {
+      KernArgs& a = plan[m].a;
+      const i64 wgs1 = (i64)a.rtiles * a.nwin, nkb = (a.kw + 31) / 32;
+      i64 ssp = std::min<i64>(target / (nd * wgs1), a.n_slow * nkb / 4);
+      ssp = std::max<i64>(1, std::min<i64>(std::min<i64>(ssp, a.n_slow), 65535 / a.nwin));
+      set_splits(a, ssp);
+      const int splits = a.nwin * a.slow_splits;
+      void* pp = nullptr;
+      TENRSO_TRY(ctx_buffer(ctx, SLOT_PARTIAL_MODE + m, (size_t)splits * shape[m] * R * sizeof(float), &pp));
+      p.a[m] = a;
+      p.partial[m] = (float*)pp;
+      p.first[m + 1] = p.first[m] + (unsigned)(a.rtiles * splits);
+      add(m, p.partial[m], splits);
+    }
+    void* args[] = {(void*)&X, &p};
+    TENRSO_HIP_TRY(hipLaunchKernel(kern, dim3(p.first[nd]), dim3(256), args, 0, ctx->stream));
+  } else {
+    for (int m = 0; m < nd; ++m) {
+      MttkrpResult res;
+      TENRSO_TRY(mttkrp_dense(ctx, TENRSO_PREC_FP32, X, nullptr, nd, shape, F, R, m, MttkrpOut::PARTIAL, nullptr, &res,
+                              nullptr, nullptr, 0, 0, pre[m], false, SLOT_PARTIAL_MODE + m));
+      add(m, res.partial, res.splits);
+    }
   }
   hipLaunchKernelGGL(reduce_many_kernel, dim3(r.first[r.count]), dim3(64 * RED_GROUPS), 0, ctx->stream, r);
   TENRSO_HIP_TRY(hipGetLastError());

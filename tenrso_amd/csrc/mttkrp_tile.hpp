@@ -39,6 +39,15 @@ struct KernArgs {
   int win_vec;        // FAST 16-byte aligned and R % 4 == 0: 16-byte window loads
 };
 
+// The MTTKRPs of all modes of a tensor in one launch: mode m takes the workgroups
+// [first[m], first[m + 1]); the last mode is case B.
+struct AllModesArgs {
+  int nd;
+  unsigned first[MAXD + 1];
+  float* partial[MAXD];
+  KernArgs a[MAXD];
+};
+
 __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
   uint32_t u = __float_as_uint(f);
   if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);  // quiet NaN

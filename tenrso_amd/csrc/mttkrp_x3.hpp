@@ -15,4 +15,8 @@ const void* mttkrp_x3_kernel_norm(int nt, bool case_b, bool wv, int xl);
 // Eight rank tiles, 8 waves, able to run the wide-rank job.
 const void* mttkrp_x3_kernel_n8(bool case_b, bool wv, int xl);
 
+// All modes in one launch (AllModesArgs); xla: the load form of modes 0 .. nd-2, xlb:
+// of the last.  4 waves a workgroup.
+const void* mttkrp_x3_kernel_all(int nt, bool wv, int xla, int xlb);
+
 }  // namespace tenrso

@@ -81,33 +81,22 @@ __device__ __forceinline__ void x3_split(const floatx8& x, bf16x8& h, bf16x8& l,
 // NORM: the sum of squares of X as well (FP64; every element of X is read by exactly
 // one lane), a partial per wave in a.norm.  In the memory-bound loop it is nearly
 // free, where a pass of its own over X takes as long as the MTTKRP.
-template <int NT, int WAVES, int JOB, bool CASE_B, bool WV, int XL, bool NORM>
-__global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __restrict__ X, KernArgs a,
-                                                                float* __restrict__ partial, AlsJob job,
-                                                                int has_job) {
+// ALL: 4 waves, and the workgroups of every mode of the tensor in one launch.
+
+// LDS bytes of the window planes and the reduction
+template <int NT, int WAVES>
+constexpr int x3_lds() {
+  constexpr int win = 3 * 16 * NT * (X3_KWMAX + 8) * 2, red = 2 * NT * WAVES * 64 * 16;
+  return win > red ? win : red;
+}
+
+// One workgroup's tile.  smem: x3_lds bytes; colmax: largest magnitude of each window
+// column, by staging wave; plain: a wave asks for the plain form.
+template <int NT, int WAVES, bool CASE_B, bool WV, int XL, bool NORM>
+__device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernArgs& a, float* __restrict__ partial,
+                                        int tile, float* smem, float (*colmax)[16 * NT], int& plain) {
   constexpr int MT = 2, NBUF = X3_NBUF<NT>, KWMAX = X3_KWMAX;
   constexpr int KB = 32, PITCH = KWMAX + 8, RT = 16 * NT, NTH = WAVES * 64, ROWS = 16 * MT;
-  constexpr int LDS_WIN = 3 * RT * PITCH * 2, LDS_RED = MT * NT * WAVES * 64 * 16;
-  constexpr int LDS_B = LDS_WIN > LDS_RED ? LDS_WIN : LDS_RED;
-  constexpr int LDS_JOB = JOB == 0 ? 0 : (JOB == 1 ? JOB_LDS_BYTES : WIDE_LDS_BYTES);
-  constexpr int LDS_BYTES = LDS_B > LDS_JOB ? LDS_B : LDS_JOB;
-  __shared__ __attribute__((aligned(16))) float smem[LDS_BYTES / 4];
-  __shared__ float colmax[WAVES][RT];  // largest magnitude of each window column, by staging wave
-  __shared__ int plain;                // a wave asks for the plain form
-  if (JOB != 0 && has_job && blockIdx.x == 0) {
-    // one such workgroup a CU, so the job has its CU to itself; waves past the
-    // rank-64 job's four end at once
-    double* lds = reinterpret_cast<double*>(smem);
-    if constexpr (JOB == 1) {
-      static_assert(NTH % JOB_THREADS == 0, "the ALS job runs on the first 256 threads");
-      if (threadIdx.x < JOB_THREADS) als_job_run(job, lds);
-    } else if constexpr (JOB == 2) {
-      static_assert(NTH == WIDE_THREADS, "the wide-rank job runs on the whole workgroup");
-      als_job_wide_run(job, lds);
-    }
-    return;
-  }
-  const int tile = (int)blockIdx.x - (JOB != 0 && has_job ? 1 : 0);
   const int xt = tile % a.rtiles;
   uint16_t* sHi = reinterpret_cast<uint16_t*>(smem);
   uint16_t* sLo = sHi + RT * PITCH;
@@ -349,6 +338,32 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
     return;
   }
   wg_reduce_store<MT, NT, WAVES, false>(acc, smem, wave, lane, out, a.I, a.R, a.r0, a.rcount, row_base, CASE_B);
+}
+
+template <int NT, int WAVES, int JOB, bool CASE_B, bool WV, int XL, bool NORM>
+__global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __restrict__ X, KernArgs a,
+                                                             float* __restrict__ partial, AlsJob job, int has_job) {
+  constexpr int LDS_B = x3_lds<NT, WAVES>();
+  constexpr int LDS_JOB = JOB == 0 ? 0 : (JOB == 1 ? JOB_LDS_BYTES : WIDE_LDS_BYTES);
+  constexpr int LDS_BYTES = LDS_B > LDS_JOB ? LDS_B : LDS_JOB;
+  __shared__ __attribute__((aligned(16))) float smem[LDS_BYTES / 4];
+  __shared__ float colmax[WAVES][16 * NT];
+  __shared__ int plain;
+  if (JOB != 0 && has_job && blockIdx.x == 0) {
+    // one such workgroup a CU, so the job has its CU to itself; waves past the
+    // rank-64 job's four end at once
+    double* lds = reinterpret_cast<double*>(smem);
+    if constexpr (JOB == 1) {
+      static_assert((WAVES * 64) % JOB_THREADS == 0, "the ALS job runs on the first 256 threads");
+      if (threadIdx.x < JOB_THREADS) als_job_run(job, lds);
+    } else if constexpr (JOB == 2) {
+      static_assert(WAVES * 64 == WIDE_THREADS, "the wide-rank job runs on the whole workgroup");
+      als_job_wide_run(job, lds);
+    }
+    return;
+  }
+  x3_tile<NT, WAVES, CASE_B, WV, XL, NORM>(X, a, partial, (int)blockIdx.x - (JOB != 0 && has_job ? 1 : 0), smem,
+                                           colmax, plain);
 }
 
 template <int NT, int WAVES, int JOB, bool CASE_B, bool WV, bool NORM>
