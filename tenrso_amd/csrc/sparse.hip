@@ -15,7 +15,7 @@
 //   semantics: fptr[l][f] indexes level l+1, unlike csf.rs:209,246).
 //
 // MTTKRP kernel: a worker of LPN lanes (one lane per rank column) owns a
-// contiguous chunk of SP_CH sorted nonzeros and accumulates row by row in
+// contiguous chunk of sorted nonzeros and accumulates row by row in
 // registers.  Rows strictly inside the chunk belong to the worker alone and are
 // stored directly; the chunk's first and last rows may be shared with
 // neighbouring chunks and go to two carry slots.  The carry slots (sorted by
@@ -148,6 +148,16 @@ __global__ __launch_bounds__(256) void chunk_fib_kernel(const int32_t* __restric
   cf[c] = pos[e] + flag[e] - 1;
 }
 
+// Nonzeros per worker: `most`, halved down to 32 while that leaves fewer than 32 workers
+// a CU.  A worker takes its nonzeros one batch of gathers after another, so few workers
+// with long runs wait for memory: 200000 nonzeros at rank 16 took 54 us a mode in runs
+// of 128; 24436 at rank 25 579 us in runs of 1024.
+static int sp_run(const tenrso_ctx* ctx, i64 nnz, int most) {
+  int run = most;
+  while (run > 32 && nnz / run < 32 * (i64)ctx->num_cus) run /= 2;
+  return run;
+}
+
 // Device temporaries of one build step, freed on every path out of it.
 struct DevTemps {
   std::vector<void*> ptrs;
@@ -186,14 +196,15 @@ static int sp_build_fibres(tenrso_ctx* ctx, tenrso_sptensor* t, int mode) {
   TENRSO_HIP_TRY(hipMemcpyAsync(&last[1], flag + nnz - 1, 4, hipMemcpyDeviceToHost, ctx->stream));
   TENRSO_HIP_TRY(hipStreamSynchronize(ctx->stream));
   md.nfib = (i64)last[0] + last[1];
-  md.nchunks = (nnz + SP_CSF_W - 1) / SP_CSF_W;
+  md.run = sp_run(ctx, nnz, 128);
+  md.nchunks = (nnz + md.run - 1) / md.run;
   TENRSO_HIP_TRY(hipMalloc(&md.leafe, (size_t)nnz * 4));
   TENRSO_HIP_TRY(hipMalloc(&md.fpre, (size_t)std::max<i64>(1, md.nfib * D) * 4));
   TENRSO_HIP_TRY(hipMalloc(&md.chunk_fib, (size_t)md.nchunks * 4));
   hipLaunchKernelGGL(fib_scatter_kernel, dim3(cdiv(nnz, 256)), dim3(256), 0, ctx->stream, flag, pos, md.row, md.oth,
                      nnz, D, md.nfib, md.leafe, md.fpre);
   hipLaunchKernelGGL(chunk_fib_kernel, dim3(cdiv(md.nchunks, 256)), dim3(256), 0, ctx->stream, flag, pos, md.nchunks,
-                     SP_CSF_W, md.chunk_fib);
+                     md.run, md.chunk_fib);
   TENRSO_HIP_TRY(hipGetLastError());
   // the temporaries are freed below: the kernels reading them must be done
   TENRSO_HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -363,7 +374,7 @@ void sp_destroy(tenrso_sptensor* t) {
 }
 
 // ---------------------------------------------------------------- MTTKRP
-constexpr int SP_CH = 1024;  // nonzeros per worker chunk
+constexpr int SP_CH = 1024;  // most nonzeros per worker of the scalar kernel
 constexpr int SP_U = 4;      // nonzeros in flight per worker step
 
 struct SpArgs {
@@ -375,6 +386,7 @@ struct SpArgs {
   const float* vals;
   const float* F[MAXD_SP];  // factors of the other modes, ascending mode order
   i64 nworkers;
+  int run;                  // nonzeros per worker
 };
 
 template <int LPN>
@@ -386,8 +398,8 @@ __global__ __launch_bounds__(256) void sp_mttkrp_kernel(SpArgs a, float* __restr
   if (w >= a.nworkers) return;
   const bool live = lane < a.rcount;
   const int col = a.r0 + (live ? lane : 0);
-  const i64 e0 = w * SP_CH;
-  const i64 e1 = (e0 + SP_CH) < a.nnz ? e0 + SP_CH : a.nnz;
+  const i64 e0 = w * a.run;
+  const i64 e1 = (e0 + a.run) < a.nnz ? e0 + a.run : a.nnz;
   float* c0 = cval + (2 * w) * a.R;
   float* c1 = cval + (2 * w + 1) * a.R;
   const int first = a.row[e0];
@@ -444,14 +456,14 @@ __global__ __launch_bounds__(256) void sp_mttkrp_kernel(SpArgs a, float* __restr
 
 // Vector form for R % 4 == 0: a worker is G lanes (lane q owns rank columns
 // r0 + 4q .. 4q+3 and gathers factor rows as 16-byte vectors), a wave holds
-// 64 / G workers, and each worker runs SP_W consecutive sorted nonzeros.  The
+// 64 / G workers, and each worker runs consecutive sorted nonzeros (a.run).  The
 // worker's row / value / index runs are staged SP_SUB at a time into
 // wave-private LDS (dynamic, (nd_oth + 2) arrays of SP_SUB words per worker)
 // with vector loads; the nonzeros are then processed SP_VU at a time with
 // every factor gather issued before any is used.  Same carry contract as
 // sp_mttkrp_kernel: the worker's first row goes to carry slot 2w, its last row
 // to slot 2w + 1, rows strictly inside the run are stored to `out` directly.
-constexpr int SP_W = 128;    // nonzeros per vector worker
+constexpr int SP_W = 128;    // most nonzeros per vector worker
 constexpr int SP_SUB = 32;   // nonzeros staged per pass
 constexpr int SP_VU = 4;     // nonzeros in flight per worker (a multiple of 4: staged entries are read as 16-byte vectors)
 
@@ -495,8 +507,8 @@ __global__ __launch_bounds__(256) void sp_mttkrp_vec_kernel(SpArgs a, float* __r
   int32_t* st = sp_stage + ((wave * NPW + g) * na) * SP_SUB;
   const i64 w = ((i64)blockIdx.x * 4 + wave) * NPW + g;
   const bool active = w < a.nworkers;
-  const i64 e0 = w * SP_W;
-  const i64 e1 = active ? ((e0 + SP_W) < a.nnz ? e0 + SP_W : a.nnz) : e0;
+  const i64 e0 = w * a.run;
+  const i64 e1 = active ? ((e0 + a.run) < a.nnz ? e0 + a.run : a.nnz) : e0;
   const bool live = 4 * q < a.rcount;
   const int col = a.r0 + (live ? 4 * q : 0);
   const int first = active ? a.row[e0] : 0;
@@ -605,6 +617,7 @@ struct SpCsfArgs {
   const int32_t* chunk_fib;
   const float* F[MAXD_SP]; // factors of the other modes, ascending mode order
   i64 nworkers;
+  int run;                 // nonzeros per worker
 };
 
 template <int G, int D>
@@ -624,8 +637,8 @@ __global__ __launch_bounds__(256) void sp_mttkrp_csf_kernel(SpCsfArgs a, float* 
   int32_t* sPre = sVal + SP_SUB;  // D x SP_FWIN prefixes (row first)
   const i64 w = ((i64)blockIdx.x * 4 + wave) * NPW + g;
   const bool active = w < a.nworkers;
-  const i64 e0 = w * SP_CSF_W;
-  const i64 e1 = active ? ((e0 + SP_CSF_W) < a.nnz ? e0 + SP_CSF_W : a.nnz) : e0;
+  const i64 e0 = w * a.run;
+  const i64 e1 = active ? ((e0 + a.run) < a.nnz ? e0 + a.run : a.nnz) : e0;
   const bool live = 4 * q < a.rcount;
   const int col = a.r0 + (live ? 4 * q : 0);
   i64 fb = active ? a.chunk_fib[w] : 0;  // fibre of the next nonzero
@@ -901,8 +914,10 @@ int sp_mttkrp(tenrso_ctx* ctx, const tenrso_sptensor* t, const float* const* F, 
     ca.chunk_fib = md.chunk_fib;
     for (int k = 0; k < a.nd_oth; ++k) ca.F[k] = a.F[k];
     ca.nworkers = md.nchunks;
+    ca.run = md.run;
   }
-  a.nworkers = use_csf ? md.nchunks : (vec ? (t->nnz + SP_W - 1) / SP_W : (t->nnz + SP_CH - 1) / SP_CH);
+  a.run = use_csf ? md.run : sp_run(ctx, t->nnz, vec ? SP_W : SP_CH);
+  a.nworkers = (t->nnz + a.run - 1) / a.run;
   const i64 nslots = 2 * a.nworkers;
   void *pv, *pk;
   TENRSO_TRY(ctx_buffer(ctx, SLOT_TMP, (size_t)2 * nslots * R * sizeof(float), &pv));

@@ -19,15 +19,14 @@ struct SpMode {
   // (i_n, i_o1, .., i_o(D-1)), D = nd - 1; fpre is D x nfib (SoA: row, then the
   // prefix's other indices).  The leaves are leafe (nnz words: the last other
   // mode's index, bit 31 set on the last nonzero of each fibre) and vals.
-  // chunk_fib[c] is the fibre holding nonzero c * SP_CSF_W.
+  // chunk_fib[c] is the fibre holding nonzero c * run.
   i64 nfib = 0;
   int32_t* leafe = nullptr;    // nnz
   int32_t* fpre = nullptr;     // D x nfib
   int32_t* chunk_fib = nullptr;
   i64 nchunks = 0;
+  int run = 0;                 // nonzeros per worker of the fibre kernel
 };
-
-constexpr int SP_CSF_W = 128;  // nonzeros per worker of the fibre kernel
 
 }  // namespace tenrso
 
