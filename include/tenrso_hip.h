@@ -101,8 +101,8 @@ int tenrso_mttkrp_f32_f64out(tenrso_ctx* ctx, const float* X, int ndim, const in
                              const float* const* factors, int64_t rank, int mode, double* out);
 
 /* BF16-input / FP32-accumulate MFMA MTTKRP.  X_bf16 is the tensor rounded to
- * bfloat16 (RNE, tenrso_convert_f32_to_bf16); factors stay FP32 and the
- * Khatri-Rao rows are formed in FP32 and rounded once to bf16.  No reference
+ * bfloat16 (RNE, tenrso_convert_f32_to_bf16); factors stay FP32 (the fastest mode's
+ * enters the matrix cores as a sum of two or three bf16 values).  No reference
  * counterpart (the reference has no reduced-precision MTTKRP). */
 int tenrso_mttkrp_bf16(tenrso_ctx* ctx, const uint16_t* X_bf16, int ndim, const int64_t* shape,
                        const float* const* factors, int64_t rank, int mode, float* out);
@@ -112,8 +112,8 @@ int tenrso_convert_f32_to_bf16(tenrso_ctx* ctx, const float* src, int64_t n, uin
  * fallback) MTTKRP kernel `reps` times back to back between two HIP events on
  * the context's stream and returns the average device time per launch in *ms.
  * precision selects the fp32 (X: float*) or bf16 (X: uint16_t*) kernel, or, with
- * 2, the three-way bf16 split kernel that the BF16 cp_als runs for its last mode
- * (X: float*, mode = ndim - 1). */
+ * 2, the fp32 kernel on a last-to-front copy of X (X: float*, mode = ndim - 1), the
+ * form that the ragged BF16 cp_als runs for its last mode. */
 int tenrso_mttkrp_profile(tenrso_ctx* ctx, int precision, const void* X, int ndim, const int64_t* shape,
                           const float* const* factors, int64_t rank, int mode, int reps, double* ms);
 
@@ -260,7 +260,7 @@ int tenrso_cp_als_f32_host(tenrso_ctx* ctx, const float* X, int ndim, const int6
  * SVD-based initial factors: InitStrategy::Svd / Nnsvd / LeverageScore of
  * initialize_factors (tenrso-decomp cp/helpers.rs:232-373), from the SVD of every
  * mode-k unfolding, on the device: the left singular vectors and singular values
- * are the eigenpairs of X_(k) X_(k)^T (FP64 Gram, one-workgroup Jacobi), each
+ * are the eigenpairs of X_(k) X_(k)^T (FP64 Gram, block Jacobi), each
  * vector's largest-magnitude entry made positive.  Mode sizes <= 1024, rank 1..64.
  * X: device tensor; factors: device buffers (shape[k] x rank, fp32).  seed drives
  * the N(0, 0.01) draws of the columns past min(rank, I_k, product of the other

@@ -189,7 +189,7 @@ int tenrso_mttkrp_profile(tenrso_ctx* ctx, int precision, const void* X, int ndi
     return TENRSO_OK;
   }
   TENRSO_TRY(set_device(ctx));
-  // precision 2: the three-way-split kernel of the BF16 ALS's last mode (fp32 X)
+  // precision 2: the fp32 kernel on a last-to-front copy (a ragged BF16 ALS's last mode)
   const bool x3 = precision == 2;
   if (x3 && mode != ndim - 1) {
     set_error("precision 2 profiles the last mode only");

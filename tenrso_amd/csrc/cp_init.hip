@@ -371,7 +371,8 @@ __global__ __launch_bounds__(512) void jacobi_update_kernel(EigArgs a, int r) {
     const double av = sT[(r0 + l16) * JPITCH + 4 * kk + q4];
 #pragma unroll
     for (int u = 0; u < 2; ++u)
-      acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, sQ[(4 * kk + q4) * JPITCH + c0 + 16 * u + l16], acc[u], 0, 0, 0);
+      acc[u] =
+          __builtin_amdgcn_mfma_f64_16x16x4f64(av, sQ[(4 * kk + q4) * JPITCH + c0 + 16 * u + l16], acc[u], 0, 0, 0);
   }
   __syncthreads();
   if (!isV) {

@@ -454,11 +454,11 @@ int solve_rows(tenrso_ctx* ctx, const float* part, int splits, const double* M, 
   }
   TENRSO_TRY(job_join(ctx));  // Winv of a wide-rank job on the side stream
   if (R > SOLVE_RMAX)
-    hipLaunchKernelGGL(solve_rows_kernel<WIDE_NE>, dim3(nblk), dim3(4 * WIDE_NE), 0, ctx->stream, part, splits, M, rows, (int)R,
-                       Winv, epi.l1, epi.nonneg, A, ip_part);
+    hipLaunchKernelGGL(solve_rows_kernel<WIDE_NE>, dim3(nblk), dim3(4 * WIDE_NE), 0, ctx->stream, part, splits, M, rows,
+                       (int)R, Winv, epi.l1, epi.nonneg, A, ip_part);
   else
-    hipLaunchKernelGGL(solve_rows_kernel<JOB_NE>, dim3(nblk), dim3(4 * JOB_NE), 0, ctx->stream, part, splits, M, rows, (int)R, Winv,
-                       epi.l1, epi.nonneg, A, ip_part);
+    hipLaunchKernelGGL(solve_rows_kernel<JOB_NE>, dim3(nblk), dim3(4 * JOB_NE), 0, ctx->stream, part, splits, M, rows,
+                       (int)R, Winv, epi.l1, epi.nonneg, A, ip_part);
   TENRSO_HIP_TRY(hipGetLastError());
   return TENRSO_OK;
 }

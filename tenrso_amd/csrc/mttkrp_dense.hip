@@ -1068,7 +1068,8 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
     // rank 32: 75 us with 576 workgroups, 70 with 1152, 69 with 1728).
     const bool with_norm = want_norm && fp32 && !bf16 && pad == 0 && !job && rchunks == 1 && NT < 8;
     if (fp32 && NT < 8 && !fuse_job && (wgs1 * ssp > target || with_norm)) {
-      kern = with_norm ? mttkrp_x3_kernel_norm(NT, caseB, a.win_vec, XL) : mttkrp_x3_kernel_w4(NT, caseB, a.win_vec, XL);
+      kern = with_norm ? mttkrp_x3_kernel_norm(NT, caseB, a.win_vec, XL)
+                       : mttkrp_x3_kernel_w4(NT, caseB, a.win_vec, XL);
       waves = 4;
       TENRSO_TRY(occupancy(ctx, kern, waves * 64, &occ));
       target = (i64)(ctx->wg_per_cu_f32 > 0 ? ctx->wg_per_cu_f32 : occ) * ctx->num_cus;

@@ -26,11 +26,11 @@ struct KernArgs {
   i64 qs;             // Q / fast_stride: slow indices per p (case A)
   const float* pre;   // PRE (rows = J / fast_size, stride R) or null (= 1)
   const float* fast;  // FAST factor (fast_size x R)
-  int kw;             // window of the fastest mode held in LDS (multiple of KB, divides fast_size)
-  int nwin;           // fast_size / kw
+  int kw;             // window of the fastest mode held in LDS (a multiple of the block)
+  int nwin;           // windows, ceil(fast_size / kw)
   i64 n_slow;         // J / fast_size
   i64 total;          // elements of X in memory
-  int slow_splits;    // splits of the slow range; grid.y = nwin * slow_splits
+  int slow_splits;    // splits of the slow range; nwin * slow_splits partials
   i64 slow_q, slow_rem;  // n_slow = slow_q * slow_splits + slow_rem
   int r0;             // first rank column of this launch
   int rcount;         // rank columns handled by the launch (<= 16*NT)

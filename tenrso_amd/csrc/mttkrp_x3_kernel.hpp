@@ -61,9 +61,8 @@ __device__ __forceinline__ void x3_split(const floatx8& x, bf16x8& h, bf16x8& l,
   }
 }
 
-// The work split: a workgroup owns 32 rows and one LDS
-// window (up to 128 rows) of the fastest mode, its waves contiguous ranges of its
-// blocks (32 consecutive j).  T = X FAST is contracted per slow index and folded
+// The work split: a workgroup owns 32 rows and one LDS window (up to 128 rows) of the
+// fastest mode, its waves contiguous ranges of its blocks (32 consecutive j).  T = X FAST is contracted per slow index and folded
 // into the accumulator with PRE[slow].  The FAST window is split once, when it
 // goes to LDS; X is split in registers, each element by one wave.
 // XL 0: whole windows, 16-byte aligned rows (case B: an even number of rows,
@@ -74,8 +73,8 @@ __device__ __forceinline__ void x3_split(const floatx8& x, bf16x8& h, bf16x8& l,
 // Forms.  JOB 1: 8 waves and the inlined ALS job, whose registers (235) leave one
 // workgroup a CU: the form of launches that carry the job or fill the GPU in one
 // round.  JOB 2: the same with the job of ranks 65 to 128, for eight rank tiles (one
-// pass over X and one split of it instead of two).  JOB 0: 4 waves: two (NT = 4) to four workgroups a CU, so that where
-// a CU runs several one after another the end of one meets the loop of the next
+// pass over X and one split of it instead of two).  JOB 0: 4 waves: two (NT = 4) to
+// four workgroups a CU, so that where a CU runs several one after another the end of one meets the loop of the next
 // (9216 rows x 9216 j at rank 32: 69-73 us against 77-85 us; one full round at
 // 256^3 rank 64: 19.1 us against 18.4 us).
 // NORM: the sum of squares of X as well (FP64; every element of X is read by exactly
