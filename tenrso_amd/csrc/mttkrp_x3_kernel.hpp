@@ -367,7 +367,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
 
 template <int NT, int WAVES, int JOB, bool CASE_B, bool WV, bool NORM>
 const void* x3_pick_xl(int xl) {
-  if constexpr (!CASE_B) {
+  if constexpr (!CASE_B && !NORM) {  // (the norm is not taken from a padded copy)
     if (xl == 4) return reinterpret_cast<const void*>(mttkrp_x3_mfma<NT, WAVES, JOB, CASE_B, WV, 4, NORM>);
   }
   if (xl == 0) return reinterpret_cast<const void*>(mttkrp_x3_mfma<NT, WAVES, JOB, CASE_B, WV, 0, NORM>);
