@@ -320,11 +320,12 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
     m = fmaxf(m, __shfl_xor(m, 32, 64));
     rmin = m > 0.f ? fminf(rmin, m) : rmin;
   }
-  {
+#pragma unroll
+  for (int r0 = 0; r0 < RT; r0 += 64) {  // a lane looks at one column, or two of 128
     float m = 0.f;
 #pragma unroll
-    for (int v = 0; v < WAVES; ++v) m = fmaxf(m, colmax[v][lane % RT]);
-    cmin = m > 0.f ? m : cmin;
+    for (int v = 0; v < WAVES; ++v) m = fmaxf(m, colmax[v][(r0 + lane) % RT]);
+    cmin = m > 0.f ? fminf(cmin, m) : cmin;
   }
   rmin = wave_min(rmin);
   cmin = wave_min(cmin);

@@ -1,0 +1,54 @@
+"""The MTTKRP on bf16 parts where some values lie near the lower end of the exponent range: in every tile form
+(window fully or partly filled, rank tiles of 1 to 8, all modes in one launch, the bf16 last mode), against FP64.
+
+TINY is 2^-121 with bits down to 2^-134, below the last bit of any bf16 value (2^-133): as a sum of bf16 parts it
+is off by 2^-13 of itself, wherever it stands, and always in the same direction.  All other values are positive, of
+magnitude 0.5 to 2, so every product with it is a normal fp32 number.
+
+Tolerance: that of the fp32 kernel's tests, (J + 8) 2^-23 sum |x kr| per element; J is below 1000, so a lost part
+of TINY exceeds it.
+"""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+from test_gpu_bf16_forms import bf16  # noqa: E402
+from test_gpu_mttkrp_split import check, mttkrp64, run  # noqa: E402
+
+from tenrso_amd import kernels  # noqa: E402
+
+TINY = np.float32(4097.4375 * 2.0 ** -133)
+
+
+def positive(shape, R):
+    rng = np.random.default_rng(sum(shape) + R)
+    X = rng.uniform(0.5, 2.0, shape).astype(np.float32)
+    return X, [rng.uniform(0.5, 2.0, (n, R)).astype(np.float32) for n in shape]
+
+
+def check_all(X, F):
+    check(X, F, run(X, F))
+    got = kernels.mttkrp_all_modes(torch.from_numpy(X).cuda(), [torch.from_numpy(f).cuda() for f in F])
+    check(X, F, [g.cpu().numpy() for g in got])
+    # bf16: the last mode takes exact parts of its fastest factor too
+    Xb, last = bf16(X), X.ndim - 1
+    got = kernels.mttkrp_bf16(Xb.cuda(), [torch.from_numpy(f).cuda() for f in F], last).cpu().numpy()
+    X32, J = Xb.float().numpy(), X.size // X.shape[-1]
+    lim = (J + 8) * 2.0 ** -23 * mttkrp64(X32, F, last, mag=True) + 1e-44
+    assert np.all(np.abs(got - mttkrp64(X32, F, last)) <= lim)
+
+
+def check_column(shape, R, col):
+    print(f"[case] small column {shape} R={R} column {col}", flush=True)
+    for k in (-1, -2):  # the fastest factor of every mode but the last, and that of the last
+        X, F = positive(shape, R)
+        F[k][:, col] = TINY
+        check_all(X, F)
+
+
+@pytest.mark.parametrize("shape,R,col", [((34, 3, 33), 65, 64), ((34, 4, 35), 100, 70), ((33, 5, 40), 128, 127),
+                                         ((5, 6, 128), 128, 64)])
+def test_small_column_past_64(shape, R, col):
+    check_column(shape, R, col)
