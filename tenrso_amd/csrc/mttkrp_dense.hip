@@ -318,7 +318,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
   for (int i = 0; i < NBUF - 1; ++i) load(i, b[i]);
   if constexpr (XL > 0) window_zero_tail(fw, kv);
   if constexpr (EXACT) {
-    window_colmax(fw, lane, colmax[wave]);
+    window_colmax(fw, lane, kv, colmax[wave]);
     stage_window_store_bf16x3<RT, PITCH, NTH, KWMAX>(sHi, sLo, sLo2, fw);
   } else {
     stage_window_store_bf16x2<RT, PITCH, NTH, KWMAX>(sHi, sLo, fw);

@@ -142,15 +142,18 @@ __device__ __forceinline__ float wave_min(float v) {
 
 // Largest magnitudes of the window's columns among the rows a wave stages, into its
 // colmax[RT].  A thread's units are all of the same four ranks (NTH is a multiple of
-// RT / 4), and the lanes RT / 4 apart hold them too.  Ranks past rcount repeat a
-// valid column.
+// RT / 4), and the lanes RT / 4 apart hold them too.  Rows past kv hold fillers of
+// another column and are passed over; ranks past rcount repeat a valid value.
 template <int RT, int NTH, int KWMAX>
-__device__ __forceinline__ void window_colmax(const FastWindow<RT, NTH, KWMAX>& fw, int lane, float* colmax) {
+__device__ __forceinline__ void window_colmax(const FastWindow<RT, NTH, KWMAX>& fw, int lane, int kv, float* colmax) {
   float m[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e)
+  for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e) {
+    const int kk = 2 * ((threadIdx.x + e * NTH) / (RT / 4));
 #pragma unroll
-    for (int q = 0; q < 4; ++q) max3_abs(m[q], fw.v[e][0][q], fw.v[e][1][q]);
+    for (int q = 0; q < 4; ++q)
+      max3_abs(m[q], kk < kv ? fw.v[e][0][q] : 0.f, kk + 1 < kv ? fw.v[e][1][q] : 0.f);
+  }
 #pragma unroll
   for (int o = RT / 4; o < 64; o <<= 1)
 #pragma unroll

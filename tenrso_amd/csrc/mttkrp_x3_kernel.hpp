@@ -287,7 +287,7 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
 #pragma unroll
   for (int i = 0; i < NBUF - 1; ++i) load(i, b[i]);
   if constexpr (XL > 0) window_zero_tail(fw, kv);
-  window_colmax(fw, lane, colmax[wave]);
+  window_colmax(fw, lane, kv, colmax[wave]);
   stage_window_store_bf16x3<RT, PITCH, NTH, KWMAX>(sHi, sLo, sLo2, fw);
   __syncthreads();  // LDS window staged
   for (int t = 0; t < T; t += NBUF) {

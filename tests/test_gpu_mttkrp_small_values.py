@@ -52,3 +52,9 @@ def check_column(shape, R, col):
                                          ((5, 6, 128), 128, 64)])
 def test_small_column_past_64(shape, R, col):
     check_column(shape, R, col)
+
+
+@pytest.mark.parametrize("shape,R,col", [((5, 2, 32), 9, 4), ((6, 32, 32), 8, 5), ((3, 64, 64), 8, 3), ((4, 96, 64), 40, 37),
+                                         ((3, 5, 160), 64, 60), ((3, 4, 32, 96), 20, 17), ((34, 4, 32), 100, 70)])
+def test_small_column_beside_an_unfilled_window(shape, R, col):
+    check_column(shape, R, col)
