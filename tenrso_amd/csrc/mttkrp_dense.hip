@@ -64,8 +64,8 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
   constexpr int LDS_BYTES = CASE_B || LDS_B > JOB_LDS_BYTES ? LDS_B : JOB_LDS_BYTES;
   static_assert(!CASE_B || KS == 1, "case B takes blocks of 32");
   __shared__ __attribute__((aligned(16))) float smem[LDS_BYTES / 4];
-  __shared__ float colmax[WAVES][RT];  // largest magnitude of each window column, by staging wave
-  __shared__ int plain;                // a wave asks for the plain form
+  __shared__ float wmin[WAVES];  // smallest magnitude of the window values that each wave stages
+  __shared__ int plain;          // a wave asks for the plain form
   if constexpr (!CASE_B) {  // the BF16 ALS contracts its last mode in fp32
     static_assert(NTH % JOB_THREADS == 0, "the ALS job runs on the first 256 threads");
     if (has_job && blockIdx.x == 0) {
@@ -231,9 +231,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
     if (t + 1 < T) cur.step(a);
   };
 
-  uint32_t rmax[MT];  // largest |x| of the lane's rows in this wave's blocks: even j, odd j
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) rmax[mt] = 0;
+  MinNonzero xmin;  // of the lane's X
   auto compute = [&](int t, const Buf& b) {
     if (t >= T) return;
 #pragma unroll
@@ -278,7 +276,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) rmax[mt] = max_u16x2(rmax[mt], xw[mt][q] & 0x7fff7fffu);
+          for (int q = 0; q < 4; ++q) xmin.add(xw[mt][q]);
       bf16x8 xv[MT];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) xv[mt] = __builtin_bit_cast(bf16x8, xw[mt]);
@@ -318,7 +316,8 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
   for (int i = 0; i < NBUF - 1; ++i) load(i, b[i]);
   if constexpr (XL > 0) window_zero_tail(fw, kv);
   if constexpr (EXACT) {
-    window_colmax(fw, lane, kv, colmax[wave]);
+    const float fw_min = window_min(fw);
+    if (lane == 0) wmin[wave] = fw_min;
     stage_window_store_bf16x3<RT, PITCH, NTH, KWMAX>(sHi, sLo, sLo2, fw);
   } else {
     stage_window_store_bf16x2<RT, PITCH, NTH, KWMAX>(sHi, sLo, fw);
@@ -334,22 +333,13 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
 
   float* out = partial + (i64)split * a.I * a.R;
   if constexpr (EXACT) {
-    // not finite, or small enough for the low parts (2^-16 of the products) to leave
-    // the exponent range: all of it again in fp32
-    float cm = 0.f;
+    // not finite, or too small for exact parts of FAST or for T (the bounds of the fp32
+    // kernel): all of it again in fp32
+    const float xm = wave_min(xmin.value());
+    float fm = wmin[0];
 #pragma unroll
-    for (int v = 0; v < WAVES; ++v) cm = fmaxf(cm, colmax[v][lane % RT]);
-    const float cmin = wave_min(cm > 0.f ? cm : 0x1p126f);
-    float xmin = 0x1p126f;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      float m = fmaxf(__uint_as_float(rmax[mt] << 16), __uint_as_float(rmax[mt] & 0xffff0000u));
-      m = fmaxf(m, __shfl_xor(m, 16, 64));
-      m = fmaxf(m, __shfl_xor(m, 32, 64));
-      xmin = m > 0.f ? fminf(xmin, m) : xmin;
-    }
-    xmin = wave_min(xmin);
-    const bool small = xmin < 0x1p-110f || cmin < 0x1p-96f || xmin * cmin < 0x1p-90f;
+    for (int v = 1; v < WAVES; ++v) fm = fminf(fm, wmin[v]);
+    const bool small = fm < 0x1p-108f || xm * fm < 0x1p-123f;
     if (__any(!(sum_of_zeros<MT, NT>(acc) == 0.f)) || small) plain = 1;
     __syncthreads();
     if (plain) {

@@ -121,18 +121,6 @@ __device__ __forceinline__ void window_zero_tail(FastWindow<RT, NTH, KWMAX>& fw,
   }
 }
 
-// m = max(m, |a|, |b|)
-__device__ __forceinline__ void max3_abs(float& m, float a, float b) {
-  asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b));
-}
-
-// maxima of two unsigned 16-bit halves
-__device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b) {
-  typedef unsigned short ushortx2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(
-      uint32_t, __builtin_elementwise_max(__builtin_bit_cast(ushortx2, a), __builtin_bit_cast(ushortx2, b)));
-}
-
 // smallest over the wave
 __device__ __forceinline__ float wave_min(float v) {
 #pragma unroll
@@ -140,27 +128,38 @@ __device__ __forceinline__ float wave_min(float v) {
   return v;
 }
 
-// Largest magnitudes of the window's columns among the rows a wave stages, into its
-// colmax[RT].  A thread's units are all of the same four ranks (NTH is a multiple of
-// RT / 4), and the lanes RT / 4 apart hold them too.  Rows past kv hold fillers of
-// another column and are passed over; ranks past rcount repeat a valid value.
-template <int RT, int NTH, int KWMAX>
-__device__ __forceinline__ void window_colmax(const FastWindow<RT, NTH, KWMAX>& fw, int lane, int kv, float* colmax) {
-  float m[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e) {
-    const int kk = 2 * ((threadIdx.x + e * NTH) / (RT / 4));
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      max3_abs(m[q], kk < kv ? fw.v[e][0][q] : 0.f, kk + 1 < kv ? fw.v[e][1][q] : 0.f);
+// The smallest magnitude of the bf16 values that are not zero, kept for each half of a
+// word as 2 |v| - 1 in 16 unsigned bits (zero becomes the largest): two instructions a
+// pair.
+struct MinNonzero {
+  typedef unsigned short ushortx2 __attribute__((ext_vector_type(2)));
+  ushortx2 m = {0xffff, 0xffff};
+  __device__ __forceinline__ void add(uint32_t pair) {
+    uint32_t two = 0x00020002u, ones = 0xffffffffu;
+    asm("" : "+s"(two), "+s"(ones));  // a multiply-add, not a shift and an add
+    const ushortx2 t =
+        __builtin_bit_cast(ushortx2, pair) * __builtin_bit_cast(ushortx2, two) + __builtin_bit_cast(ushortx2, ones);
+    m = __builtin_elementwise_min(m, t);
   }
+  // 2^126 if there is none
+  __device__ __forceinline__ float value() const {
+    const uint32_t b = ((uint32_t)min(m[0], m[1]) + 1) >> 1;
+    return b == 0x8000u ? 0x1p126f : __uint_as_float(b << 16);
+  }
+};
+
+// The smallest magnitude of the values a wave stages that are not zero, 2^126 if there
+// is none.  (Fillers of rows and ranks that do not exist repeat values of the window.)
+template <int RT, int NTH, int KWMAX>
+__device__ __forceinline__ float window_min(const FastWindow<RT, NTH, KWMAX>& fw) {
+  float m = 0x1p126f;
 #pragma unroll
-  for (int o = RT / 4; o < 64; o <<= 1)
+  for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) m[q] = fmaxf(m[q], __shfl_xor(m[q], o, 64));
-  if (lane < RT / 4)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) colmax[4 * lane + q] = m[q];
+      for (int q = 0; q < 4; ++q) m = fw.v[e][h][q] != 0.f ? fminf(m, fabsf(fw.v[e][h][q])) : m;
+  return wave_min(m);
 }
 
 // The window in LDS as a bf16 pair: FAST = hi + lo with hi = bf16(FAST) and

@@ -13,11 +13,13 @@
 // included), the five other terms 2 us more and the split of X 1 us.
 //
 // Special values.  The split of an infinity, or of a value that rounds to one in
-// bf16, gives NaN where fp32 arithmetic gives an infinity or a number; and a row of
-// X, a column of the window or their products near the end of the exponent range
-// would lose the low parts.  Both are seen at the end of the loop (an accumulator
-// that is not finite; the largest magnitudes of every row and column, kept on the
-// way), and the workgroup then forms its tile again in plain fp32 arithmetic.
+// bf16, gives NaN where fp32 arithmetic gives an infinity or a number.  A value below
+// 2^-109 has bits below the last one of any bf16 value (2^-133; denormal operands and
+// sums are exact here), and products below 2^-126, which a large PRE may bring back,
+// lose bits in T.  Both are seen at the end of the loop (an accumulator that is not
+// finite; the smallest magnitudes of X and of the window other than zero, kept on the
+// way), and the workgroup then forms its tile again in plain fp32 arithmetic.  The
+// smallest, not the largest of a row or column: the large ones may meet zeros.
 #pragma once
 #include "als_job_wide.hpp"
 #include "mttkrp_tile.hpp"
@@ -89,11 +91,11 @@ constexpr int x3_lds() {
   return win > red ? win : red;
 }
 
-// One workgroup's tile.  smem: x3_lds bytes; colmax: largest magnitude of each window
-// column, by staging wave; plain: a wave asks for the plain form.
+// One workgroup's tile.  smem: x3_lds bytes; wmin: smallest magnitude of the window
+// values that each wave stages; plain: a wave asks for the plain form.
 template <int NT, int WAVES, bool CASE_B, bool WV, int XL, bool NORM>
 __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernArgs& a, float* __restrict__ partial,
-                                        int tile, float* smem, float (*colmax)[16 * NT], int& plain) {
+                                        int tile, float* smem, float* wmin, int& plain) {
   constexpr int MT = 2, NBUF = X3_NBUF<NT>, KWMAX = X3_KWMAX;
   constexpr int KB = 32, PITCH = KWMAX + 8, RT = 16 * NT, NTH = WAVES * 64, ROWS = 16 * MT;
   const int xt = tile % a.rtiles;
@@ -132,9 +134,7 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
   double sumsq[MT];  // sum of squares of the lane's rows (NORM)
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) sumsq[mt] = 0.0;
-  float rmax[MT];  // largest |x| of the lane's row(s) in this wave's blocks
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) rmax[mt] = 0.f;
+  MinNonzero xmin;  // of the lane's X, rounded to bf16
   struct Buf {
     floatx8 x[MT];
     float pre[NT];
@@ -246,13 +246,14 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
           for (int e = 0; e < 8; ++e) x[e] = b.kb * KB + 8 * g + e < kv ? x[e] : 0.f;
         }
       }
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) max3_abs(rmax[mt], x[e], x[e + 1]);
       if constexpr (NORM) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) sumsq[mt] = fma((double)x[e], (double)x[e], sumsq[mt]);
       }
       x3_split(x, xh[mt], xl[mt], xl2[mt]);
+      const uint32x4 hw = __builtin_bit_cast(uint32x4, xh[mt]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xmin.add(hw[e]);
     }
     // Two rank tiles at a time, term by term (smallest first): consecutive MFMAs
     // then update 2 * MT different accumulators, so none waits for the previous
@@ -287,7 +288,8 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
 #pragma unroll
   for (int i = 0; i < NBUF - 1; ++i) load(i, b[i]);
   if constexpr (XL > 0) window_zero_tail(fw, kv);
-  window_colmax(fw, lane, kv, colmax[wave]);
+  const float fw_min = window_min(fw);
+  if (lane == 0) wmin[wave] = fw_min;
   stage_window_store_bf16x3<RT, PITCH, NTH, KWMAX>(sHi, sLo, sLo2, fw);
   __syncthreads();  // LDS window staged
   for (int t = 0; t < T; t += NBUF) {
@@ -311,25 +313,12 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
     if (lane == 0) a.norm[(i64)blockIdx.x * WAVES + wave] = v;
   }
 
-  // not finite, or small enough for the low parts (2^-16 of the products) to leave
-  // the exponent range: all of it again in fp32
-  float rmin = 0x1p126f, cmin = 0x1p126f;
+  // not finite, or too small: all of it again in fp32
+  const float xm = wave_min(xmin.value());
+  float fm = wmin[0];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    float m = fmaxf(rmax[mt], __shfl_xor(rmax[mt], 16, 64));
-    m = fmaxf(m, __shfl_xor(m, 32, 64));
-    rmin = m > 0.f ? fminf(rmin, m) : rmin;
-  }
-#pragma unroll
-  for (int r0 = 0; r0 < RT; r0 += 64) {  // a lane looks at one column, or two of 128
-    float m = 0.f;
-#pragma unroll
-    for (int v = 0; v < WAVES; ++v) m = fmaxf(m, colmax[v][(r0 + lane) % RT]);
-    cmin = m > 0.f ? fminf(cmin, m) : cmin;
-  }
-  rmin = wave_min(rmin);
-  cmin = wave_min(cmin);
-  const bool small = rmin < 0x1p-96f || cmin < 0x1p-96f || rmin * cmin < 0x1p-90f;
+  for (int v = 1; v < WAVES; ++v) fm = fminf(fm, wmin[v]);
+  const bool small = xm < 0x1p-108f || fm < 0x1p-108f || xm * fm < 0x1p-123f;
   if (__any(!(sum_of_zeros<MT, NT>(acc) == 0.f)) || small) plain = 1;
   __syncthreads();
   float* out = partial + (i64)split * a.I * a.R;
@@ -347,7 +336,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
   constexpr int LDS_JOB = JOB == 0 ? 0 : (JOB == 1 ? JOB_LDS_BYTES : WIDE_LDS_BYTES);
   constexpr int LDS_BYTES = LDS_B > LDS_JOB ? LDS_B : LDS_JOB;
   __shared__ __attribute__((aligned(16))) float smem[LDS_BYTES / 4];
-  __shared__ float colmax[WAVES][16 * NT];
+  __shared__ float wmin[WAVES];
   __shared__ int plain;
   if (JOB != 0 && has_job && blockIdx.x == 0) {
     // one such workgroup a CU, so the job has its CU to itself; waves past the
@@ -363,7 +352,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
     return;
   }
   x3_tile<NT, WAVES, CASE_B, WV, XL, NORM>(X, a, partial, (int)blockIdx.x - (JOB != 0 && has_job ? 1 : 0), smem,
-                                           colmax, plain);
+                                           wmin, plain);
 }
 
 template <int NT, int WAVES, int JOB, bool CASE_B, bool WV, bool NORM>

@@ -58,3 +58,36 @@ def test_small_column_past_64(shape, R, col):
                                          ((3, 5, 160), 64, 60), ((3, 4, 32, 96), 20, 17), ((34, 4, 32), 100, 70)])
 def test_small_column_beside_an_unfilled_window(shape, R, col):
     check_column(shape, R, col)
+
+
+@pytest.mark.parametrize("shape,R", [((5, 2, 32), 9), ((35, 3, 33), 20), ((6, 32, 64), 64), ((6, 4, 32), 100), ((3, 4, 5, 64), 40)])
+def test_small_entries_that_decide_a_result(shape, R):
+    """Small entries of a row or column whose other entries are not, where those others meet exact zeros."""
+    print(f"[case] small entries {shape} R={R}", flush=True)
+    X, F = positive(shape, R)
+    X[..., 5] = TINY
+    F[-1][:, 3] = 0.0
+    F[-1][5, 3] = 1.75
+    check_all(X, F)
+    X, F = positive(shape, R)
+    X[..., 7] = 0.0
+    X[1, ..., 7] = 1.5
+    X[1, ..., :7] = 0.0
+    X[1, ..., 8:] = 0.0
+    F[-1][7, 3] = TINY
+    check_all(X, F)
+
+
+def test_products_that_only_the_third_factor_makes_normal():
+    print("[case] small products", flush=True)
+    X, F = positive((40, 3, 32), 20)
+    X *= np.float32(2.0 ** -70)
+    F[2] *= np.float32(2.0 ** -70)
+    F[1] *= np.float32(2.0 ** 60)
+    check_all(X, F)
+    X, F = positive((40, 32, 33), 70)
+    X *= np.float32(2.0 ** -70)
+    F[1] *= np.float32(2.0 ** -70)
+    F[0] *= np.float32(2.0 ** 60)
+    F[2] *= np.float32(2.0 ** 60)
+    check_all(X, F)
