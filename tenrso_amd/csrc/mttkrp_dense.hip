@@ -47,7 +47,7 @@ namespace tenrso {
 // 70 us here).  Vectors are loaded unaligned, elements past the window's end (the next
 // row's) are masked, except where the load would pass the end of X.  As in the fp32
 // kernel a tile that is not finite, or whose values are too small for their low parts,
-// is formed again in plain fp32.
+// is formed again with the fp32 instruction.
 //   Case B: 64 rows a workgroup, lanes along i; each lane loads four rows (8 bytes) of
 // its 8 j, a full 128-byte line per j and 16 lanes, and byte permutes turn the 8 x 4
 // block into four A operands.  (A copy of X with the last mode in front took 43 us of
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
   static_assert(!CASE_B || KS == 1, "case B takes blocks of 32");
   __shared__ __attribute__((aligned(16))) float smem[LDS_BYTES / 4];
   __shared__ float wmin[WAVES];  // smallest magnitude of the window values that each wave stages
-  __shared__ int plain;          // a wave asks for the plain form
+  __shared__ int redo;           // a wave asks for the fp32 form
   if constexpr (!CASE_B) {  // the BF16 ALS contracts its last mode in fp32
     static_assert(NTH % JOB_THREADS == 0, "the ALS job runs on the first 256 threads");
     if (has_job && blockIdx.x == 0) {
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
   const i64 wb0 = uniform_i64(wave * nblk_wg / WAVES), wb1 = (wave + 1) * nblk_wg / WAVES;
   const int T = __builtin_amdgcn_readfirstlane((int)(wb1 - wb0));  // blocks of this wave
   const i64 row_base = (i64)xt * ROWS;
-  if (tid == 0) plain = 0;
+  if (tid == 0) redo = 0;
 
   FastWindow<RT, NTH, KWMAX> fw;  // window loads before the X blocks
   stage_window_load<WV>(fw, a, w, kv);
@@ -232,46 +232,50 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
   };
 
   MinNonzero xmin;  // of the lane's X
+  // eight j of each of the lane's rows, zero past the window's end
+  auto rows_of = [&](const Buf& b, int ks, uint32x4 (&xw)[MT]) {
+    if constexpr (!CASE_B) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        xw[mt] = b.x[mt][ks];
+        if constexpr (XL == 1) {
+          if (!((b.okm >> ks) & 1u)) xw[mt] = uint32x4{};
+        }
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        uint32x2 j0 = {b.x[e / 2][0][0], b.x[e / 2][0][1]}, j1 = {b.x[e / 2][0][2], b.x[e / 2][0][3]};
+        if constexpr (XL == 3) {
+          j0 = __builtin_bit_cast(uint32x2, __builtin_bit_cast(uint64_t, j0) >> shift);
+          j1 = __builtin_bit_cast(uint32x2, __builtin_bit_cast(uint64_t, j1) >> shift);
+        }
+        // low halves of (j0, j1), then high halves
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          xw[2 * h][e / 2] = __builtin_amdgcn_perm(j1[h], j0[h], 0x05040100u);
+          xw[2 * h + 1][e / 2] = __builtin_amdgcn_perm(j1[h], j0[h], 0x07060302u);
+        }
+      }
+    }
+    if constexpr (XL == 3) {
+      if (b.kb * KB + KB > kv) {  // the window's partly filled last block
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          const int k = b.kb * KB + 8 * g + e;
+          const uint32_t mask = (k < kv ? 0xffffu : 0u) | (k + 1 < kv ? 0xffff0000u : 0u);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) xw[mt][e / 2] &= mask;
+        }
+      }
+    }
+  };
   auto compute = [&](int t, const Buf& b) {
     if (t >= T) return;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       uint32x4 xw[MT];
-      if constexpr (!CASE_B) {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          xw[mt] = b.x[mt][ks];
-          if constexpr (XL == 1) {
-            if (!((b.okm >> ks) & 1u)) xw[mt] = uint32x4{};
-          }
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-          uint32x2 j0 = {b.x[e / 2][0][0], b.x[e / 2][0][1]}, j1 = {b.x[e / 2][0][2], b.x[e / 2][0][3]};
-          if constexpr (XL == 3) {
-            j0 = __builtin_bit_cast(uint32x2, __builtin_bit_cast(uint64_t, j0) >> shift);
-            j1 = __builtin_bit_cast(uint32x2, __builtin_bit_cast(uint64_t, j1) >> shift);
-          }
-          // low halves of (j0, j1), then high halves
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            xw[2 * h][e / 2] = __builtin_amdgcn_perm(j1[h], j0[h], 0x05040100u);
-            xw[2 * h + 1][e / 2] = __builtin_amdgcn_perm(j1[h], j0[h], 0x07060302u);
-          }
-        }
-      }
-      if constexpr (XL == 3) {
-        if (b.kb * KB + KB > kv) {  // the window's partly filled last block
-#pragma unroll
-          for (int e = 0; e < 8; e += 2) {
-            const int k = b.kb * KB + 8 * g + e;
-            const uint32_t mask = (k < kv ? 0xffffu : 0u) | (k + 1 < kv ? 0xffff0000u : 0u);
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) xw[mt][e / 2] &= mask;
-          }
-        }
-      }
+      rows_of(b, ks, xw);
       if constexpr (EXACT)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
@@ -340,11 +344,30 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
 #pragma unroll
     for (int v = 1; v < WAVES; ++v) fm = fminf(fm, wmin[v]);
     const bool small = fm < 0x1p-108f || xm * fm < 0x1p-123f;
-    if (__any(!(sum_of_zeros<MT, NT>(acc) == 0.f)) || small) plain = 1;
+    if (__any(!(sum_of_zeros<MT, NT>(acc) == 0.f)) || small) redo = 1;
     __syncthreads();
-    if (plain) {
-      plain_tile<CASE_B>(X, a, out, row_base, ROWS, w, kv, s_lo, s_hi, NTH);
-      return;
+    if (redo) {
+      redo_window<RT, NTH, KWMAX>(smem, a, w, kv);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+      cur = BlockCursor<1, KB, CASE_B>(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
+      __syncthreads();
+#pragma unroll 1
+      for (int t = 0; t < T; ++t) {
+        load(t, b[0]);
+        uint32x4 xw[MT];
+        rows_of(b[0], 0, xw);
+        floatx8 x[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            x[mt][e] = __uint_as_float(e % 2 ? xw[mt][e / 2] & 0xffff0000u : xw[mt][e / 2] << 16);
+        redo_block(acc, x, b[0].pre, smem, c, b[0].kb * KB + 8 * g, kv);
+      }
+      __syncthreads();  // window no longer read
     }
   }
   wg_reduce_store<MT, NT, WAVES, !EXACT>(acc, smem, wave, lane, out, a.I, a.R, a.r0, a.rcount, row_base, CASE_B);

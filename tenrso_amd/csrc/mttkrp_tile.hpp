@@ -353,28 +353,47 @@ __device__ __forceinline__ float sum_of_zeros(const floatx4 (&acc)[MT][NT]) {
   return z;
 }
 
-__device__ __forceinline__ float to_f32(float x) { return x; }
-__device__ __forceinline__ float to_f32(uint16_t x) { return __uint_as_float((uint32_t)x << 16); }
+// The form of a tile whose values bf16 parts cannot hold: the same blocks again with
+// v_mfma_f32_16x16x4_f32, products x (pre fast) in fp32.  The window goes to LDS in
+// fp32, s[r][kk] with a pitch of REDO_PITCH; the X blocks are loaded as before, one at a
+// time.  A mode of 256^3 at rank 64 takes 24 us, with one NaN in X 45 to 49, with a
+// small value in every tile 51 (one thread an output, in turn over the tile's j, took
+// 820 to 950 us for the one NaN); the bf16 last mode with infinities in every tile 41
+// (1218).
+constexpr int REDO_PITCH = 128 + 4;
 
-// The tile of one workgroup in plain fp32: acc = fma(x, pre * fast, acc) over its
-// slow range and window, one thread an output.
-template <bool CASE_B, typename TX>
-__device__ __forceinline__ void plain_tile(const TX* X, const KernArgs& a, float* out, i64 row_base, int rows, int w,
-                                           int kv, i64 s_lo, i64 s_hi, int nth) {
-  for (int e = threadIdx.x; e < rows * a.rcount; e += nth) {
-    const i64 row = row_base + e / a.rcount;
-    const int r = a.r0 + e % a.rcount;
-    if (row >= a.I) continue;
-    float acc = 0.f;
-    for (i64 slow = s_lo; slow < s_hi; ++slow) {
-      const float pre = a.pre ? a.pre[slow * a.R + r] : 1.f;
-      const i64 p = CASE_B ? 0 : slow / a.qs;
-      const TX* x = CASE_B ? X + (slow * a.fast_size + (i64)w * a.kw) * a.I + row
-                           : X + (p * a.I + row) * a.Q + (slow - p * a.qs) * a.fast_stride + (i64)w * a.kw;
-      const float* f = a.fast + (i64)w * a.kw * a.R + r;
-      for (int k = 0; k < kv; ++k) acc = fmaf(to_f32(x[CASE_B ? (i64)k * a.I : k]), pre * f[(i64)k * a.R], acc);
+// (Its addresses are its own: those of stage_window_load would stay in registers
+// through the main loop, up to 38 of them.)
+template <int RT, int NTH, int KWMAX>
+__device__ __forceinline__ void redo_window(float* __restrict__ s, const KernArgs& a, int w, int kv) {
+  static_assert(KWMAX + 4 == REDO_PITCH, "rows of the window are 16-byte aligned");
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  const float* base = a.fast + (i64)w * a.kw * a.R + a.r0;
+#pragma unroll 4
+  for (int u = tid; u < RT * KWMAX; u += NTH) {
+    const int r = u % RT, kk = u / RT;
+    s[r * REDO_PITCH + kk] = kk < kv && r < a.rcount ? base[kk * a.R + r] : 0.f;
+  }
+}
+
+// acc += x (pre fast) over one block of 32 j: a lane holds eight j of each of its rows,
+// from k0 = kb * 32 + 8 g on.
+template <int MT, int NT>
+__device__ __forceinline__ void redo_block(floatx4 (&acc)[MT][NT], const floatx8 (&x)[MT], const float (&pre)[NT],
+                                           const float* __restrict__ s, int c, int k0, int kv) {
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const float* row = s + (16 * nt + c) * REDO_PITCH + k0;
+    const floatx4 f0 = *reinterpret_cast<const floatx4*>(row), f1 = *reinterpret_cast<const floatx4*>(row + 4);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      // rows past kv are zero, but pre may be infinite
+      const float kr = k0 + e < kv ? pre[nt] * (e < 4 ? f0[e & 3] : f1[e & 3]) : 0.f;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[mt][e], kr, acc[mt][nt], 0, 0, 0);
     }
-    out[row * a.R + r] = acc;
   }
 }
 

@@ -14,13 +14,13 @@ __global__ __launch_bounds__(256) void mttkrp_x3_all(const float* __restrict__ X
   constexpr int WAVES = 4;
   __shared__ __attribute__((aligned(16))) float smem[x3_lds<NT, WAVES>() / 4];
   __shared__ float wmin[WAVES];
-  __shared__ int plain;
+  __shared__ int redo;
   int m = 0;
   while (m + 1 < p.nd && blockIdx.x >= p.first[m + 1]) ++m;
   const int tile = (int)(blockIdx.x - p.first[m]);
   const KernArgs a = p.a[m];
-  if (m == p.nd - 1) x3_tile<NT, WAVES, true, WV, XLB, false>(X, a, p.partial[m], tile, smem, wmin, plain);
-  else x3_tile<NT, WAVES, false, WV, XLA, false>(X, a, p.partial[m], tile, smem, wmin, plain);
+  if (m == p.nd - 1) x3_tile<NT, WAVES, true, WV, XLB, false>(X, a, p.partial[m], tile, smem, wmin, redo);
+  else x3_tile<NT, WAVES, false, WV, XLA, false>(X, a, p.partial[m], tile, smem, wmin, redo);
 }
 
 template <int NT, bool WV>

@@ -18,7 +18,7 @@
 // sums are exact here), and products below 2^-126, which a large PRE may bring back,
 // lose bits in T.  Both are seen at the end of the loop (an accumulator that is not
 // finite; the smallest magnitudes of X and of the window other than zero, kept on the
-// way), and the workgroup then forms its tile again in plain fp32 arithmetic.  The
+// way), and the workgroup then forms its tile again with the fp32 instruction.  The
 // smallest, not the largest of a row or column: the large ones may meet zeros.
 #pragma once
 #include "als_job_wide.hpp"
@@ -88,14 +88,15 @@ __device__ __forceinline__ void x3_split(const floatx8& x, bf16x8& h, bf16x8& l,
 template <int NT, int WAVES>
 constexpr int x3_lds() {
   constexpr int win = 3 * 16 * NT * (X3_KWMAX + 8) * 2, red = 2 * NT * WAVES * 64 * 16;
+  static_assert(win >= 16 * NT * REDO_PITCH * 4, "the fp32 window of a tile formed again");
   return win > red ? win : red;
 }
 
 // One workgroup's tile.  smem: x3_lds bytes; wmin: smallest magnitude of the window
-// values that each wave stages; plain: a wave asks for the plain form.
+// values that each wave stages; redo: a wave asks for the fp32 form.
 template <int NT, int WAVES, bool CASE_B, bool WV, int XL, bool NORM>
 __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernArgs& a, float* __restrict__ partial,
-                                        int tile, float* smem, float* wmin, int& plain) {
+                                        int tile, float* smem, float* wmin, int& redo) {
   constexpr int MT = 2, NBUF = X3_NBUF<NT>, KWMAX = X3_KWMAX;
   constexpr int KB = 32, PITCH = KWMAX + 8, RT = 16 * NT, NTH = WAVES * 64, ROWS = 16 * MT;
   const int xt = tile % a.rtiles;
@@ -118,7 +119,7 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
   const i64 wb0 = uniform_i64(wave * nblk_wg / WAVES), wb1 = (wave + 1) * nblk_wg / WAVES;
   const int T = __builtin_amdgcn_readfirstlane((int)(wb1 - wb0));  // blocks of this wave
   const i64 row_base = (i64)xt * ROWS;
-  if (tid == 0) plain = 0;
+  if (tid == 0) redo = 0;
 
   FastWindow<RT, NTH, KWMAX> fw;  // window loads before the X blocks
   stage_window_load<WV>(fw, a, w, kv);
@@ -229,23 +230,28 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
     if (t + 1 < T) cur.step(a);
   };
 
+  // eight j of the lane's row mt, zero past the window's end
+  auto row_of = [&](const Buf& b, int mt) -> floatx8 {
+    floatx8 x = b.x[mt];
+    if constexpr (XL == 1) {
+      if constexpr (CASE_B) {
+        if (mt == 0)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[e] = tail ? b.x[1][e] : x[e];
+      }
+      if (b.kb * KB + KB > kv) {  // the window's partly filled last block
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = b.kb * KB + 8 * g + e < kv ? x[e] : 0.f;
+      }
+    }
+    return x;
+  };
   auto compute = [&](int t, const Buf& b) {
     if (t >= T) return;
     bf16x8 xh[MT], xl[MT], xl2[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      floatx8 x = b.x[mt];
-      if constexpr (XL == 1) {
-        if constexpr (CASE_B) {
-          if (mt == 0)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = tail ? b.x[1][e] : x[e];
-        }
-        if (b.kb * KB + KB > kv) {  // the window's partly filled last block
-#pragma unroll
-          for (int e = 0; e < 8; ++e) x[e] = b.kb * KB + 8 * g + e < kv ? x[e] : 0.f;
-        }
-      }
+      const floatx8 x = row_of(b, mt);
       if constexpr (NORM) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) sumsq[mt] = fma((double)x[e], (double)x[e], sumsq[mt]);
@@ -319,12 +325,24 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
 #pragma unroll
   for (int v = 1; v < WAVES; ++v) fm = fminf(fm, wmin[v]);
   const bool small = xm < 0x1p-108f || fm < 0x1p-108f || xm * fm < 0x1p-123f;
-  if (__any(!(sum_of_zeros<MT, NT>(acc) == 0.f)) || small) plain = 1;
+  if (__any(!(sum_of_zeros<MT, NT>(acc) == 0.f)) || small) redo = 1;
   __syncthreads();
   float* out = partial + (i64)split * a.I * a.R;
-  if (plain) {
-    plain_tile<CASE_B>(X, a, out, row_base, ROWS, w, kv, s_lo, s_hi, NTH);
-    return;
+  if (redo) {
+    redo_window<RT, NTH, KWMAX>(smem, a, w, kv);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    cur = BlockCursor<1, KB, CASE_B>(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
+    __syncthreads();
+#pragma unroll 1
+    for (int t = 0; t < T; ++t) {
+      load(t, b[0]);
+      const floatx8 x[MT] = {row_of(b[0], 0), row_of(b[0], 1)};
+      redo_block(acc, x, b[0].pre, smem, c, b[0].kb * KB + 8 * g, kv);
+    }
+    __syncthreads();  // window no longer read
   }
   wg_reduce_store<MT, NT, WAVES, false>(acc, smem, wave, lane, out, a.I, a.R, a.r0, a.rcount, row_base, CASE_B);
 }
@@ -337,7 +355,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
   constexpr int LDS_BYTES = LDS_B > LDS_JOB ? LDS_B : LDS_JOB;
   __shared__ __attribute__((aligned(16))) float smem[LDS_BYTES / 4];
   __shared__ float wmin[WAVES];
-  __shared__ int plain;
+  __shared__ int redo;
   if (JOB != 0 && has_job && blockIdx.x == 0) {
     // one such workgroup a CU, so the job has its CU to itself; waves past the
     // rank-64 job's four end at once
@@ -352,7 +370,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
     return;
   }
   x3_tile<NT, WAVES, CASE_B, WV, XL, NORM>(X, a, partial, (int)blockIdx.x - (JOB != 0 && has_job ? 1 : 0), smem,
-                                           wmin, plain);
+                                           wmin, redo);
 }
 
 template <int NT, int WAVES, int JOB, bool CASE_B, bool WV, bool NORM>

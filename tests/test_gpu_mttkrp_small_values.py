@@ -91,3 +91,48 @@ def test_products_that_only_the_third_factor_makes_normal():
     F[0] *= np.float32(2.0 ** 60)
     F[2] *= np.float32(2.0 ** 60)
     check_all(X, F)
+
+
+@pytest.mark.parametrize("shape,R", [((70, 33, 130), 16), ((64, 40, 256), 33), ((33, 70, 97), 64), ((9000, 2, 20), 8), ((2, 20, 9001), 24),
+                                     ((40, 64, 66), 128), ((35, 3, 4, 67), 100), ((20, 9, 11, 32), 40)])
+def test_tiles_formed_again(shape, R):
+    """A small value, an infinity and a NaN in many tiles: every other result keeps its tolerance."""
+    print(f"[case] tiles again {shape} R={R}", flush=True)
+    X, F = positive(shape, R)
+    X.reshape(-1)[::97] = TINY
+    check_all(X, F)
+    X.reshape(-1)[0] = np.inf
+    X.reshape(-1)[X.size // 2] = np.nan
+    got = kernels.mttkrp_all_modes(torch.from_numpy(X).cuda(), [torch.from_numpy(f).cuda() for f in F])
+    one = run(X, F)
+    for m in range(X.ndim):
+        with np.errstate(invalid="ignore"):
+            ref = mttkrp64(X, F, m)
+        fin = np.isfinite(ref)
+        lim = (X.size // X.shape[m] + 8) * 2.0 ** -23 * np.abs(ref)
+        for g in (got[m].cpu().numpy(), one[m]):
+            assert np.array_equal(np.isnan(g), np.isnan(ref)) and np.array_equal(np.isposinf(g), np.isposinf(ref)), m
+            assert np.all(np.abs(g[fin] - ref[fin]) <= lim[fin]), m
+
+
+def test_a_nan_costs_a_second_pass():
+    """Forming a tile again takes the order of the launch's time, not that of a serial loop (25 to 50 times it)."""
+    print("[case] time with a NaN", flush=True)
+    X = torch.ones((256, 256, 256), device="cuda")
+    F = [torch.ones((256, 64), device="cuda") for _ in range(3)]
+
+    def best():
+        ms = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                kernels.mttkrp(X, F, 1)
+            b.record()
+            b.synchronize()
+            ms.append(a.elapsed_time(b))
+        return min(ms)
+
+    ordinary = best()
+    X[3, 4, 5] = float("nan")
+    assert best() <= 8 * ordinary
