@@ -34,34 +34,55 @@ __device__ __forceinline__ double wide_block_sum(double v, double* red) {
 }
 
 // Inverse of the 4 x 4 pivot block at lds[pb] (rows of stride WIDE_NE) by one wave,
-// into lds[pi], the block itself replaced by the identity: lane (r, c) = (lane / 4 %
-// 4, lane % 4) forms the cofactor C[r][c], det is the row-r expansion summed over
-// the lane's quad, and P^-1[c][r] = C[r][c] / det.  Positive definiteness by
-// Sylvester's criterion (see job_block_gj).
+// into lds[pi], the block itself replaced by the identity.  Every lane sweeps the
+// symmetric block's upper triangle, one scalar pivot after another (the sweep of
+// pivot p: a_ij -= a_ip a_pj / a_pp, a_ip /= a_pp, a_pp = -1 / a_pp, which ends with
+// minus the inverse).  A pivot that is not positive and finite sets the flag.  Cofactors
+// over the determinant were shorter by 0.1 us a step, but their error grows with the
+// cube of the block's condition, not with the condition itself: factors with four
+// collinear columns (condition 1e7) came out with an inverse off by 1e-3 instead of
+// 1e-9, and at 1e9 the determinant's sign was noise.
 __device__ __forceinline__ void wide_invert_pivot(double* lds, int pb, int pi) {
   const int lane = threadIdx.x & 63, lr = (lane >> 2) & 3, lc = lane & 3;
-  const int rr[3] = {lr == 0 ? 1 : 0, lr <= 1 ? 2 : 1, lr <= 2 ? 3 : 2};
-  const int cc[3] = {lc == 0 ? 1 : 0, lc <= 1 ? 2 : 1, lc <= 2 ? 3 : 2};
   const double* Pb = lds + pb;
-  double m[9];
+  double p[4][4];  // upper triangle
 #pragma unroll
-  for (int u = 0; u < 3; ++u)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int v = 0; v < 3; ++v) m[3 * u + v] = Pb[rr[u] * WIDE_NE + cc[v]];
-  const double pself = Pb[lr * WIDE_NE + lc], p00 = Pb[0], p01 = Pb[1], p11 = Pb[WIDE_NE + 1];
+    for (int k = i; k < 4; ++k) p[i][k] = Pb[i * WIDE_NE + k];
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   const int none = WIDE_NONE + lane;
   lds[lane < 16 ? pb + lr * WIDE_NE + lc : none] = lr == lc ? 1.0 : 0.0;
-  const double d3 = m[0] * fma(m[4], m[8], -(m[5] * m[7])) - m[1] * fma(m[3], m[8], -(m[5] * m[6])) +
-                    m[2] * fma(m[3], m[7], -(m[4] * m[6]));
-  const double cof = ((lr + lc) & 1) ? -d3 : d3;
-  double det = pself * cof;
-  det += job_quad_perm<0xB1>(det);
-  det += job_quad_perm<0x4E>(det);
-  const bool good = (p00 > 0.0) & (fma(p00, p11, -(p01 * p01)) > 0.0) & (det > 0.0) & (det <= DBL_MAX) &
-                    ((lane != 15) | (cof > 0.0));
-  const double rd = job_recip(det);
-  lds[lane < 16 ? pi + lc * 4 + lr : none] = cof * rd;
+  bool good = true;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    good = good & (p[k][k] > 0.0) & (p[k][k] <= DBL_MAX);
+    const double d = job_recip(p[k][k]);
+    double b[4], t[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      b[i] = i < k ? p[i][k] : p[k][i];
+      t[i] = b[i] * d;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int m = i; m < 4; ++m)
+        if (i != k && m != k) p[i][m] = fma(-t[i], b[m], p[i][m]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (i < k) p[i][k] = t[i];
+      if (i > k) p[k][i] = t[i];
+    }
+    p[k][k] = -d;
+  }
+  // lane (r, c) stores entry (r, c)
+  double v = p[0][0];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int k = i; k < 4; ++k) v = (lr == i && lc == k) || (lr == k && lc == i) ? p[i][k] : v;
+  lds[lane < 16 ? pi + lr * 4 + lc : none] = -v;
   lds[((lane < 16) & !good) ? WIDE_FLAG : none] = 1.0;
 }
 
