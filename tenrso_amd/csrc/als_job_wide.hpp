@@ -166,10 +166,13 @@ __device__ __forceinline__ bool wide_block_gj(doublex4 (&acc)[8 - ST], int R, do
         __builtin_amdgcn_s_setprio(0);
       }
       if (ps1 > ST && s1 < steps) {
-        // The accumulators are read behind a chain of scalar branches below.  The
-        // compiler counts those instructions towards the wait that a read of an
-        // FP64 MFMA's result needs, and the hardware runs them faster: a last tile
-        // read that way came out stale.  So the wait stands here, tied to them.
+        // Left to itself the compiler turns the choice of tile below into one indexed
+        // register read (s_set_gpr_idx_on, v_mov_b32 from the first tile's registers),
+        // and the wait that a read of an FP64 MFMA's result needs is then counted from
+        // the first tile's MFMA, not from the last one's: a last tile read that way
+        // came out stale.  Tied to the accumulators, the wait stands here for all of
+        // them, and the reads name their registers, as those of the pivot's wave above
+        // do anyway.
 #pragma unroll
         for (int u = 1; u < NU; ++u) asm volatile("" : "+v"(acc[u]));
         asm volatile("s_nop 15\n\ts_nop 15" : "+v"(acc[NU - 1]));
