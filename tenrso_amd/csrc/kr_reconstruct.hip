@@ -7,6 +7,7 @@
 // cp_reconstruct (tenrso-kernels/src/outer.rs:223-274):
 //   out[i_0..i_{N-1}] = sum_r (prod_k F_k[i_k, r]) * w_r.
 //   An FP32 matrix product of two Khatri-Rao factors formed in LDS.
+#include <cfloat>
 #include <type_traits>
 
 #include "kr_reconstruct.hpp"
@@ -69,6 +70,11 @@ struct ReconArgs {
 // Operands are read from LDS as 4 consecutive ranks (lane group g, step s
 // contracts rank 16u + 4g + s on both sides); the pitch of KT + 4 floats keeps
 // those 16-byte reads free of bank conflicts.
+// A product of one side alone may leave the exponent range where the whole product,
+// left to right, does not (factors of sizes 1e30, 1e-25, 1e-25).  Every thread keeps
+// the extremes of its products; where one is subnormal or not finite although its
+// factors are neither zero nor infinite, and the other side could bring it back, the
+// tile is formed again element by element.
 // Bound: at 256^3 rank 64 the 2.1 GFLOP take 14 us at the matrix cores' FP32
 // peak and the 64 MiB of output 13 us at 5.2 TB/s; the form with one thread per
 // element, each lane reading factor rows at a stride of R floats, took 2580 us; this
@@ -78,11 +84,13 @@ __global__ __launch_bounds__(256) void reconstruct_kernel(ReconArgs a, float* __
   constexpr int TILE = 32 * T, PITCH = KT + 4;
   __shared__ __attribute__((aligned(16))) float sk[2 * TILE * PITCH];  // rows, then columns
   __shared__ i64 sidx[MAXD_RECON][TILE];
+  __shared__ int range;  // 1, 2: a product of the rows, columns is subnormal; 4, 8: one is above 1; 16: not finite
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
   const i64 r_base = (i64)(blockIdx.x / a.ctiles) * TILE, c_base = (i64)(blockIdx.x % a.ctiles) * TILE;
   // factor rows of every tile row (modes < h) and column (modes >= h); those past
   // the end repeat the last one and are not stored
+  if (tid == 0) range = 0;
   if (tid < 2 * TILE) {
     const bool col = tid >= TILE;
     const int e = col ? tid - TILE : tid;
@@ -99,6 +107,8 @@ __global__ __launch_bounds__(256) void reconstruct_kernel(ReconArgs a, float* __
     for (int i = 0; i < T; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
   const float* sr = sk + (16 * T * (wave >> 1) + c) * PITCH + 4 * g;
   const float* sc = sk + (TILE + 16 * T * (wave & 1) + c) * PITCH + 4 * g;
+  int seen = 0;  // bits of `range`
+  float big[2] = {0.f, 0.f};
   for (i64 r0 = 0; r0 < a.R; r0 += KT) {
     __syncthreads();  // indices written, or the previous chunk read
     // one side at a time: a thread's units (4 ranks of one row each) load their
@@ -130,11 +140,42 @@ __global__ __launch_bounds__(256) void reconstruct_kernel(ReconArgs a, float* __
       float wq[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) wq[q] = (a.w && side == 0 && r + q < a.R) ? a.w[r + q] : 1.f;
+      float least = 1.f, zeros = 0.f;  // zeros: NaN where a product is not finite
 #pragma unroll
       for (int u = 0; u < UN; ++u) {
+        floatx4 sv;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[u][q] = r + q < a.R ? v[u][q] * wq[q] : 0.f;
-        *reinterpret_cast<floatx4*>(sk + (side * TILE + (tid + 256 * u) / (KT / 4)) * PITCH + q4) = v[u];
+        for (int q = 0; q < 4; ++q) {
+          v[u][q] = r + q < a.R ? v[u][q] * wq[q] : 1.f;
+          sv[q] = r + q < a.R ? v[u][q] : 0.f;
+          least = fminf(least, fabsf(v[u][q]));
+          big[side] = fmaxf(big[side], fabsf(v[u][q]));
+          zeros = fmaf(v[u][q], 0.f, zeros);
+        }
+        *reinterpret_cast<floatx4*>(sk + (side * TILE + (tid + 256 * u) / (KT / 4)) * PITCH + q4) = sv;
+      }
+      if (least < 0x1p-126f || !(zeros == 0.f)) {
+#pragma unroll 1
+        for (int x = 0; x < UN * 4; ++x) {
+          const i64 rx = r + x % 4;
+          if (rx >= a.R) continue;
+          bool nonzero = true, finite = true;
+          float p = 1.f;
+          for (int k = k0; k < k1; ++k) {
+            const float f = a.F[k][sidx[k][(tid + 256 * (x / 4)) / (KT / 4)] * a.R + rx];
+            nonzero = nonzero && f != 0.f;
+            finite = finite && fabsf(f) <= FLT_MAX;
+            p *= f;
+          }
+          if (a.w && side == 0) {
+            const float f = a.w[rx];
+            nonzero = nonzero && f != 0.f;
+            finite = finite && fabsf(f) <= FLT_MAX;
+            p *= f;
+          }
+          if (nonzero && fabsf(p) < 0x1p-126f) seen |= 1 << side;
+          if (finite && !(fabsf(p) <= FLT_MAX)) seen |= 16;
+        }
       }
     }
     __syncthreads();
@@ -155,7 +196,35 @@ __global__ __launch_bounds__(256) void reconstruct_kernel(ReconArgs a, float* __
             acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(cv[j][s], rv[i][s], acc[j][i], 0, 0, 0);
     }
   }
+  if (big[0] > 1.f) seen |= 4;
+  if (big[1] > 1.f) seen |= 8;
+#pragma unroll
+  for (int b = 0; b < 5; ++b)
+    if (__any(seen >> b & 1) && lane == 0) atomicOr(&range, 1 << b);
+  __syncthreads();
   const float gs = a.gscale ? a.gscale[0] : 1.0f;
+  if ((range & 16) || ((range & 1) && (range & 8)) || ((range & 2) && (range & 4))) {
+    int x0 = tid;
+    asm volatile("" : "+v"(x0));  // (nothing of this in registers during the loop above)
+#pragma unroll 1
+    for (int x = x0; x < TILE * TILE; x += 256) {
+      const i64 row = r_base + x / TILE, col = c_base + x % TILE;
+      if (row >= a.M || col >= a.N) continue;
+      float s = 0.f;
+#pragma unroll 1
+      for (i64 r = 0; r < a.R; ++r) {
+        float p = 1.f;
+        for (int k = 0; k < a.nd; ++k) p *= a.F[k][sidx[k][k < a.h ? x / TILE : x % TILE] * a.R + r];
+        if (a.w) p *= a.w[r];
+        s += p;
+      }
+      const i64 o = row * a.N + col;
+      if (a.xsub) s = a.xsub[o] - s;
+      if (a.gscale) s *= gs;
+      out[o] = s;
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < T; ++i) {
     const i64 row = r_base + 16 * T * (wave >> 1) + 16 * i + c;
