@@ -65,9 +65,10 @@ struct tenrso_ctx {
   std::vector<tenrso::DevBuf> bufs;  // indexed by slot id
   void* pinned = nullptr;            // small pinned (coherent) host buffer for scalar readback
   double* pinned_dev = nullptr;      // the same buffer as a device pointer (kernels write the fit there)
-  // workgroups per CU of each MTTKRP kernel instance (occupancy query cache)
-  const void* occ_kern[64] = {};
-  int occ_val[64] = {};
+  // workgroups per CU of each MTTKRP kernel instance (occupancy query cache; there are
+  // 160 of them, and a query costs the host more than a launch)
+  const void* occ_kern[256] = {};
+  int occ_val[256] = {};
   int occ_n = 0;
   void* blas = nullptr;              // rocBLAS handle of the n-mode products, made on first use
   // side stream of the wide-rank ALS job (made on first use): the job overlaps the

@@ -854,7 +854,7 @@ static int occupancy(tenrso_ctx* ctx, const void* kern, int threads, int* occ) {
   int nb = 0;
   TENRSO_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, threads, 0));
   *occ = std::max(1, nb);
-  if (ctx->occ_n < 64) {
+  if (ctx->occ_n < (int)(sizeof(ctx->occ_val) / sizeof(ctx->occ_val[0]))) {
     ctx->occ_kern[ctx->occ_n] = kern;
     ctx->occ_val[ctx->occ_n++] = *occ;
   }
