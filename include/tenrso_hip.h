@@ -261,7 +261,7 @@ int tenrso_cp_als_f32_host(tenrso_ctx* ctx, const float* X, int ndim, const int6
  * initialize_factors (tenrso-decomp cp/helpers.rs:232-373), from the SVD of every
  * mode-k unfolding, on the device: the left singular vectors and singular values
  * are the eigenpairs of X_(k) X_(k)^T (FP64 Gram, block Jacobi), each
- * vector's largest-magnitude entry made positive.  Mode sizes <= 1024, rank 1..64.
+ * vector's largest-magnitude entry made positive.  Mode sizes <= 1024, rank 1..128.
  * X: device tensor; factors: device buffers (shape[k] x rank, fp32).  seed drives
  * the N(0, 0.01) draws of the columns past min(rank, I_k, product of the other
  * modes), which the reference takes from an unseeded thread_rng.

@@ -65,8 +65,8 @@ struct tenrso_ctx {
   std::vector<tenrso::DevBuf> bufs;  // indexed by slot id
   void* pinned = nullptr;            // small pinned (coherent) host buffer for scalar readback
   double* pinned_dev = nullptr;      // the same buffer as a device pointer (kernels write the fit there)
-  // workgroups per CU of each MTTKRP kernel instance (occupancy query cache; there are
-  // 160 of them, and a query costs the host more than a launch)
+  // workgroups per CU of each MTTKRP kernel instance (occupancy query cache, for all of
+  // the 160 there are)
   const void* occ_kern[256] = {};
   int occ_val[256] = {};
   int occ_n = 0;

@@ -36,8 +36,8 @@ struct MttkrpScratch {
 // last mode's MTTKRP contracts instead of X, at FP32 accuracy also in a BF16 call.
 // job (optional): the ALS linear algebra of this mode; it runs as workgroup 0 of the
 // MTTKRP launch (or, where it cannot, as its own kernel just before it).
-// x_pad / xt_pad (BF16 only, 0 = none): the memory extent of the last mode of X
-// and of X_t when those copies have it padded with zeros.
+// x_pad / xt_pad (0 = none): the memory extent of the last mode of X and of X_t when
+// those are copies that have it padded with zeros (an ALS of ragged shapes).
 // want_norm: also leave FP64 partial sums of ||X||^2 in res->norm (FP32 calls whose
 // ranks fit one launch of the MFMA kernel; null otherwise).
 // slot: the context buffer of the split partials.  plan: only fill it, launch nothing

@@ -51,7 +51,7 @@ namespace tenrso {
 //   Case B: 64 rows a workgroup, lanes along i; each lane loads four rows (8 bytes) of
 // its 8 j, a full 128-byte line per j and 16 lanes, and byte permutes turn the 8 x 4
 // block into four A operands.  (A copy of X with the last mode in front took 43 us of
-// the 64 of a 512x256x256 rank 64 last mode; this form takes 19.)
+// the 64 of a 512x512x128 rank 64 last mode; this form takes 20.)
 // ---------------------------------------------------------------------------
 template <int NT, int WAVES, int KS, int KWMAX, bool CASE_B, bool WV, int XL>
 __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* __restrict__ X, KernArgs a,
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) poff[nt] = (has_pre ? a.r0 : 0) + (16 * nt + c < a.rcount ? 16 * nt + c : 0);
 
-  BlockCursor<1, KB, CASE_B> cur(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
+  BlockCursor<KB, CASE_B> cur(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
 
   auto load = [&](int t, Buf& b) {
     b.kb = cur.kb;
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-      cur = BlockCursor<1, KB, CASE_B>(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
+      cur = BlockCursor<KB, CASE_B>(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
       __syncthreads();
 #pragma unroll 1
       for (int t = 0; t < T; ++t) {
@@ -374,9 +374,9 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
 }
 
 // ---------------------------------------------------------------------------
-// Generic fallback for shapes the MFMA tiling does not cover (fastest other mode
-// not a multiple of the block, rank > 64 corner cases are handled by chunks).
-// One thread per (i, r); grid.y splits j.  FP32 accumulate like the MFMA path.
+// What the MFMA kernels do not take: empty contractions (the result is zero) and a
+// tensor that is not aligned to its own element type.  One thread per (i, r); grid.y
+// splits j.
 // ---------------------------------------------------------------------------
 struct GenericArgs {
   int nd, mode, n_oth;

@@ -61,9 +61,11 @@ __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
 // (fp32) or two 4-byte (bf16 hi, lo) pairs per rank.  With a 16-byte aligned
 // FAST and R % 4 == 0 (win_vec) a unit is two 16-byte loads, else eight 4-byte
 // loads (one kernel instance per case, so that every instance has a single
-// load sequence and the waits stay exact).  Ranks past rcount and rows past kw load column r0 of window row 0
-// instead (always inside FAST): those rank columns are never stored and those
-// rows never read, so no value select is needed and no load waits early.
+// load sequence and the waits stay exact).  Ranks past rcount and rows past kv load
+// the first columns of window row 0 instead (always inside FAST), so no load waits for
+// a select: those rank columns are never stored, those rows are never read or
+// (window_zero_tail) zeroed, and window_min, which does see them, sees values of the
+// window.
 // Split in two so the window loads are issued before the first X blocks: the
 // LDS writes then wait for the window only (vector loads retire in issue order).
 template <int RT, int NTH, int KWMAX>
@@ -232,23 +234,21 @@ static __device__ float kPreOnes[128] = {
     TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8};
 #undef TENRSO_ONES8
 
-// Block schedule of one wave.  Block t of the wave is block kb = t % nkb of the
-// slow index s_lo + wave + WAVES*(t / nkb).  Loads run in t order, so the cursor
-// only steps forward, and it stops on the wave's last block (loads past the end
-// are redirected by the kernels to one cache line).  Every X and PRE load is thus unconditional
-// and the wait before a block's MFMAs counts exactly the loads issued after it,
-// which keeps the prefetch in flight.  A wave with no block reads the block of
-// slow index min(s_lo + wave, n_slow - 1), always inside X, and computes nothing.
+// Block schedule of one wave: a contiguous range of the workgroup's blocks, from block
+// kb0 of slow index slow0 on, nkb blocks a slow index.  Loads run in that order, so the
+// cursor only steps forward, and it stops on the wave's last block (loads past the end
+// are redirected by the kernels to one cache line).  Every X and PRE load is thus
+// unconditional and the wait before a block's MFMAs counts exactly the loads issued
+// after it, which keeps the prefetch in flight.  A wave with no block reads PRE at
+// slow index min(slow0, n_slow - 1) and computes nothing.
 // Case A (X as [P, I, Q], slow = p*qs + sq): the block starts at element
 // p*I*Q + sq*fast_size + w*kw + kb*KB.  Case B: the block covers j = slow*fast_size
 // + w*kw + kb*KB onwards, one row of I elements per j.  All fields are uniform.
-template <int STRIDE, int KB, bool CASE_B>
+template <int KB, bool CASE_B>
 struct BlockCursor {
   int kb, nkb;
   i64 slow, sq, base, wrap;
 
-  // starts at block kb0 of slow index slow0; each slow index has nkb blocks, and
-  // after its last one the cursor moves STRIDE slow indices on
   __device__ __forceinline__ BlockCursor(const KernArgs& a, i64 slow0, int w, int nkb_, int kb0) {
     kb = kb0;
     nkb = nkb_;
@@ -273,11 +273,10 @@ struct BlockCursor {
   __device__ __forceinline__ void step(const KernArgs& a) {
     if (++kb == nkb) {
       kb = 0;
-      slow += STRIDE;
-      base += (i64)STRIDE * a.fast_stride;
+      ++slow;
+      base += a.fast_stride;
       if constexpr (!CASE_B) {
-        sq += STRIDE;
-        while (sq >= a.qs) {
+        if (++sq >= a.qs) {
           sq -= a.qs;
           base += wrap;
         }

@@ -172,7 +172,7 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) poff[nt] = (has_pre ? a.r0 : 0) + (16 * nt + c < a.rcount ? 16 * nt + c : 0);
 
-  BlockCursor<1, KB, CASE_B> cur(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
+  BlockCursor<KB, CASE_B> cur(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
 
   auto load = [&](int t, Buf& b) {
     b.kb = cur.kb;
@@ -334,7 +334,7 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    cur = BlockCursor<1, KB, CASE_B>(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
+    cur = BlockCursor<KB, CASE_B>(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
     __syncthreads();
 #pragma unroll 1
     for (int t = 0; t < T; ++t) {
