@@ -34,12 +34,16 @@
 
 namespace tenrso {
 
+constexpr int EIG_NMAX = 1024;  // bound of the mode sizes
 constexpr int INIT_RMAX = 128;  // rank bound of the SVD-based initialisations (that of the ALS)
 // Sweeps queued before the host first looks whether every mode has converged (it takes
 // 11 to 19 at 256 to 1024 rows), and the bound.
 constexpr int JACOBI_FIRST = 12, JACOBI_SWEEPS = 60;
 constexpr double JACOBI_TOL = 1e-14;       // off-diagonal over diagonal, Frobenius norms
-constexpr double JACOBI_ENTRY = 0x1p-54;  // an entry over the diagonal: below its rounding errors
+// An entry over sqrt(w_i w_j), the weights of its row and column: rounding noise up to
+// the first (2^-46 to 2^-50 give the same vectors in 13 to 17 sweeps at 256 rows); none
+// above the second once done, so that small rows beside large ones converge as well.
+constexpr double JACOBI_NOISE = 0x1p-47, JACOBI_ROW = 0x1p-34;
 
 namespace {
 
@@ -148,7 +152,7 @@ struct EigMode {
   double* V;    // N x N: eigenvectors in columns
   double* Q;    // [N / 64][64][64]: the rotations of a round
   int* done;
-  double* thr;  // entries off the diagonal up to this size count as zero
+  double* w;    // N: weights of the rows (noise_root)
   double* U;    // n x R: eigenvectors of the top R, descending
   double* lam;  // R
   int n, N;
@@ -168,6 +172,7 @@ __global__ __launch_bounds__(256) void unfold_gram_reduce_kernel(const double* _
   m.V[e] = i == i2 ? 1.0 : 0.0;
   if (i >= I || i2 >= I) {
     m.A[e] = 0.0;
+    if (i == i2) m.w[i] = 0.0;
     return;
   }
   if (i / GT > i2 / GT) return;
@@ -175,6 +180,7 @@ __global__ __launch_bounds__(256) void unfold_gram_reduce_kernel(const double* _
   for (int k = 0; k < splits; ++k) s += part[(i64)k * I * I + i * I + i2];
   m.A[i * N + i2] = s;
   m.A[i2 * N + i] = s;
+  if (i == i2) m.w[i] = s;
 }
 
 // pair k of round r of the circle method over `count` (even) indices
@@ -224,21 +230,29 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
   return s;
 }
 
+// Rounding noise: an entry up to r_i r_j.  K_ij was summed with an error relative to
+// sqrt(K_ii K_jj), so the weights start as the diagonal of K and are carried through the
+// rotations as variances are.  (Relative to the whole matrix instead, rows of a small
+// scale come out as they went in: slices of 1e-6 beside ordinary ones.)
+__device__ __forceinline__ double noise_root(double w) { return sqrt(JACOBI_NOISE * w); }
+
 // done once the off-diagonal mass is below JACOBI_TOL of the diagonal's; one workgroup a
-// mode.  Entries below the rounding errors of the matrix count as zero and are not
-// rotated: in the null space of an exact low-rank tensor there is nothing else, diagonal
-// entries included, so every rotation there is one of about 45 degrees, and the block
-// method then converges linearly.  (256 rows, rank 64, weights down to 1e-4: 16 sweeps;
-// with those rotations 1e-10 off after 24, and vectors off by 7e-6 after 18.)
+// mode.  Entries that are rounding errors count as zero and are not rotated: in the null
+// space of an exact low-rank tensor there is nothing else, diagonal entries included, so
+// every rotation there is one of about 45 degrees, and the block method then converges
+// linearly.  (256 rows, rank 64, weights down to 1e-4: 17 sweeps; with those rotations
+// 1e-10 off after 24, and vectors off by 7e-6 after 18.)
 __global__ __launch_bounds__(1024) void jacobi_check_kernel(EigArgs a) {
-  __shared__ double red[16];
+  __shared__ double red[16], rt[EIG_NMAX];
   const EigMode& m = a.m[blockIdx.x];
   if (*m.done) return;
   const i64 N = m.N;
-  double off = 0.0, dia = 0.0;
-  for (i64 i = threadIdx.x; i < N; i += 1024) dia = fma(m.A[i * N + i], m.A[i * N + i], dia);
+  double off = 0.0, dia = 0.0, large = 0.0;
+  for (i64 i = threadIdx.x; i < N; i += 1024) {
+    dia = fma(m.A[i * N + i], m.A[i * N + i], dia);
+    rt[i] = noise_root(m.w[i]);
+  }
   dia = block_sum<1024>(dia, red);
-  const double thr = JACOBI_ENTRY * sqrt(dia);
   // four rows in flight (N is a multiple of 64)
   for (i64 i = threadIdx.x >> 6; i < N; i += 64)
     for (i64 j = threadIdx.x & 63; j < N; j += 64) {
@@ -246,14 +260,16 @@ __global__ __launch_bounds__(1024) void jacobi_check_kernel(EigArgs a) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) v[u] = m.A[(i + 16 * u) * N + j];
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (i + 16 * u != j && !(fabs(v[u]) <= thr)) off = fma(v[u], v[u], off);
+      for (int u = 0; u < 4; ++u) {
+        const double r = rt[i + 16 * u] * rt[j];
+        v[u] = i + 16 * u == j || fabs(v[u]) <= r ? 0.0 : v[u];
+        off = fma(v[u], v[u], off);
+        large = fabs(v[u]) <= JACOBI_ROW / JACOBI_NOISE * r ? large : 1.0;
+      }
     }
   off = block_sum<1024>(off, red);
-  if (threadIdx.x == 0) {
-    *m.thr = thr;
-    if (off <= JACOBI_TOL * JACOBI_TOL * dia) *m.done = 1;
-  }
+  large = block_sum<1024>(large, red);
+  if (threadIdx.x == 0 && large == 0.0 && off <= JACOBI_TOL * JACOBI_TOL * dia) *m.done = 1;
 }
 
 // The rotation of one pair of blocks of round r, accumulated into Q: Jacobi on their
@@ -269,6 +285,7 @@ constexpr int JP = 2 * JB;        // order of a pair
 constexpr int JPITCH = JP + 1;    // doubles
 __global__ __launch_bounds__(1024) void jacobi_pair_kernel(EigArgs a, int r) {
   __shared__ double S[JP * JPITCH], W[JP * JPITCH], cs[JP], red[16];
+  __shared__ double w0[JP], rt[JP], part[16][JP];  // weights, their roots
   const EigMode& m = a.m[blockIdx.y];
   const int blocks = m.N / JB;
   if ((int)blockIdx.x >= blocks / 2 || r >= blocks - 1 || *m.done) return;
@@ -282,8 +299,12 @@ __global__ __launch_bounds__(1024) void jacobi_pair_kernel(EigArgs a, int r) {
     S[i * JPITCH + j] = m.A[gi * N + gj];
     W[i * JPITCH + j] = i == j ? 1.0 : 0.0;
   }
+  double* gw = m.w + (tid < JB ? p * JB + tid : q * JB + tid - JB);  // (tid < JP)
+  if (tid < JP) {
+    w0[tid] = *gw;
+    rt[tid] = noise_root(w0[tid]);
+  }
   __syncthreads();
-  const double thr = *m.thr;
   const int inner = blocks == 2 ? 30 : 1;
   const bool all = r == 0;  // (two blocks have no other round)
   auto pair_of = [&](int rr, int k, int& i, int& j) {
@@ -294,17 +315,40 @@ __global__ __launch_bounds__(1024) void jacobi_pair_kernel(EigArgs a, int r) {
       j = JB + ((k + rr) & (JB - 1));
     }
   };
+  // the weights after the rotations so far; the steps of one sweep use those before it
+  auto weights = [&]() {
+    const int j = tid & 63, i = 4 * (tid >> 6);
+    double v = 0.0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v = fma(W[(i + e) * JPITCH + j] * W[(i + e) * JPITCH + j], w0[i + e], v);
+    part[tid >> 6][j] = v;
+    __syncthreads();
+    if (tid < JP) {
+      v = part[0][j];
+#pragma unroll
+      for (int e = 1; e < 16; ++e) v += part[e][j];
+    }
+    return v;  // of the first JP threads
+  };
   for (int sweep = 0; sweep < inner; ++sweep) {
     if (sweep > 0) {
-      double off = 0.0, dia = 0.0;
+      const double wj = weights();
+      if (tid < JP) rt[tid] = noise_root(wj);
+      __syncthreads();
+      double off = 0.0, dia = 0.0, large = 0.0;
       for (int e = tid; e < JP * JP; e += 1024) {
-        const double v = S[(e / JP) * JPITCH + e % JP];
-        if (e / JP == e % JP) dia += v * v;
-        else if (!(fabs(v) <= thr)) off += v * v;
+        const double v = S[(e / JP) * JPITCH + e % JP], r = rt[e / JP] * rt[e % JP];
+        if (e / JP == e % JP) {
+          dia += v * v;
+        } else if (!(fabs(v) <= r)) {
+          off += v * v;
+          large = fabs(v) <= JACOBI_ROW / JACOBI_NOISE * r ? large : 1.0;
+        }
       }
       off = block_sum<1024>(off, red);
       dia = block_sum<1024>(dia, red);
-      if (off <= JACOBI_TOL * JACOBI_TOL * dia) break;
+      large = block_sum<1024>(large, red);
+      if (large == 0.0 && off <= JACOBI_TOL * JACOBI_TOL * dia) break;
     }
     for (int rr = 0; rr < (all ? JP - 1 : JB); ++rr) {
       if (tid < JB) {
@@ -312,7 +356,7 @@ __global__ __launch_bounds__(1024) void jacobi_pair_kernel(EigArgs a, int r) {
         pair_of(rr, tid, i, j);
         const double apq = S[i * JPITCH + j];
         double c = 1.0, s = 0.0;
-        if (!(fabs(apq) <= thr)) rotation(S[j * JPITCH + j] - S[i * JPITCH + i], 2.0 * apq, c, s);
+        if (!(fabs(apq) <= rt[i] * rt[j])) rotation(S[j * JPITCH + j] - S[i * JPITCH + i], 2.0 * apq, c, s);
         cs[2 * tid] = c;
         cs[2 * tid + 1] = s;
       }
@@ -345,6 +389,8 @@ __global__ __launch_bounds__(1024) void jacobi_pair_kernel(EigArgs a, int r) {
   }
   double* out = m.Q + (i64)blockIdx.x * JP * JP;
   for (int e = tid; e < JP * JP; e += 1024) out[e] = W[(e / JP) * JPITCH + e % JP];
+  const double wj = weights();
+  if (tid < JP) *gw = wj;
 }
 
 // A <- J^T A J and V <- V J for the rotations J of round r: workgroup (x, y) owns the
@@ -632,8 +678,9 @@ int cp_init_svd(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, i64 R
     return TENRSO_ERR_UNSUPPORTED;
   }
   for (int k = 0; k < nd; ++k) {
-    if (shape[k] > 1024) {
-      set_error("mode %d of size %lld exceeds the on-device SVD initialisation bound 1024", k, (long long)shape[k]);
+    if (shape[k] > EIG_NMAX) {
+      set_error("mode %d of size %lld exceeds the on-device SVD initialisation bound %d", k, (long long)shape[k],
+                EIG_NMAX);
       return TENRSO_ERR_UNSUPPORTED;
     }
     if (shape[k] <= 0) {
@@ -644,10 +691,10 @@ int cp_init_svd(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, i64 R
   // what depends on a mode: J columns of its unfolding, the splits of its Gram
   // (about 1024 workgroups, at most 64 MiB of partials), the layout of its buffers
   struct Mode {
-    i64 P, I, Q, J, nt, splits, nn_blk, oA, oQ, oU, oNN, oR;
+    i64 P, I, Q, J, nt, splits, nn_blk, oA, oQ, oW, oU, oNN, oR;
     int ar;
   } md[MAXD];
-  i64 totA = 0, totQ = 0, totU = 0, totNN = 0, totR = 0, part = 0;
+  i64 totA = 0, totQ = 0, totN = 0, totU = 0, totNN = 0, totR = 0, part = 0;
   EigArgs ea{};
   ea.R = (int)R;
   for (int k = 0; k < nd; ++k) {
@@ -670,6 +717,8 @@ int cp_init_svd(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, i64 R
     totA += N * N;
     m.oQ = totQ;
     totQ += N / JP * JP * JP;
+    m.oW = totN;
+    totN += N;
     m.oU = totU;
     totU += m.I * R + R;
     m.nn_blk = (m.J + 255) / 256;
@@ -680,7 +729,7 @@ int cp_init_svd(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, i64 R
   }
   void *pA, *pV, *pPart, *pW;
   TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_A, (size_t)(totA + totQ) * 8, &pA));
-  TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_V, (size_t)(totA + MAXD) * 8 + MAXD * sizeof(int), &pV));
+  TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_V, (size_t)(totA + totN) * 8 + MAXD * sizeof(int), &pV));
   TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_PART, (size_t)part * 8, &pPart));
   TENRSO_TRY(ctx_buffer(ctx, SLOT_EIG_W, (size_t)(totU + totNN) * 8 + (size_t)totR * 4 + 16, &pW));
   float* rnd = (float*)((double*)pW + totU + totNN);
@@ -691,8 +740,8 @@ int cp_init_svd(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, i64 R
     e.A = (double*)pA + m.oA;
     e.Q = (double*)pA + totA + m.oQ;
     e.V = (double*)pV + m.oA;
-    e.thr = (double*)pV + totA + k;
-    e.done = (int*)((double*)pV + totA + MAXD) + k;
+    e.w = (double*)pV + totA + m.oW;
+    e.done = (int*)((double*)pV + totA + totN) + k;
     e.U = (double*)pW + m.oU;
     e.lam = e.U + m.I * R;
     maxN = std::max(maxN, e.N);

@@ -51,6 +51,31 @@ def test_close_eigenvalues(n, R):
     assert np.abs(l - lam[:R]).max() <= 2.0 ** -22 * lam[0]
 
 
+@pytest.mark.parametrize("n,R,scale", [(96, 64, 1e-6), (64, 50, 1e-8), (300, 80, 1e-7)])
+def test_slices_of_two_scales(n, R, scale):
+    """Small slices beside ordinary ones: their vectors, which span the small rows up to `scale`, by residual and
+    orthogonality, relative to the small part of K.  Rows are multiplied by a power of two, so that the small part is
+    exact; what couples the two parts moves it by the large part's projection only, a factor of order one."""
+    print(f"[case] svd init two scales {n} rows R={R} scale {scale}", flush=True)
+    rng = np.random.default_rng(n)
+    big = 20
+    X = rng.standard_normal((n, 64, 64)).astype(np.float32)
+    p2 = np.float32(2.0 ** np.round(np.log2(scale)))
+    X[big:] *= p2
+    U = left_vectors(X, R)[big:, big:] * 1.0  # the small rows of the small vectors
+    Y = X.reshape(n, -1).astype(np.float64)
+    A, B = Y[:big], Y[big:] / float(p2)
+    # the small part with the large rows' span taken out: what the small vectors diagonalise, up to p2^2
+    B = B - (B @ A.T) @ np.linalg.solve(A @ A.T, A)
+    K = B @ B.T
+    KU = K @ U
+    l = (U * KU).sum(0)
+    lam = np.linalg.eigvalsh(K)[::-1][:R - big]
+    assert np.abs(U.T @ U - np.eye(R - big)).max() <= 2.0 ** -22
+    assert np.linalg.norm(KU - U * l, axis=0).max() <= 2.0 ** -18 * lam[0]
+    assert np.abs(l - lam).max() <= 2.0 ** -22 * lam[0]
+
+
 def test_leading_vector_of_a_constant_tensor():
     print("[case] svd init constant tensor", flush=True)
     U = left_vectors(np.ones((70, 66, 3), np.float32), 3)
