@@ -109,6 +109,8 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
   const i64 nblk_wg = (s_hi - s_lo) * nkb;
   const i64 wb0 = uniform_i64(wave * nblk_wg / WAVES), wb1 = (wave + 1) * nblk_wg / WAVES;
   const int T = __builtin_amdgcn_readfirstlane((int)(wb1 - wb0));  // blocks of this wave
+  const i64 wq = whole_slow(wb0, nkb);
+  const int wr = (int)(wb0 - wq * nkb);  // its first: block wr of slow index s_lo + wq
   const i64 row_base = (i64)xt * ROWS;
   if (tid == 0) redo = 0;
 
@@ -162,7 +164,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) poff[nt] = (has_pre ? a.r0 : 0) + (16 * nt + c < a.rcount ? 16 * nt + c : 0);
 
-  BlockCursor<KB, CASE_B> cur(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
+  BlockCursor<KB, CASE_B> cur(a, s_lo + wq, w, nkb, wr);
 
   auto load = [&](int t, Buf& b) {
     b.kb = cur.kb;
@@ -339,12 +341,12 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
   if constexpr (EXACT) {
     // not finite, or too small for exact parts of FAST or for T (the bounds of the fp32
     // kernel): all of it again in fp32
-    const float xm = wave_min(xmin.value());
+    const float xm = xmin.value();  // of the lane
     float fm = wmin[0];
 #pragma unroll
     for (int v = 1; v < WAVES; ++v) fm = fminf(fm, wmin[v]);
     const bool small = fm < 0x1p-108f || xm * fm < 0x1p-123f;
-    if (__any(!(sum_of_zeros<MT, NT>(acc) == 0.f)) || small) redo = 1;
+    if (__any(small || !(sum_of_zeros<MT, NT>(acc) == 0.f))) redo = 1;
     __syncthreads();
     if (redo) {
       redo_window<RT, NTH, KWMAX>(smem, a, w, kv);
@@ -352,7 +354,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-      cur = BlockCursor<KB, CASE_B>(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
+      cur = BlockCursor<KB, CASE_B>(a, s_lo + wq, w, nkb, wr);
       __syncthreads();
 #pragma unroll 1
       for (int t = 0; t < T; ++t) {

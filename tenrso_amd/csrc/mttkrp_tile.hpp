@@ -123,11 +123,19 @@ __device__ __forceinline__ void window_zero_tail(FastWindow<RT, NTH, KWMAX>& fw,
   }
 }
 
-// smallest over the wave
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
-  return v;
+// Smallest over the wave: within rows of 16 lanes, then across them, by DPP (a shuffle
+// through LDS takes six round trips of 60 ns; with two of those a launch of 32^3 took
+// 5.7 us instead of 5.1).
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
+#define TENRSO_DPP_MIN(CTRL, ROWS) v = min(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROWS, 0xf, false))
+  TENRSO_DPP_MIN(0x111, 0xf);  // row_shr:1, 2, 4, 8
+  TENRSO_DPP_MIN(0x112, 0xf);
+  TENRSO_DPP_MIN(0x114, 0xf);
+  TENRSO_DPP_MIN(0x118, 0xf);
+  TENRSO_DPP_MIN(0x142, 0xa);  // row_bcast:15 into rows 1 and 3, row_bcast:31 into 2 and 3
+  TENRSO_DPP_MIN(0x143, 0xc);
+#undef TENRSO_DPP_MIN
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
 // The smallest magnitude of the bf16 values that are not zero, kept for each half of a
@@ -152,16 +160,18 @@ struct MinNonzero {
 
 // The smallest magnitude of the values a wave stages that are not zero, 2^126 if there
 // is none.  (Fillers of rows and ranks that do not exist repeat values of the window.)
+// Kept as 2 |v| - 1 in unsigned words, which zero makes the largest.
 template <int RT, int NTH, int KWMAX>
 __device__ __forceinline__ float window_min(const FastWindow<RT, NTH, KWMAX>& fw) {
-  float m = 0x1p126f;
+  uint32_t m = 0xffffffffu;
 #pragma unroll
   for (int e = 0; e < FastWindow<RT, NTH, KWMAX>::PERU; ++e)
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) m = fw.v[e][h][q] != 0.f ? fminf(m, fabsf(fw.v[e][h][q])) : m;
-  return wave_min(m);
+      for (int q = 0; q < 4; ++q) m = min(m, (__float_as_uint(fw.v[e][h][q]) << 1) - 1);
+  m = wave_min(m);
+  return m == 0xffffffffu ? 0x1p126f : __uint_as_float((m >> 1) + 1);
 }
 
 // The window in LDS as a bf16 pair: FAST = hi + lo with hi = bf16(FAST) and
@@ -233,6 +243,10 @@ static __device__ float kPreOnes[128] = {
     TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8,
     TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8, TENRSO_ONES8};
 #undef TENRSO_ONES8
+
+// Blocks below b of nkb (1 to 4) a slow index: the slow indices they fill.  Without a
+// division by a variable in a workgroup's start (0.15 us of a launch of 24^3).
+__device__ __forceinline__ i64 whole_slow(i64 b, int nkb) { return nkb == 3 ? b / 3 : b >> (nkb >> 1); }
 
 // Block schedule of one wave: a contiguous range of the workgroup's blocks, from block
 // kb0 of slow index slow0 on, nkb blocks a slow index.  Loads run in that order, so the

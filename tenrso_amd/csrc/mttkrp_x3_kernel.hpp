@@ -118,6 +118,8 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
   const i64 nblk_wg = (s_hi - s_lo) * nkb;
   const i64 wb0 = uniform_i64(wave * nblk_wg / WAVES), wb1 = (wave + 1) * nblk_wg / WAVES;
   const int T = __builtin_amdgcn_readfirstlane((int)(wb1 - wb0));  // blocks of this wave
+  const i64 wq = whole_slow(wb0, nkb);
+  const int wr = (int)(wb0 - wq * nkb);  // its first: block wr of slow index s_lo + wq
   const i64 row_base = (i64)xt * ROWS;
   if (tid == 0) redo = 0;
 
@@ -172,7 +174,7 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) poff[nt] = (has_pre ? a.r0 : 0) + (16 * nt + c < a.rcount ? 16 * nt + c : 0);
 
-  BlockCursor<KB, CASE_B> cur(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
+  BlockCursor<KB, CASE_B> cur(a, s_lo + wq, w, nkb, wr);
 
   auto load = [&](int t, Buf& b) {
     b.kb = cur.kb;
@@ -320,12 +322,12 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
   }
 
   // not finite, or too small: all of it again in fp32
-  const float xm = wave_min(xmin.value());
+  const float xm = xmin.value();  // of the lane
   float fm = wmin[0];
 #pragma unroll
   for (int v = 1; v < WAVES; ++v) fm = fminf(fm, wmin[v]);
   const bool small = xm < 0x1p-108f || fm < 0x1p-108f || xm * fm < 0x1p-123f;
-  if (__any(!(sum_of_zeros<MT, NT>(acc) == 0.f)) || small) redo = 1;
+  if (__any(small || !(sum_of_zeros<MT, NT>(acc) == 0.f))) redo = 1;
   __syncthreads();
   float* out = partial + (i64)split * a.I * a.R;
   if (redo) {
@@ -334,7 +336,7 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    cur = BlockCursor<KB, CASE_B>(a, s_lo + wb0 / nkb, w, nkb, (int)(wb0 % nkb));
+    cur = BlockCursor<KB, CASE_B>(a, s_lo + wq, w, nkb, wr);
     __syncthreads();
 #pragma unroll 1
     for (int t = 0; t < T; ++t) {
