@@ -136,13 +136,16 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
 
   // per-lane element offsets, fixed for the whole loop; the per-block part of
   // every address is wave-uniform
+  // Case A, XL 3: eights of a block that are read.  In a window of one block those past
+  // its end are not: their lanes load what the last ones do.
+  const int eights = XL == 3 && nkb == 1 ? (kv + 7) / 8 : KB / 8, gl = min(g, eights - 1);
   i64 loff[MT];
   int shift = 0;  // case B: bits by which the lane's rows lie above the loaded four
   if constexpr (!CASE_B) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const i64 rr = row_base + 16 * mt + c;
-      loff[mt] = (rr < a.I ? rr : a.I - 1) * a.Q + 8 * g;
+      loff[mt] = (rr < a.I ? rr : a.I - 1) * a.Q + 8 * gl;
     }
   } else {
     const i64 rr = row_base + MT * c, top = a.I > MT ? a.I - MT : 0;
@@ -153,7 +156,8 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
   i64 lim = 0;
   if constexpr (XL == 3) {
     const i64 last = (row_base + ROWS < a.I ? row_base + ROWS : a.I) - 1;
-    lim = uniform_i64(CASE_B ? a.total - (i64)(KB - 1) * a.I - (a.I > MT ? a.I : MT) : a.total - last * a.Q - KB);
+    lim = uniform_i64(CASE_B ? a.total - (i64)(KB - 1) * a.I - (a.I > MT ? a.I : MT)
+                             : a.total - last * a.Q - 8 * eights);
   }
   // PRE column of each lane: columns past rcount read column r0 (those
   // accumulator columns are never stored)
@@ -168,11 +172,11 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
 
   auto load = [&](int t, Buf& b) {
     b.kb = cur.kb;
-    const float* prow = pre_base + cur.slow * pre_stride;
+    const float* prow = pre_base + opaque_uniform(cur.slow * pre_stride);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) b.pre[nt] = prow[poff[nt]];
     const bool live = t < T;  // past the end: one cache line at X (see the fp32 kernel)
-    const i64 off = live ? cur.offset(a) : 0;
+    const i64 off = opaque_uniform(live ? cur.offset(a) : 0);
     const uint16_t* ubase = X + off;
     bool inside = true;  // uniform
     if constexpr (XL == 3) inside = live ? off <= lim : a.total >= 8;
@@ -187,7 +191,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
       if (XL != 3 || inside) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          const uint16_t* base = ubase + (live ? loff[mt] : 0);
+          const uint16_t* base = ubase + opaque_lane(live ? loff[mt] : 0);
 #pragma unroll
           for (int ks = 0; ks < KS; ++ks) {
             if constexpr (XL == 3) __builtin_memcpy(&b.x[mt][ks], __builtin_assume_aligned(base + 32 * ks, 2), 16);
@@ -195,18 +199,17 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
           }
         }
       } else {
+        const int top = live ? kv - 1 - b.kb * KB - 8 * gl : 0;  // past the window's end: its last element
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int mt = 0; mt < MT; ++mt) {
+          const uint16_t* base = ubase + opaque_lane(live ? loff[mt] : 0);
 #pragma unroll
-          for (int e = 0; e < 8; e += 2) {
-            const int k = b.kb * KB + 8 * g + e;
-            const uint32_t lo = *(live && k < kv ? ubase + loff[mt] + e : X);
-            const uint32_t hi = *(live && k + 1 < kv ? ubase + loff[mt] + e + 1 : X);
-            b.x[mt][0][e / 2] = lo | hi << 16;
-          }
+          for (int e = 0; e < 8; e += 2)
+            b.x[mt][0][e / 2] = (uint32_t)base[min(e, top)] | (uint32_t)base[min(e + 1, top)] << 16;
+        }
       }
     } else {
-      const uint16_t* base = ubase + (live ? loff[0] : 0);
+      const uint16_t* base = ubase + opaque_lane(live ? loff[0] : 0);
       const i64 stride = live ? a.I : 0;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {

@@ -237,6 +237,21 @@ __device__ __forceinline__ i64 uniform_i64(i64 v) {
   return (i64)(((uint64_t)hi << 32) | lo);
 }
 
+// Block loads take their offsets through these, so that each is one unconditional vector
+// load.  The compiler otherwise reads a loaded value again from its register where the
+// offset may not have changed (after a wait for all loads), and with scalar loads, behind
+// a branch, where a wave has no block left: a workgroup's first loads went out one round
+// trip after another.
+__device__ __forceinline__ i64 opaque_uniform(i64 v) {
+  v = uniform_i64(v);
+  asm volatile("" : "+s"(v));
+  return v;
+}
+__device__ __forceinline__ i64 opaque_lane(i64 v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
 // PRE row used when the MTTKRP has no PRE factor (a matrix): KR = FAST.
 #define TENRSO_ONES8 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f
 static __device__ float kPreOnes[128] = {

@@ -146,13 +146,16 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
 
   // per-lane element offsets, fixed for the whole loop; the per-block part of
   // every address is wave-uniform
+  // Case A, XL 1: eights of a block that are read.  In a window of one block those past
+  // its end are not: their lanes load what the last ones do.
+  const int eights = XL == 1 && nkb == 1 ? (kv + 7) / 8 : KB / 8, gl = min(g, eights - 1);
   i64 loff[MT];
   bool tail = false;  // case B, odd I: the lane's row is the second of its pair
   if constexpr (!CASE_B) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const i64 rr = row_base + 16 * mt + c;
-      loff[mt] = (rr < a.I ? rr : a.I - 1) * a.Q + 8 * g;
+      loff[mt] = (rr < a.I ? rr : a.I - 1) * a.Q + 8 * gl;
     }
   } else {
     const i64 rr = row_base + MT * c;
@@ -163,7 +166,7 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
   i64 lim = 0;
   if constexpr (XL == 1) {
     const i64 last = (row_base + ROWS < a.I ? row_base + ROWS : a.I) - 1;
-    lim = uniform_i64(CASE_B ? a.total - (i64)KB * a.I : a.total - last * a.Q - KB);
+    lim = uniform_i64(CASE_B ? a.total - (i64)KB * a.I : a.total - last * a.Q - 8 * eights);
   }
   // PRE column of each lane: columns past rcount read column r0 (those
   // accumulator columns are never stored)
@@ -178,13 +181,13 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
 
   auto load = [&](int t, Buf& b) {
     b.kb = cur.kb;
-    const float* prow = pre_base + cur.slow * pre_stride;
+    const float* prow = pre_base + opaque_uniform(cur.slow * pre_stride);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) b.pre[nt] = prow[poff[nt]];
     // past the last block every lane reads the first elements of X (one cache
     // line): the load stays unconditional and costs the memory pipeline little
     const bool live = t < T;
-    const i64 off = live ? cur.offset(a) : 0;
+    const i64 off = opaque_uniform(live ? cur.offset(a) : 0);
     const float* ubase = X + off;
     bool inside = true;  // uniform
     if constexpr (XL == 1) inside = live ? off <= lim : a.total >= 8;
@@ -192,7 +195,7 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
       if (XL != 1 || inside) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          const float* base = ubase + (live ? loff[mt] : 0);
+          const float* base = ubase + opaque_lane(live ? loff[mt] : 0);
           floatx4 v0, v1;
           if constexpr (XL == 1) {
             __builtin_memcpy(&v0, __builtin_assume_aligned(base, 4), sizeof(v0));
@@ -204,14 +207,16 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
           b.x[mt] = floatx8{v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
         }
       } else {
+        const int top = live ? kv - 1 - b.kb * KB - 8 * gl : 0;  // past the window's end: its last element
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int mt = 0; mt < MT; ++mt) {
+          const float* base = ubase + opaque_lane(live ? loff[mt] : 0);
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            b.x[mt][e] = *(live && b.kb * KB + 8 * g + e < kv ? ubase + loff[mt] + e : X);
+          for (int e = 0; e < 8; ++e) b.x[mt][e] = base[min(e, top)];
+        }
       }
     } else {
-      const float* base = ubase + (live ? loff[0] : 0);
+      const float* base = ubase + opaque_lane(live ? loff[0] : 0);
       const i64 stride = live ? a.I : 0;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
