@@ -86,7 +86,7 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
       __syncthreads();
     }
   }
-  const int tile = (int)blockIdx.x - (!CASE_B && has_job ? 1 : 0);
+  const int tile = a.tile0 + (int)blockIdx.x - (!CASE_B && has_job ? 1 : 0);
   const int xt = tile % a.rtiles;
   uint16_t* sHi = reinterpret_cast<uint16_t*>(smem);
   uint16_t* sLo = sHi + RT * PITCH;
@@ -866,6 +866,8 @@ static int occupancy(tenrso_ctx* ctx, const void* kern, int threads, int* occ) {
   return TENRSO_OK;
 }
 
+constexpr i64 MAX_THREADS = UINT32_MAX;  // of a launch in one dimension
+
 // a.slow_splits splits of the slow range, balanced
 static void set_splits(KernArgs& a, i64 ssp) {
   a.slow_splits = (int)std::max<i64>(1, ssp);
@@ -1130,12 +1132,16 @@ int mttkrp_dense(tenrso_ctx* ctx, int prec, const void* X, const void* X_t, int 
             jarg.gate_stamp = ++ctx->gate_stamp;
           }
         }
-        const dim3 grid((unsigned)(rtiles * splits + has_job), 1, 1);
         a.r0 = rc * RT;
         a.rcount = (int)std::min<i64>(RT, R - a.r0);
-        int hj = has_job;
-        void* args[] = {(void*)&Xuse, &a, &partial, &jarg, &hj};
-        TENRSO_HIP_TRY(hipLaunchKernel(kern, grid, block, args, 0, ctx->stream));
+        // (a matrix of tens of millions of rows has more tiles than a launch takes)
+        for (i64 t0 = 0; t0 < rtiles * splits; t0 += MAX_THREADS / block.x - 1) {
+          int hj = t0 == 0 ? has_job : 0;
+          const i64 tiles_now = std::min<i64>(rtiles * splits - t0, MAX_THREADS / block.x - 1);
+          a.tile0 = (int)t0;
+          void* args[] = {(void*)&Xuse, &a, &partial, &jarg, &hj};
+          TENRSO_HIP_TRY(hipLaunchKernel(kern, dim3((unsigned)(tiles_now + hj)), block, args, 0, ctx->stream));
+        }
       }
       return TENRSO_OK;
     };
@@ -1236,7 +1242,9 @@ int mttkrp_all_modes(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, 
     one = plan[m].ok && plan[m].case_b == (m == nd - 1) && plan[m].xl == plan[m < nd - 1 ? 0 : m].xl;
     wv = wv && plan[m].a.win_vec;
   }
-  if (one) {
+  i64 tiles = 64 * ctx->num_cus;  // a bound of the workgroups of one launch
+  for (int m = 0; one && m < nd; ++m) tiles += (i64)plan[m].a.rtiles * plan[m].a.nwin;
+  if (one && tiles < MAX_THREADS / 256) {
     const void* kern = mttkrp_x3_kernel_all(plan[0].nt, wv, plan[0].xl, plan[nd - 1].xl);
     int occ = 0;
     TENRSO_TRY(occupancy(ctx, kern, 256, &occ));

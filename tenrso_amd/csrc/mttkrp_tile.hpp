@@ -35,6 +35,7 @@ struct KernArgs {
   int r0;             // first rank column of this launch
   int rcount;         // rank columns handled by the launch (<= 16*NT)
   int rtiles;         // row tiles; workgroup tile -> (tile % rtiles, split = tile / rtiles)
+  int tile0;          // the launch's first tile
   double* norm;       // sums of squares of X, one per wave of the launch (NORM kernels)
   int win_vec;        // FAST 16-byte aligned and R % 4 == 0: 16-byte window loads
 };

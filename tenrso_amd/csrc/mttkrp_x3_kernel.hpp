@@ -323,7 +323,7 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if (lane == 0) a.norm[(i64)blockIdx.x * WAVES + wave] = v;
+    if (lane == 0) a.norm[(i64)tile * WAVES + wave] = v;
   }
 
   // not finite, or too small: all of it again in fp32
@@ -376,8 +376,8 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_x3_mfma(const float* __rest
     }
     return;
   }
-  x3_tile<NT, WAVES, CASE_B, WV, XL, NORM>(X, a, partial, (int)blockIdx.x - (JOB != 0 && has_job ? 1 : 0), smem,
-                                           wmin, redo);
+  x3_tile<NT, WAVES, CASE_B, WV, XL, NORM>(X, a, partial,
+                                           a.tile0 + (int)blockIdx.x - (JOB != 0 && has_job ? 1 : 0), smem, wmin, redo);
 }
 
 template <int NT, int WAVES, int JOB, bool CASE_B, bool WV, bool NORM>
