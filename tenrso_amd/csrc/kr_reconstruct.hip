@@ -7,6 +7,7 @@
 // cp_reconstruct (tenrso-kernels/src/outer.rs:223-274):
 //   out[i_0..i_{N-1}] = sum_r (prod_k F_k[i_k, r]) * w_r.
 //   An FP32 matrix product of two Khatri-Rao factors formed in LDS.
+#include <algorithm>
 #include <cfloat>
 #include <type_traits>
 
@@ -56,6 +57,7 @@ struct ReconArgs {
   const float* w;
   int vec;              // R % 4 == 0 and every factor 16-byte aligned: 16-byte factor loads
   unsigned ctiles;
+  unsigned tile0;       // the launch's first tile
   const float* xsub;    // not null: out = xsub - reconstruction (a residual)
   const float* gscale;  // not null: out *= gscale[0] (a device scalar)
 };
@@ -87,7 +89,8 @@ __global__ __launch_bounds__(256) void reconstruct_kernel(ReconArgs a, float* __
   __shared__ int range;  // 1, 2: a product of the rows, columns is subnormal; 4, 8: one is above 1; 16: not finite
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
-  const i64 r_base = (i64)(blockIdx.x / a.ctiles) * TILE, c_base = (i64)(blockIdx.x % a.ctiles) * TILE;
+  const unsigned tile = a.tile0 + blockIdx.x;
+  const i64 r_base = (i64)(tile / a.ctiles) * TILE, c_base = (i64)(tile % a.ctiles) * TILE;
   // factor rows of every tile row (modes < h) and column (modes >= h); those past
   // the end repeat the last one and are not stored
   if (tid == 0) range = 0;
@@ -306,12 +309,18 @@ int cp_residual_f32(tenrso_ctx* ctx, int nd, const i64* shape, const float* cons
   a.ctiles = cdiv(a.N, tile);
   const bool vs = a.N % 4 == 0 && (uintptr_t)out % 16 == 0 && (!X || (uintptr_t)X % 16 == 0);
   auto launch = [&](auto kt, auto t) {
-    if (vs)
-      hipLaunchKernelGGL((reconstruct_kernel<decltype(kt)::value, decltype(t)::value, true>), dim3((unsigned)best),
-                         dim3(256), 0, ctx->stream, a, out);
-    else
-      hipLaunchKernelGGL((reconstruct_kernel<decltype(kt)::value, decltype(t)::value, false>), dim3((unsigned)best),
-                         dim3(256), 0, ctx->stream, a, out);
+    // (a vector of 2^31 elements has more tiles than the 2^32 - 1 threads of a launch)
+    constexpr i64 MOST = UINT32_MAX / 256;
+    for (i64 t0 = 0; t0 < best; t0 += MOST) {
+      a.tile0 = (unsigned)t0;
+      const dim3 grid((unsigned)std::min<i64>(MOST, best - t0));
+      if (vs)
+        hipLaunchKernelGGL((reconstruct_kernel<decltype(kt)::value, decltype(t)::value, true>), grid, dim3(256), 0,
+                           ctx->stream, a, out);
+      else
+        hipLaunchKernelGGL((reconstruct_kernel<decltype(kt)::value, decltype(t)::value, false>), grid, dim3(256), 0,
+                           ctx->stream, a, out);
+    }
   };
   auto by_rank = [&](auto t) {
     if (R <= 16) launch(std::integral_constant<int, 16>{}, t);
