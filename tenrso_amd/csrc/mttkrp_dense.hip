@@ -1251,7 +1251,11 @@ int mttkrp_all_modes(tenrso_ctx* ctx, const float* X, int nd, const i64* shape, 
     // Splits: the resident workgroups of one round shared between the modes, at least a
     // block a wave (256^3 rank 64: 43.9 us in one round, 48.7 in two, 54.6 in three,
     // 61.4 in one with a few workgroups over).
-    const i64 target = (i64)(ctx->wg_per_cu_f32 > 0 ? ctx->wg_per_cu_f32 : occ) * ctx->num_cus;
+    // Resident workgroups a CU: three of the registers' four (96^4 rank 32: 200 us against
+    // 206 with four and 201 with two), two where X is read at any alignment (250^3 rank 16
+    // 42 against 46 with three, 80x90x100x110 rank 30 263 against 304).
+    const int most = plan[0].xl == 0 ? 3 : 2;
+    const i64 target = (i64)(ctx->wg_per_cu_f32 > 0 ? ctx->wg_per_cu_f32 : std::min(occ, most)) * ctx->num_cus;
     AllModesArgs p{};
     p.nd = nd;
     for (int m = 0; m < nd; ++m) {
