@@ -124,9 +124,9 @@ __device__ __forceinline__ void window_zero_tail(FastWindow<RT, NTH, KWMAX>& fw,
   }
 }
 
-// Smallest over the wave: within rows of 16 lanes, then across them, by DPP (a shuffle
-// through LDS takes six round trips of 60 ns; with two of those a launch of 32^3 took
-// 5.7 us instead of 5.1).
+// Smallest over the wave: within rows of 16 lanes, then across them, by DPP (shuffles
+// through LDS are six round trips; with two such reductions a launch of 32^3 took 5.9 us
+// instead of 5.5).
 __device__ __forceinline__ uint32_t wave_min(uint32_t v) {
 #define TENRSO_DPP_MIN(CTRL, ROWS) v = min(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROWS, 0xf, false))
   TENRSO_DPP_MIN(0x111, 0xf);  // row_shr:1, 2, 4, 8

@@ -7,7 +7,7 @@
 // products and adds them in fp32, sixteen times as fast as the fp32 instruction:
 // six terms run at 2.7 times its rate, and the kernel becomes bound by memory.
 //
-// Measured, one launch, X in memory (256^3 rank 64, 64 MiB): 18.0-18.9 us against
+// Measured, one launch, X in memory (256^3 rank 64, 64 MiB): 16.6-18.0 us against
 // 26-28 us with v_mfma_f32_16x16x4_f32, whose matrix pipe was busy for 16 us; the
 // same launch with one term and no split takes 14.9 us (4.5 TB/s, start and end
 // included), the five other terms 2 us more and the split of X 1 us.

@@ -228,7 +228,7 @@ def initialize_factors(shape, rank, init=InitStrategy.Random, seed=None, tensor=
     Random / RandomNormal are drawn here (seeded; the reference uses an unseeded
     thread_rng).  Svd / Nnsvd / LeverageScore need the tensor: the SVD of every
     unfolding runs on the device (tenrso_cp_init_svd; mode sizes <= 1024, rank
-    <= 64).  Returns float32 numpy arrays.
+    <= 128).  Returns float32 numpy arrays.
     """
     rng = np.random.default_rng(seed)
     if init == InitStrategy.Random:
