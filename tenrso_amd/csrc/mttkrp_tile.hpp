@@ -243,13 +243,17 @@ __device__ __forceinline__ i64 uniform_i64(i64 v) {
 // offset may not have changed (after a wait for all loads), and with scalar loads, behind
 // a branch, where a wave has no block left: a workgroup's first loads went out one round
 // trip after another.
+template <bool ON = true>
 __device__ __forceinline__ i64 opaque_uniform(i64 v) {
-  v = uniform_i64(v);
-  asm volatile("" : "+s"(v));
+  if constexpr (ON) {
+    v = uniform_i64(v);
+    asm volatile("" : "+s"(v));
+  }
   return v;
 }
+template <bool ON = true>
 __device__ __forceinline__ i64 opaque_lane(i64 v) {
-  asm volatile("" : "+v"(v));
+  if constexpr (ON) asm volatile("" : "+v"(v));
   return v;
 }
 

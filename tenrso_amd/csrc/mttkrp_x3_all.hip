@@ -1,7 +1,11 @@
 // mttkrp_x3_all.hip -- the fp32 MTTKRP kernel over all modes of a tensor.
 //
 // A launch a mode leaves the GPU idle between the last workgroups of one and the first
-// data of the next; here a CU goes on with the next mode's workgroups.
+// data of the next; here a CU goes on with the next mode's workgroups.  With whole
+// windows the block loads are left to the compiler here (x3_tile's OPAQUE): other
+// workgroups cover their start, and X streams better for it (X from memory each time: 96^4
+// rank 32 199 us against 207, 512x512x128 rank 32 64 against 69; with masked windows
+// 250^3 rank 16 takes 49 that way, 43 this).
 #include "mttkrp_x3.hpp"
 #include "mttkrp_x3_kernel.hpp"
 
@@ -19,8 +23,8 @@ __global__ __launch_bounds__(256) void mttkrp_x3_all(const float* __restrict__ X
   while (m + 1 < p.nd && blockIdx.x >= p.first[m + 1]) ++m;
   const int tile = (int)(blockIdx.x - p.first[m]);
   const KernArgs a = p.a[m];
-  if (m == p.nd - 1) x3_tile<NT, WAVES, true, WV, XLB, false>(X, a, p.partial[m], tile, smem, wmin, redo);
-  else x3_tile<NT, WAVES, false, WV, XLA, false>(X, a, p.partial[m], tile, smem, wmin, redo);
+  if (m == p.nd - 1) x3_tile<NT, WAVES, true, WV, XLB, false, XLB != 0>(X, a, p.partial[m], tile, smem, wmin, redo);
+  else x3_tile<NT, WAVES, false, WV, XLA, false, XLA != 0>(X, a, p.partial[m], tile, smem, wmin, redo);
 }
 
 template <int NT, bool WV>

@@ -92,9 +92,10 @@ constexpr int x3_lds() {
   return win > red ? win : red;
 }
 
-// One workgroup's tile.  smem: x3_lds bytes; wmin: smallest magnitude of the window
-// values that each wave stages; redo: a wave asks for the fp32 form.
-template <int NT, int WAVES, bool CASE_B, bool WV, int XL, bool NORM>
+// One workgroup's tile.  OPAQUE: block loads through opaque_uniform and opaque_lane.
+// smem: x3_lds bytes; wmin: smallest magnitude of the window values that each wave
+// stages; redo: a wave asks for the fp32 form.
+template <int NT, int WAVES, bool CASE_B, bool WV, int XL, bool NORM, bool OPAQUE = true>
 __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernArgs& a, float* __restrict__ partial,
                                         int tile, float* smem, float* wmin, int& redo) {
   constexpr int MT = 2, NBUF = X3_NBUF<NT>, KWMAX = X3_KWMAX;
@@ -181,13 +182,13 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
 
   auto load = [&](int t, Buf& b) {
     b.kb = cur.kb;
-    const float* prow = pre_base + opaque_uniform(cur.slow * pre_stride);
+    const float* prow = pre_base + opaque_uniform<OPAQUE>(cur.slow * pre_stride);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) b.pre[nt] = prow[poff[nt]];
     // past the last block every lane reads the first elements of X (one cache
     // line): the load stays unconditional and costs the memory pipeline little
     const bool live = t < T;
-    const i64 off = opaque_uniform(live ? cur.offset(a) : 0);
+    const i64 off = opaque_uniform<OPAQUE>(live ? cur.offset(a) : 0);
     const float* ubase = X + off;
     bool inside = true;  // uniform
     if constexpr (XL == 1) inside = live ? off <= lim : a.total >= 8;
@@ -195,7 +196,7 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
       if (XL != 1 || inside) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          const float* base = ubase + opaque_lane(live ? loff[mt] : 0);
+          const float* base = ubase + opaque_lane<OPAQUE>(live ? loff[mt] : 0);
           floatx4 v0, v1;
           if constexpr (XL == 1) {
             __builtin_memcpy(&v0, __builtin_assume_aligned(base, 4), sizeof(v0));
@@ -210,13 +211,13 @@ __device__ __forceinline__ void x3_tile(const float* __restrict__ X, const KernA
         const int top = live ? kv - 1 - b.kb * KB - 8 * gl : 0;  // past the window's end: its last element
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          const float* base = ubase + opaque_lane(live ? loff[mt] : 0);
+          const float* base = ubase + opaque_lane<OPAQUE>(live ? loff[mt] : 0);
 #pragma unroll
           for (int e = 0; e < 8; ++e) b.x[mt][e] = base[min(e, top)];
         }
       }
     } else {
-      const float* base = ubase + opaque_lane(live ? loff[0] : 0);
+      const float* base = ubase + opaque_lane<OPAQUE>(live ? loff[0] : 0);
       const i64 stride = live ? a.I : 0;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
