@@ -172,7 +172,9 @@ __global__ __launch_bounds__(WAVES * 64) void mttkrp_bf16_mfma(const uint16_t* _
 
   auto load = [&](int t, Buf& b) {
     b.kb = cur.kb;
-    const float* prow = pre_base + opaque_uniform(cur.slow * pre_stride);
+    // (whole windows: PRE is loaded again only where the slow index changes; at rank 64
+    // four loads a block beside X's four cost a BF16 ALS of 256^3 1 to 2 %)
+    const float* prow = pre_base + opaque_uniform<CASE_B || XL != 0>(cur.slow * pre_stride);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) b.pre[nt] = prow[poff[nt]];
     const bool live = t < T;  // past the end: one cache line at X (see the fp32 kernel)
